@@ -27,6 +27,7 @@
 #include "fft_plan.h"
 #include "fused_x.h"
 #include "hist_device.h"
+#include "load_ylm.h"
 #include "ylm_device.h"
 
 struct fc_corr {
@@ -239,25 +240,6 @@ __global__ void __launch_bounds__(1024)
     if (cc < ncol) q[((int64_t)sx * n1 + y) * ldc + c0 + cc] = lds[e * tc + cc];
   }
 }
-
-// ---- z-pass loader with Y_lm(x) weighting (correlator.h:435-436) -----------
-struct LoadYlm {
-  int ell, m, n1;
-  double c, x0, y0, z0;  // cell centres relative to the observer: x0 + i etc.
-  int i0 = 0;            // x slab of row 0
-  void shift_x(int dx) { i0 += dx; }
-  struct Row {
-    int ell, m;
-    double c, x, y, z0;
-    __device__ __forceinline__ double operator()(double v, int k) const {
-      return ylm_eval(ell, m, x, y, z0 + (double)k * 1.0, c, v);
-    }
-  };
-  __device__ __forceinline__ Row row(int64_t r) const {
-    const int i = i0 + (int)(r / n1), j = (int)(r % n1);
-    return Row{ell, m, c, x0 + (double)i * 1.0, y0 + (double)j * 1.0, z0};
-  }
-};
 
 // Histogram entries.  A histogram sample is weight * value with the weight
 // Y_l0 (x) sqrt(4 pi (2l+1)) times the rescaling (and W^-1(k) in k space),

@@ -79,6 +79,79 @@ __device__ __forceinline__ double ylm_eval(int ell, int m, double x, double y, d
   }
 }
 
+// The same D-free numerator c P_lm(x, y, z) as a polynomial a[0] + a[1] z + ..
+// of degree l <= 4 in z, for fixed x and y (every formula above expanded).
+__device__ __forceinline__ void ylm_row(int ell, int m, double x, double y, double c, double* a) {
+  a[0] = c;
+  a[1] = a[2] = a[3] = a[4] = 0.0;
+  if (ell == 0) return;
+  const double x2 = x * x, y2 = y * y;
+  if (ell == 2) {
+    const double h = c * sqrt(15.0 / 8.0);
+    switch (m) {
+      case 2:
+        a[0] = c * sqrt(15.0 / 32.0) * (x2 - y2);
+        return;
+      case 1:
+        a[0] = 0.0;
+        a[1] = h * x;
+        return;
+      case 0:
+        a[0] = c * sqrt(5.0 / 16.0) * -(x2 + y2);
+        a[2] = c * sqrt(5.0 / 16.0) * 2.0;
+        return;
+      case -1:
+        a[0] = 0.0;
+        a[1] = h * y;
+        return;
+      default:
+        a[0] = h * x * y;
+        return;
+    }
+  }
+  const double p = x2 + y2, d = x2 - y2;
+  const double c2 = c * 3.0 / 8.0 * sqrt(5.0 / 2.0);
+  const double c1 = c * 3.0 / 8.0 * sqrt(5.0);
+  const double c3 = c * 3.0 / 8.0 * sqrt(35.0);
+  const double c4 = c * 3.0 / 16.0 * sqrt(35.0 / 2.0);
+  a[0] = 0.0;
+  switch (m) {
+    case 4:
+      a[0] = c4 * (x2 * x2 - 6.0 * x2 * y2 + y2 * y2);
+      return;
+    case 3:
+      a[1] = c3 * (x2 - 3.0 * y2) * x;
+      return;
+    case 2:
+      a[0] = c2 * -(d * p);
+      a[2] = c2 * 6.0 * d;
+      return;
+    case 1:
+      a[1] = c1 * -3.0 * p * x;
+      a[3] = c1 * 4.0 * x;
+      return;
+    case 0:
+      a[0] = c * 9.0 / 16.0 * p * p;
+      a[2] = c * -4.5 * p;
+      a[4] = c * 1.5;
+      return;
+    case -1:
+      a[1] = c1 * -3.0 * p * y;
+      a[3] = c1 * 4.0 * y;
+      return;
+    case -2:
+      a[0] = c2 * -2.0 * x * y * p;
+      a[2] = c2 * 12.0 * x * y;
+      return;
+    case -3:
+      a[1] = c3 * (3.0 * x2 - y2) * y;
+      return;
+    default:
+      a[0] = c4 * 4.0 * x * y * d;
+      return;
+  }
+}
+
 // |(x, y, z)| as the reference's subgrid setup computes it
 // (correlator.h:133, :185): sqrt((x*x + y*y) + z*z), no contraction.
 __device__ __forceinline__ double norm3(double x, double y, double z) {
