@@ -118,9 +118,11 @@ void tune(fc_ctx* ctx, const int shape[3], int prec, int reps, double* best_ms) 
     const FftPlan& pt = *pa;
     if constexpr (wide)
       launch_cols_wide<T, -1, A>(L, v, tc, (ax == 1 ? pt.tw1 : pt.tw0).template as<cplx<A>>(),
-                                 (ax == 1 ? p->tw1 : p->tw0).template as<cplx<T>>(), s, var);
+                                 (ax == 1 ? p->tw1 : p->tw0).template as<cplx<T>>(), s,
+                                 p->gen[ax].get(), var);
     else
-      launch_cols<T, -1>(L, v, tc, (ax == 1 ? p->tw1 : p->tw0).template as<cplx<T>>(), s, var);
+      launch_cols<T, -1>(L, v, tc, (ax == 1 ? p->tw1 : p->tw0).template as<cplx<T>>(), s,
+                         p->gen[ax].get(), var);
   };
   for (int ax = 1; ax >= 0; --ax) {
     const int L = shape[ax];
@@ -170,9 +172,11 @@ void tune(fc_ctx* ctx, const int shape[3], int prec, int reps, double* best_ms) 
               v.A = nx;
               if constexpr (wide)
                 launch_cols_wide<T, -1, A>(shape[1], v, p->tile[1], pa->tw1.as<cplx<A>>(),
-                                           p->tw1.as<cplx<T>>(), s, p->var[1]);
+                                           p->tw1.as<cplx<T>>(), s,
+                                           p->gen[1].get(), p->var[1]);
               else
-                launch_cols<T, -1>(shape[1], v, p->tile[1], p->tw1.as<cplx<T>>(), s, p->var[1]);
+                launch_cols<T, -1>(shape[1], v, p->tile[1], p->tw1.as<cplx<T>>(), s,
+                                           p->gen[1].get(), p->var[1]);
             }
           },
           reps);

@@ -24,6 +24,7 @@
 #include <type_traits>
 
 #include "fc_objects.h"
+#include "fft_gen_px.h"
 #include "fft_plan.h"
 #include "fused_x.h"
 #include "hist_device.h"
@@ -742,7 +743,7 @@ void forward_zy(fc_corr* c, fc_grid* g, cplx<T>* dst, Loader ld) {
     ColView<T> v = y_view<T>(p, d);
     v.A = nx;
     launch_cols_wide<T, -1, A>(p.n[1], v, p.tile[1], pa.tw1.as<cplx<A>>(), p.tw1.as<cplx<T>>(),
-                               s, p.var[1]);
+                               s, p.gen[1].get(), p.var[1]);
   }
 }
 
@@ -780,7 +781,7 @@ void forward_zy_pair(fc_corr* c, fc_grid* ga, fc_grid* gb, cplx<T>* dst) {
   ColView<T> v = y_view<T>(p, dst);
   v.A = 2 * p.n[0];
   launch_cols_wide<T, -1, A>(p.n[1], v, p.tile[1], pa.tw1.as<cplx<A>>(), p.tw1.as<cplx<T>>(), s,
-                             p.var[1]);
+                             p.gen[1].get(), p.var[1]);
 }
 
 template <typename T, typename A = T>
@@ -789,7 +790,7 @@ void forward_x(fc_corr* c, cplx<T>* dst) {
   Stage st(c, FC_STAGE_FFT_X_FWD);
   launch_cols_wide<T, -1, A>(p.n[0], x_view<T>(p, dst), p.tile[0],
                              c->plan_inv->tw0.as<cplx<A>>(), p.tw0.as<cplx<T>>(),
-                             c->ctx->stream, p.var[0]);
+                             c->ctx->stream, p.gen[0].get(), p.var[0]);
 }
 
 // Full forward 3D FFT.
@@ -962,9 +963,39 @@ bool px_fits(const fc_corr* c) {
   return px_len_ok(p.n[0]) && p.complex_bytes() <= lim && q1 <= lim && pk <= lim;
 }
 
+// Mixed-radix fused x pass (x lengths without a compile-time plan).
+bool px_gen_ok(const fc_corr* c) { return c->plan->gen[0] && gen_px_ok(*c->plan->gen[0]); }
+
+template <typename T, typename TI, int MODE>
+void launch_px_gen(fc_corr* c, const cplx<T>* a, const cplx<T>* b, const PxOut& po) {
+  const FftPlan& p = *c->plan;
+  const int rs = c->rshape;
+  const GenPx<T> g{a,
+                   b,
+                   p.n[1],
+                   p.n2h,
+                   (int64_t)p.ldc,
+                   c->ph[0].as<double2>(),
+                   c->ph[1].as<double2>(),
+                   c->ph[2].as<double2>(),
+                   static_cast<T*>(po.pk),
+                   kslots(c),
+                   po.q1,
+                   (int64_t)c->plan_inv->ldc,
+                   rs,
+                   (rs / 2) % p.n[0],
+                   po.nb,
+                   po.a_bstride,
+                   po.pk_bstride,
+                   po.q_bstride};
+  launch_gen_px<T, TI, MODE>(*p.gen[0], g, c->ctx->stream);
+}
+
 template <typename T, typename TI, int MODE>
 void fused_x(fc_corr* c, cplx<T>* w, const cplx<T>* b) {
-  if (px_fits(c))
+  if (px_gen_ok(c))
+    launch_px_gen<T, TI, MODE>(c, w, b, PxOut{c->pk.as<void>(), c->q1.as<void>()});
+  else if (px_fits(c))
     launch_periodic_x2<T, TI, MODE>(c, w, b, PxOut{c->pk.as<void>(), c->q1.as<void>()});
   else if constexpr (std::is_same<T, TI>::value)
     launch_periodic_x<T, MODE>(c, w, b);
@@ -1013,7 +1044,7 @@ void power_x(fc_corr* c, cplx<T>* w, const cplx<T>* b, int mode) {
   const FftPlan& pi = *c->plan_inv;
   const int64_t ldq = pi.ldc;
   const int rs = c->rshape, o = rs / 2;
-  const bool fused = px_fits(c) || (p.fast[0] && !px_len_ok(p.n[0]) &&
+  const bool fused = px_gen_ok(c) || px_fits(c) || (p.fast[0] && !px_len_ok(p.n[0]) &&
                                     std::is_same<T, TI>::value);
   if (fused) {
     Stage st(c, FC_STAGE_COMBINE);
@@ -1031,7 +1062,7 @@ void power_x(fc_corr* c, cplx<T>* w, const cplx<T>* b, int mode) {
     Stage st(c, FC_STAGE_FFT_X_INV);
     ColView<TI, T> v{w, 0, (int64_t)p.n[1] * p.ldc, (int64_t)p.ldc, c->q1.as<cplx<TI>>(), 0,
                      (int64_t)p.n[1] * ldq, ldq, 1, p.n[1], p.n2h, rs, o};
-    launch_cols<TI, +1, T>(p.n[0], v, pi.tile[0], pi.tw0.as<cplx<TI>>(), s);
+    launch_cols<TI, +1, T>(p.n[0], v, pi.tile[0], pi.tw0.as<cplx<TI>>(), s, pi.gen[0].get());
   }
 }
 
@@ -1047,7 +1078,7 @@ void pruned_inverse_yz(fc_corr* c) {
     Stage st(c, FC_STAGE_FFT_Y_INV);
     ColView<TI> v{c->q1.as<cplx<TI>>(), (int64_t)pi.n[1] * ldq, ldq, 0, c->q2.as<cplx<TI>>(),
                   (int64_t)rs * ldq, ldq, 0, rs, 1, pi.n2h, rs, o};
-    launch_cols<TI, +1>(pi.n[1], v, pi.tile[1], pi.tw1.as<cplx<TI>>(), s);
+    launch_cols<TI, +1>(pi.n[1], v, pi.tile[1], pi.tw1.as<cplx<TI>>(), s, pi.gen[1].get());
   }
   // Pruned z C2R: rows of q2 -> r subgrid rows xi[sx][sy][sz].
   Stage st(c, FC_STAGE_FFT_Z_INV);
@@ -1196,11 +1227,13 @@ T* full_inverse(fc_corr* c, cplx<T>* w) {
   hipStream_t s = c->ctx->stream;
   {
     Stage st(c, FC_STAGE_FFT_X_INV);
-    launch_cols<T, +1>(p.n[0], x_view<T>(p, w), p.tile[0], p.tw0.as<cplx<T>>(), s);
+    launch_cols<T, +1>(p.n[0], x_view<T>(p, w), p.tile[0], p.tw0.as<cplx<T>>(), s,
+                       p.gen[0].get());
   }
   {
     Stage st(c, FC_STAGE_FFT_Y_INV);
-    launch_cols<T, +1>(p.n[1], y_view<T>(p, w), p.tile[1], p.tw1.as<cplx<T>>(), s);
+    launch_cols<T, +1>(p.n[1], y_view<T>(p, w), p.tile[1], p.tw1.as<cplx<T>>(), s,
+                       p.gen[1].get());
   }
   Stage st(c, FC_STAGE_FFT_Z_INV);
   T* xr = reinterpret_cast<T*>(w);
@@ -1791,12 +1824,15 @@ void batch_sequence(fc_batch* bt, int n) {
     ColView<T> v = y_view<T>(p, w);
     v.A = n * p.n[0];
     launch_cols_wide<T, -1, TI>(p.n[1], v, p.tile[1], pi.tw1.as<cplx<TI>>(),
-                                p.tw1.as<cplx<T>>(), s, p.var[1]);
+                                p.tw1.as<cplx<T>>(), s, p.gen[1].get(), p.var[1]);
   }
-  if (px_fits(c)) {
+  if (px_fits(c) || px_gen_ok(c)) {
     PxOut po{bt->pk.as<void>(), bt->q1.as<void>(), n, (int64_t)p.n[0] * p.n[1] * p.ldc, bt->npk,
              bt->nq1};
-    launch_periodic_x2<T, TI, kModeAuto>(c, w, nullptr, po);
+    if (px_fits(c))
+      launch_periodic_x2<T, TI, kModeAuto>(c, w, nullptr, po);
+    else
+      launch_px_gen<T, TI, kModeAuto>(c, w, nullptr, po);
   } else {
     // x lengths without the fused kernel (e.g. 384 = 3 x 128): per member,
     // the x pass, |F|^2, the compact k values and the pruned inverse x pass
@@ -1807,7 +1843,7 @@ void batch_sequence(fc_batch* bt, int n) {
     for (int i = 0; i < n; ++i) {
       cplx<T>* wi = w + (int64_t)i * nc;
       launch_cols_wide<T, -1, TI>(p.n[0], x_view<T>(p, wi), p.tile[0], pi.tw0.as<cplx<TI>>(),
-                                  p.tw0.as<cplx<T>>(), s, p.var[0]);
+                                  p.tw0.as<cplx<T>>(), s, p.gen[0].get(), p.var[0]);
       hipLaunchKernelGGL(k_conj_mult<T>, dim3(grid1d(nc, 256, 65536)), dim3(256), 0, s, wi,
                          nullptr, nc);
       FC_LAUNCH_CHECK();
@@ -1817,16 +1853,16 @@ void batch_sequence(fc_batch* bt, int n) {
       ColView<TI, T> v{wi, 0, (int64_t)p.n[1] * p.ldc, (int64_t)p.ldc,
                        bt->q1.as<cplx<TI>>() + i * bt->nq1, 0, (int64_t)p.n[1] * ldq, ldq, 1,
                        p.n[1], p.n2h, rs, o};
-      launch_cols<TI, +1, T>(p.n[0], v, pi.tile[0], pi.tw0.as<cplx<TI>>(), s);
+      launch_cols<TI, +1, T>(p.n[0], v, pi.tile[0], pi.tw0.as<cplx<TI>>(), s, pi.gen[0].get());
     }
   }
   {
     ColView<TI> v{bt->q1.as<cplx<TI>>(), (int64_t)pi.n[1] * ldq, ldq, 0, bt->q2.as<cplx<TI>>(),
                   (int64_t)rs * ldq, ldq, 0, n * rs, 1, pi.n2h, rs, o};
-    launch_cols<TI, +1>(pi.n[1], v, pi.tile[1], pi.tw1.as<cplx<TI>>(), s);
+    launch_cols<TI, +1>(pi.n[1], v, pi.tile[1], pi.tw1.as<cplx<TI>>(), s, pi.gen[1].get());
   }
   launch_rows_c2r<TI, TI>(pi, bt->q2.as<cplx<TI>>(), ldq, bt->xisub.as<TI>(), rs, s,
-                          (int64_t)n * rs * rs, rs, o);
+                          (int64_t)n * rs * rs, rs, o, (int64_t)rs * rs);
   if (c->khalf_ok) {
     run_hist_khalf<T, NV>(c, bt->pk.as<T>(), bt->npk, bt->part, bt->k_hist.as<double>(),
                           bt->k_counts.as<int>(), 0, 0, NV, s, n, hk);

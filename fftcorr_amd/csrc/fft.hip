@@ -190,6 +190,10 @@ std::shared_ptr<FftPlan> build_plan(int device, const int shape[3], int prec) {
     if (p->zy_chunk >= shape[0]) p->zy_chunk = 0;
   }
   DeviceGuard g(device);
+  for (int i = 0; i < 3; ++i)
+    if (!p->fast[i])
+      for (int q = 0; q <= i && !p->gen[i]; ++q)  // equal lengths share their tables
+        p->gen[i] = q < i ? (shape[q] == shape[i] ? p->gen[q] : nullptr) : make_gen_axis(shape[i]);
   if (prec == FC_FP64) {
     upload_twiddles<double>(p->tw0, shape[0]);
     upload_twiddles<double>(p->tw1, shape[1]);

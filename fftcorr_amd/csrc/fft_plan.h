@@ -10,6 +10,7 @@
 #include <type_traits>
 
 #include "fc_internal.h"
+#include "fft_gen.h"
 #include "fft_kernels.h"
 
 namespace fc {
@@ -44,6 +45,9 @@ struct FftPlan {
   int zy_chunk_kib = 0;
   // Twiddle tables exp(-2 pi i m / L) in the plan's precision.
   DeviceBuffer tw0, tw1;      // lengths n0, n1
+  // Mixed-radix tables of the axes without a compile-time plan (axis 2: the
+  // whole row length n2); null where fast[] or where only the direct DFT is left.
+  std::shared_ptr<GenAxis> gen[3];
   DeviceBuffer tw2M, tw2N;    // lengths n2/2 (fast rows) and n2 (post-process / DFT)
   size_t csize() const { return prec == FC_FP64 ? sizeof(double2) : sizeof(float2); }
   int64_t nrows() const { return (int64_t)n[0] * n[1]; }
@@ -167,11 +171,17 @@ void launch_cols_rc(int L, const ColView<T, Tin>& v, const cplx<A>* tw, hipStrea
   FC_LAUNCH_CHECK();
 }
 
+// gen: the length's mixed-radix tables (FftPlan::gen), taken where present.
 template <typename T, int DIR, typename Tin = T>
 void launch_cols(int L, const ColView<T, Tin>& v, int tc, const cplx<T>* tw, hipStream_t s,
-                 int var = 0) {
+                 const GenAxis* gen, int var = 0) {
   const size_t cs = sizeof(cplx<T>);
   const int nout = v.nout ? v.nout : L;
+  if (gen) {
+    const GenCols gc{v.inA, v.inL, v.inG, v.outA, v.outL, v.outG,
+                     v.A,   v.G,   v.B,   nout,   ((v.off % L) + L) % L};
+    return launch_gen_cols<Tin, T>(*gen, v.in, v.out, gc, DIR, s);
+  }
   if (rc_len_ok(L) && (size_t)L * tc * cs <= kLdsBudget && tc * (L / 8) <= 1024 &&
       rc_offsets_fit<T, Tin>(L, tc, v.inL, v.outL, nout)) {
     const int vr = fft_var_ok(L, var) ? var : 0;
@@ -222,7 +232,7 @@ void launch_cols(int L, const ColView<T, Tin>& v, int tc, const cplx<T>* tw, hip
 // register-chained kernel takes L (tw_a: twiddles in A), else in T (tw_t).
 template <typename T, int DIR, typename A>
 void launch_cols_wide(int L, const ColView<T>& v, int tc, const cplx<A>* tw_a,
-                      const cplx<T>* tw_t, hipStream_t s, int var = 0) {
+                      const cplx<T>* tw_t, hipStream_t s, const GenAxis* gen, int var = 0) {
   if constexpr (!std::is_same<T, A>::value) {
     int t = tc;
     while (t > 4 && ((size_t)L * t * sizeof(cplx<T>) > kLdsBudget || t * (L / 8) > 1024)) t /= 2;
@@ -234,7 +244,7 @@ void launch_cols_wide(int L, const ColView<T>& v, int tc, const cplx<A>* tw_a,
       return launch_cols_rc<T, DIR, T, 4, A>(L, v, tw_a, s, vr);
     }
   }
-  launch_cols<T, DIR>(L, v, tc, tw_t, s, var);
+  launch_cols<T, DIR>(L, v, tc, tw_t, s, gen, var);
 }
 
 // In-place y pass over the work grid [n0][n1][ldc].
@@ -267,6 +277,9 @@ void launch_rows_r2c(const FftPlan& p, const Tin* in, int64_t ldi, cplx<T>* out,
   const int tr = p.tile[2];
   const cplx<T>* twM = p.tw2M.as<cplx<T>>();
   const cplx<T>* twN = p.tw2N.as<cplx<T>>();
+  if (p.gen[2] && !in2)
+    return launch_gen_r2c<Tin, T>(*p.gen[2], in, ldi, out, ldo, nrows,
+                                  std::min(nrows, p.nrows()), ld, s);
   if (in2 && !(p.fast[2] && rc_len_ok(M)))
     fail(FC_ERR_RUNTIME, "internal: two-grid z pass needs the register-chained rows");
   if (p.fast[2] && rc_len_ok(M)) {
@@ -342,16 +355,21 @@ void launch_rows_r2c(const FftPlan& p, const Tin* in, int64_t ldi, cplx<T>* out,
 }
 
 // nrows rows of ldi complex -> real rows of ldo; nsel > 0 keeps only samples
-// (o - off) mod n2, o < nsel (pruned inverse).
+// (o - off) mod n2, o < nsel (pruned inverse).  grp: rows of one batch member
+// (0: one member), where rows are transformed in pairs.
 template <typename T, typename Tout>
 void launch_rows_c2r(const FftPlan& p, const cplx<T>* in, int64_t ldi, Tout* out, int64_t ldo,
-                     hipStream_t s, int64_t nrows = -1, int nsel = 0, int off = 0) {
+                     hipStream_t s, int64_t nrows = -1, int nsel = 0, int off = 0, int64_t grp = 0) {
   const size_t cs = sizeof(cplx<T>);
   if (nrows < 0) nrows = p.nrows();
   const int M = p.n[2] / 2;
   const int tr = p.tile[2];
   const cplx<T>* twM = p.tw2M.as<cplx<T>>();
   const cplx<T>* twN = p.tw2N.as<cplx<T>>();
+  if constexpr (std::is_same<T, Tout>::value)
+    if (p.gen[2])
+      return launch_gen_c2r<T>(*p.gen[2], in, ldi, out, ldo, nrows, grp ? grp : nrows, nsel,
+                               nsel ? ((off % p.n[2]) + p.n[2]) % p.n[2] : 0, s);
   if (p.fast[2] && rc_len_ok(M)) {
     int trc = tr;
     while (trc > 1 && (size_t)trc * row_pad_len(M) * cs > kLdsBudget) trc /= 2;
@@ -411,15 +429,19 @@ void launch_rows_c2r(const FftPlan& p, const cplx<T>* in, int64_t ldi, Tout* out
 // y then x forward passes over the complex work grid [n0][n1][ldc].
 template <typename T>
 void fft_yx_forward(const FftPlan& p, cplx<T>* data, hipStream_t s) {
-  launch_cols<T, -1>(p.n[1], y_view<T>(p, data), p.tile[1], p.tw1.as<cplx<T>>(), s, p.var[1]);
-  launch_cols<T, -1>(p.n[0], x_view<T>(p, data), p.tile[0], p.tw0.as<cplx<T>>(), s, p.var[0]);
+  launch_cols<T, -1>(p.n[1], y_view<T>(p, data), p.tile[1], p.tw1.as<cplx<T>>(), s,
+                     p.gen[1].get(), p.var[1]);
+  launch_cols<T, -1>(p.n[0], x_view<T>(p, data), p.tile[0], p.tw0.as<cplx<T>>(), s,
+                     p.gen[0].get(), p.var[0]);
 }
 
 // x then y inverse passes.
 template <typename T>
 void fft_xy_inverse(const FftPlan& p, cplx<T>* data, hipStream_t s) {
-  launch_cols<T, +1>(p.n[0], x_view<T>(p, data), p.tile[0], p.tw0.as<cplx<T>>(), s);
-  launch_cols<T, +1>(p.n[1], y_view<T>(p, data), p.tile[1], p.tw1.as<cplx<T>>(), s);
+  launch_cols<T, +1>(p.n[0], x_view<T>(p, data), p.tile[0], p.tw0.as<cplx<T>>(), s,
+                     p.gen[0].get());
+  launch_cols<T, +1>(p.n[1], y_view<T>(p, data), p.tile[1], p.tw1.as<cplx<T>>(), s,
+                     p.gen[1].get());
 }
 
 }  // namespace fc
