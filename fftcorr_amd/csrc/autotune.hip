@@ -56,7 +56,7 @@ struct Timer {
 };
 
 bool col_tile_ok(int L, int tc, size_t cs) {
-  const int tcol = fft_len_fast(L) ? L / fft_len_e(L) : 1;
+  const int tcol = rc_len_ok(L) ? L / fft_len_e(L) : 1;
   return tc * tcol <= 1024 && (size_t)L * tc * cs <= kLdsBudget;
 }
 
@@ -136,15 +136,14 @@ void tune(fc_ctx* ctx, const int shape[3], int prec, int reps, double* best_ms) 
     double bt = 1e300;
     for (int var = 0; var < kFftVariants; ++var) {
       if (!fft_var_ok(L, var)) continue;
-      for (int tc : {1, 2, 4, 8, 16, 32}) {
-        if (!col_tile_ok(L, tc, cs)) continue;
-        if (var > 0 && !(tc == 4 || tc == 8 || tc == 16)) continue;  // register-chained only
-        p->tile[ax] = tc;
-        p->var[ax] = var;
+      for (int tc : {4, 8, 16}) {  // the column widths of the register-chained pass
+        // The plan's own width is always timed (other passes choose theirs).
+        if (!(var == bestv && tc == best) && (!rc_len_ok(L) || !col_tile_ok(L, tc, cs))) continue;
         const double t = tm.time([&] { col_pass(ax, tc, var); }, reps);
         if (t < bt) bt = t, best = tc, bestv = var;
       }
     }
+    if (bt == 1e300) bt = tm.time([&] { col_pass(ax, best, bestv); }, reps);
     p->tile[ax] = best;
     p->var[ax] = bestv;
     out[2 - ax] = bt;

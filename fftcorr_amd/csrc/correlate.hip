@@ -159,89 +159,6 @@ __global__ void k_gather_pk(T* __restrict__ pk, const cplx<T>* __restrict__ P, K
   }
 }
 
-// ---- fused periodic x pass --------------------------------------------------
-// One workgroup per (y row, tile of tc kz columns); block = tc * (L / E).
-// A: grid a after its z and y passes; B: grid b likewise (interlaced) or the
-// fully transformed grid 2 (cross).  Writes pk and the pruned inverse-x
-// output q[sx][y][c] for x lags sx - rs/2, sx < rs.
-template <typename T, int L, int MODE>
-__global__ void __launch_bounds__(1024)
-    k_periodic_x(const cplx<T>* __restrict__ A, const cplx<T>* __restrict__ B, int n1, int n2h,
-                 int64_t ldc, int tilesC, int tc, const cplx<T>* __restrict__ tw,
-                 const double2* __restrict__ ph0, const double2* __restrict__ ph1,
-                 const double2* __restrict__ ph2, T* __restrict__ pk, KSlots ks,
-                 cplx<T>* __restrict__ q, int rs) {
-  using C = cplx<T>;
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  C* lds = reinterpret_cast<C*>(smem_raw);
-  constexpr int E = FftCfg<L>::E;
-  constexpr int TCOL = L / E;
-  const int y = blockIdx.x / tilesC;
-  const int c0 = (blockIdx.x - y * tilesC) * tc;
-  const int ncol = min(tc, n2h - c0);
-  const int64_t sL = (int64_t)n1 * ldc;
-  const int64_t base = (int64_t)y * ldc + c0;
-  const int tid = threadIdx.x, nthr = blockDim.x;
-  const int c = tid % tc, t = tid / tc;
-  C rb[E];
-  // L * tc elements over tc * (L / E) threads: E loads per thread, issued
-  // before the LDS stores.
-  auto load_tile = [&](const C* __restrict__ src) {
-    C tmp[E];
-#pragma unroll
-    for (int qq = 0; qq < E; ++qq) {
-      const int idx = tid + qq * nthr;
-      const int e = idx / tc, cc = idx - e * tc;
-      tmp[qq] = cc < ncol ? src[base + e * sL + cc] : C{T(0), T(0)};
-    }
-#pragma unroll
-    for (int qq = 0; qq < E; ++qq) lds[tid + qq * nthr] = tmp[qq];
-  };
-  if (MODE == kModeInterlaced) {
-    load_tile(B);
-    __syncthreads();
-    fft_lds<T, L, -1>(lds, tw, c, t, LayColFast{tc});
-#pragma unroll
-    for (int qq = 0; qq < E; ++qq) rb[qq] = lds[(t + qq * TCOL) * tc + c];
-    __syncthreads();
-  }
-  load_tile(A);
-  __syncthreads();
-  fft_lds<T, L, -1>(lds, tw, c, t, LayColFast{tc});
-  {
-#pragma clang fp contract(off)
-    const int cg = c0 + c;
-#pragma unroll
-    for (int qq = 0; qq < E; ++qq) {
-      const int e = t + qq * TCOL;
-      const C fa = lds[e * tc + c];
-      C p;
-      if (MODE == kModeInterlaced) {
-        const double2 ph = cmul(cmul(ph0[e], ph1[y]), ph2[c < ncol ? cg : 0]);
-        const C fb = rb[qq];
-        const double fx = 0.5 * ((double)fa.x + ((double)fb.x * ph.x - (double)fb.y * ph.y));
-        const double fy = 0.5 * ((double)fa.y + ((double)fb.x * ph.y + (double)fb.y * ph.x));
-        p = C{T(fx * fx + fy * fy), T(0)};
-      } else if (MODE == kModeCross) {
-        const C g = c < ncol ? B[base + e * sL + c] : C{T(0), T(0)};
-        p = C{fa.x * g.x + fa.y * g.y, fa.y * g.x - fa.x * g.y};
-      } else {
-        p = C{fa.x * fa.x + fa.y * fa.y, T(0)};
-      }
-      lds[e * tc + c] = p;
-      if (c < ncol) put_pk<T>(pk, ks, L, n1, e, y, cg, p.x);
-    }
-  }
-  __syncthreads();
-  fft_lds<T, L, +1>(lds, tw, c, t, LayColFast{tc});
-  const int o = rs / 2;
-  for (int idx = tid; idx < rs * tc; idx += nthr) {
-    const int sx = idx / tc, cc = idx - sx * tc;
-    const int e = ((sx - o) % L + L) % L;
-    if (cc < ncol) q[((int64_t)sx * n1 + y) * ldc + c0 + cc] = lds[e * tc + cc];
-  }
-}
-
 // Histogram entries.  A histogram sample is weight * value with the weight
 // Y_l0 (x) sqrt(4 pi (2l+1)) times the rescaling (and W^-1(k) in k space),
 // formed by the same FP64 operations, in the same order, as the reference's
@@ -527,6 +444,7 @@ struct Stage {
   fc_corr* c;
   int id;
   int e0 = -1;
+  bool keep = true;  // false: nothing was launched, the interval is dropped
   Stage(fc_corr* c_, int id_) : c(c_), id(id_) {
     if (!c->profile) return;
     if (c->ev_used + 2 > c->ev_pool.size()) {
@@ -541,6 +459,10 @@ struct Stage {
   }
   ~Stage() {
     if (e0 < 0) return;
+    if (!keep) {
+      --c->ev_used;
+      return;
+    }
     const int e1 = (int)c->ev_used++;
     if (hipEventRecord(c->ev_pool[e1], c->ctx->stream) == hipSuccess)
       c->pending.push_back({id, e0, e1});
@@ -754,7 +676,7 @@ void forward_zy(fc_corr* c, fc_grid* g, cplx<T>* dst, Loader ld) {
 // separate launches measured 0.5% faster.
 bool forward_pair_plan_ok(const fc_corr* c) {
   const FftPlan& p = *c->plan;
-  return c->prec != FC_FP64 && p.zy_chunk == 0 && p.fast[2] && rc_len_ok(p.n[2] / 2);
+  return c->prec != FC_FP64 && p.zy_chunk == 0 && p.fast[2];
 }
 bool forward_pair_ok(const fc_corr* c, const fc_grid* ga, const fc_grid* gb) {
   return forward_pair_plan_ok(c) && ga->prec == gb->prec;
@@ -860,147 +782,37 @@ struct PxOut {
   int64_t a_bstride = 0, pk_bstride = 0, q_bstride = 0;
 };
 
-// Register-chained fused x pass (power-of-two x lengths up to 512).
+// The fused x pass: the compile-time plan of the x length, else the mixed-radix
+// one.  False if neither takes it (then the x pass runs in separate steps).
 template <typename T, typename TI, int MODE>
-void launch_periodic_x2(fc_corr* c, const cplx<T>* a, const cplx<T>* b, const PxOut& po) {
+bool fused_x(fc_corr* c, const cplx<T>* a, const cplx<T>* b, const PxOut& po) {
   const FftPlan& p = *c->plan;
   const FftPlan& pi = *c->plan_inv;
-  constexpr int TC = px_tc<T>();
-  const int tilesC = (p.n2h + TC - 1) / TC;
-  const int64_t per = (int64_t)p.n[1] * tilesC;
-  const int64_t nblocks = per * po.nb;
-  if (nblocks > INT32_MAX) fail(FC_ERR_INVALID, "grid too large for the fused x pass");
-  const double2* ph[3] = {c->ph[0].as<double2>(), c->ph[1].as<double2>(),
-                          c->ph[2].as<double2>()};
   const int rs = c->rshape;
-  const int offm = (rs / 2) % p.n[0];
-  if constexpr (std::is_same<T, float>::value && MODE == kModeCross) {
-    // Cross mode, 512-point x over FP32 spectra, one correlation: the
-    // persistent prefetching form, when each tile's 64-byte row segments lie
-    // inside the row pitch and its in-tile offsets fit 32 bits.
-    const uint64_t pitch = (uint64_t)p.n[1] * p.ldc * sizeof(cplx<T>);
-    if (p.n[0] == 512 && po.nb == 1 && (int64_t)tilesC * TC <= p.ldc &&
-        pitch * 16 < (1ull << 32)) {
-      const int grid = (int)std::min<int64_t>(nblocks, current_device_cus());
-      hipLaunchKernelGGL((k_periodic_x2_cross_pipe<TI, 512>), dim3((unsigned)grid),
-                         dim3(px_threads<T, 512>()), 0, c->ctx->stream, a, b, p.n[1], p.n2h,
-                         (int64_t)p.ldc, tilesC, p.tw0.as<cplx<T>>(), pi.tw0.as<cplx<TI>>(),
-                         static_cast<T*>(po.pk), kslots(c), static_cast<cplx<TI>*>(po.q1),
-                         (int64_t)pi.ldc, rs, offm, (int)nblocks);
-      FC_LAUNCH_CHECK();
-      return;
-    }
-  }
-#define FC_PX2_CASE(Lv)                                                                       \
-  case Lv:                                                                                    \
-    hipLaunchKernelGGL((k_periodic_x2<T, TI, Lv, MODE>), dim3((unsigned)nblocks),             \
-                       dim3(px_threads<T, Lv>()), (px_lds_bytes<T, TI, Lv, MODE>()),           \
-                       c->ctx->stream, a, b, p.n[1], p.n2h, (int64_t)p.ldc, tilesC,            \
-                       p.tw0.as<cplx<T>>(), pi.tw0.as<cplx<TI>>(), ph[0], ph[1], ph[2],        \
-                       static_cast<T*>(po.pk), kslots(c), static_cast<cplx<TI>*>(po.q1),     \
-                       (int64_t)pi.ldc, rs, offm, (int)per, po.a_bstride, po.pk_bstride,      \
-                       po.q_bstride);                                                         \
-    break;
-  switch (p.n[0]) {
-    FC_PX2_CASE(8)
-    FC_PX2_CASE(16)
-    FC_PX2_CASE(32)
-    FC_PX2_CASE(64)
-    FC_PX2_CASE(128)
-    FC_PX2_CASE(256)
-    FC_PX2_CASE(512)
-    default:
-      fail(FC_ERR_RUNTIME, "internal: no register-chained x kernel for this length");
-  }
-#undef FC_PX2_CASE
-  FC_LAUNCH_CHECK();
-}
-
-// LDS-staged fused x pass for the longer fast lengths (forward precision only).
-template <typename T, int MODE>
-void launch_periodic_x(fc_corr* c, cplx<T>* a, const cplx<T>* b) {
-  const FftPlan& p = *c->plan;
-  const int tc = p.tile[0];
-  const int tilesC = (p.n2h + tc - 1) / tc;
-  const size_t cs = sizeof(cplx<T>);
-  const double2* ph[3] = {c->ph[0].as<double2>(), c->ph[1].as<double2>(),
-                          c->ph[2].as<double2>()};
-#define FC_PX_CASE(Lv)                                                                      \
-  case Lv: {                                                                                \
-    const int thr = tc * (Lv / FftCfg<Lv>::E);                                              \
-    hipLaunchKernelGGL((k_periodic_x<T, Lv, MODE>), dim3((unsigned)(p.n[1] * tilesC)),     \
-                       dim3(thr), (size_t)Lv * tc * cs, c->ctx->stream, a, b, p.n[1], p.n2h, \
-                       (int64_t)p.ldc, tilesC, tc, p.tw0.as<cplx<T>>(), ph[0], ph[1], ph[2],  \
-                       c->pk.as<T>(), kslots(c), c->q1.as<cplx<T>>(), c->rshape);          \
-    break;                                                                                  \
-  }
-  switch (p.n[0]) {
-    FC_PX_CASE(1024)
-    FC_PX_CASE(2048)
-    FC_PX_CASE(4096)
-    FC_PX_CASE(24)
-    FC_PX_CASE(48)
-    FC_PX_CASE(96)
-    FC_PX_CASE(192)
-    FC_PX_CASE(384)
-    FC_PX_CASE(768)
-    FC_PX_CASE(1536)
-    FC_PX_CASE(3072)
-    default:
-      fail(FC_ERR_RUNTIME, "internal: no fused x kernel for this length");
-  }
-#undef FC_PX_CASE
-  FC_LAUNCH_CHECK();
-}
-
-// The register-chained kernel addresses its arrays with 32-bit byte offsets.
-bool px_fits(const fc_corr* c) {
-  const FftPlan& p = *c->plan;
-  const FftPlan& pi = *c->plan_inv;
-  const uint64_t lim = 0xffffffffull;
-  const uint64_t q1 = (uint64_t)c->rshape * pi.n[1] * pi.ldc * pi.csize();
-  const uint64_t pk = (uint64_t)c->kshape[0] * c->kshape[1] * (c->kshape[2] / 2 + 1) * 8;
-  return px_len_ok(p.n[0]) && p.complex_bytes() <= lim && q1 <= lim && pk <= lim;
-}
-
-// Mixed-radix fused x pass (x lengths without a compile-time plan).
-bool px_gen_ok(const fc_corr* c) { return c->plan->gen[0] && gen_px_ok(*c->plan->gen[0]); }
-
-template <typename T, typename TI, int MODE>
-void launch_px_gen(fc_corr* c, const cplx<T>* a, const cplx<T>* b, const PxOut& po) {
-  const FftPlan& p = *c->plan;
-  const int rs = c->rshape;
-  const GenPx<T> g{a,
-                   b,
-                   p.n[1],
-                   p.n2h,
-                   (int64_t)p.ldc,
-                   c->ph[0].as<double2>(),
-                   c->ph[1].as<double2>(),
-                   c->ph[2].as<double2>(),
-                   static_cast<T*>(po.pk),
-                   kslots(c),
-                   po.q1,
-                   (int64_t)c->plan_inv->ldc,
-                   rs,
-                   (rs / 2) % p.n[0],
-                   po.nb,
-                   po.a_bstride,
-                   po.pk_bstride,
-                   po.q_bstride};
+  const PxArgs<T> g{a,
+                    b,
+                    p.n[1],
+                    p.n2h,
+                    (int64_t)p.ldc,
+                    c->ph[0].as<double2>(),
+                    c->ph[1].as<double2>(),
+                    c->ph[2].as<double2>(),
+                    static_cast<T*>(po.pk),
+                    kslots(c),
+                    po.q1,
+                    (int64_t)pi.ldc,
+                    rs,
+                    (rs / 2) % p.n[0],
+                    po.nb,
+                    po.a_bstride,
+                    po.pk_bstride,
+                    po.q_bstride};
+  if (launch_px_rc<T, TI, MODE>(p.n[0], g, p.tw0.as<cplx<T>>(), pi.tw0.as<cplx<TI>>(),
+                                c->ctx->stream))
+    return true;
+  if (!p.gen[0] || !gen_px_ok(*p.gen[0])) return false;
   launch_gen_px<T, TI, MODE>(*p.gen[0], g, c->ctx->stream);
-}
-
-template <typename T, typename TI, int MODE>
-void fused_x(fc_corr* c, cplx<T>* w, const cplx<T>* b) {
-  if (px_gen_ok(c))
-    launch_px_gen<T, TI, MODE>(c, w, b, PxOut{c->pk.as<void>(), c->q1.as<void>()});
-  else if (px_fits(c))
-    launch_periodic_x2<T, TI, MODE>(c, w, b, PxOut{c->pk.as<void>(), c->q1.as<void>()});
-  else if constexpr (std::is_same<T, TI>::value)
-    launch_periodic_x<T, MODE>(c, w, b);
-  else
-    fail(FC_ERR_RUNTIME, "internal: fused x pass unavailable");
+  return true;
 }
 
 // Forward x pass(es), interlacing and the conjugate product over the whole
@@ -1044,17 +856,19 @@ void power_x(fc_corr* c, cplx<T>* w, const cplx<T>* b, int mode) {
   const FftPlan& pi = *c->plan_inv;
   const int64_t ldq = pi.ldc;
   const int rs = c->rshape, o = rs / 2;
-  const bool fused = px_gen_ok(c) || px_fits(c) || (p.fast[0] && !px_len_ok(p.n[0]) &&
-                                    std::is_same<T, TI>::value);
-  if (fused) {
+  const PxOut po{c->pk.as<void>(), c->q1.as<void>()};
+  bool fused;
+  {
     Stage st(c, FC_STAGE_COMBINE);
     if (mode == kModeInterlaced)
-      fused_x<T, TI, kModeInterlaced>(c, w, b);
+      fused = fused_x<T, TI, kModeInterlaced>(c, w, b, po);
     else if (mode == kModeCross)
-      fused_x<T, TI, kModeCross>(c, w, b);
+      fused = fused_x<T, TI, kModeCross>(c, w, b, po);
     else
-      fused_x<T, TI, kModeAuto>(c, w, b);
-  } else {
+      fused = fused_x<T, TI, kModeAuto>(c, w, b, po);
+    st.keep = fused;
+  }
+  if (!fused) {
     // Other x lengths: separate x pass, combine, gather, pruned inverse x
     // (reading the power grid in T, transforming in TI).
     full_power<T, TI>(c, w, b, mode);
@@ -1826,15 +1640,10 @@ void batch_sequence(fc_batch* bt, int n) {
     launch_cols_wide<T, -1, TI>(p.n[1], v, p.tile[1], pi.tw1.as<cplx<TI>>(),
                                 p.tw1.as<cplx<T>>(), s, p.gen[1].get(), p.var[1]);
   }
-  if (px_fits(c) || px_gen_ok(c)) {
-    PxOut po{bt->pk.as<void>(), bt->q1.as<void>(), n, (int64_t)p.n[0] * p.n[1] * p.ldc, bt->npk,
-             bt->nq1};
-    if (px_fits(c))
-      launch_periodic_x2<T, TI, kModeAuto>(c, w, nullptr, po);
-    else
-      launch_px_gen<T, TI, kModeAuto>(c, w, nullptr, po);
-  } else {
-    // x lengths without the fused kernel (e.g. 384 = 3 x 128): per member,
+  const PxOut po{bt->pk.as<void>(), bt->q1.as<void>(), n, (int64_t)p.n[0] * p.n[1] * p.ldc,
+                 bt->npk, bt->nq1};
+  if (!fused_x<T, TI, kModeAuto>(c, w, nullptr, po)) {
+    // x lengths without a fused kernel (chirp convolutions): per member,
     // the x pass, |F|^2, the compact k values and the pruned inverse x pass
     // (the single correlator's separate-pass sequence) into its slices.
     const int64_t nc = p.nrows() * p.ldc;

@@ -10,18 +10,7 @@
 
 namespace fc {
 
-bool fft_len_fast(int L) {
-  switch (L) {
-    case 8: case 16: case 32: case 64: case 128: case 256: case 512: case 1024:
-    case 2048: case 4096: case 24: case 48: case 96: case 192: case 384: case 768:
-    case 1536: case 3072:
-      return true;
-    default:
-      return false;
-  }
-}
-
-int fft_len_e(int L) { return (L % 3 == 0) ? 24 : 8; }
+int fft_len_e(int L) { return L % 3 == 0 ? 12 : 8; }
 
 namespace {
 template <int... Rs>
@@ -48,6 +37,14 @@ int fft_radices(int L, int var, int* out) {
     case 128: return radices_of<128>(var, out);
     case 256: return radices_of<256>(var, out);
     case 512: return radices_of<512>(var, out);
+    case 1024: return radices_of<1024>(var, out);
+    case 192: return radices_of<192>(var, out);
+    case 384: return radices_of<384>(var, out);
+    case 768: return radices_of<768>(var, out);
+    case 1536: return radices_of<1536>(var, out);
+    case 2048: return radices_of<2048>(var, out);
+    case 3072: return radices_of<3072>(var, out);
+    case 4096: return radices_of<4096>(var, out);
     default: return 0;
   }
 }
@@ -93,7 +90,11 @@ int stage_entries(Put put) {
   if constexpr (FftCfgV<L, 1>::fast)
     stage_twiddles_<L>(typename FftCfgV<L, 1>::radices{},
                        [&](int idx, int m) { put(b1 + idx, m); });
-  return stage_twiddle_base<L, kFftVariants>();
+  const int b2 = stage_twiddle_base<L, 2>();
+  if constexpr (FftCfgV<L, 2>::fast)
+    stage_twiddles_<L>(typename FftCfgV<L, 2>::radices{},
+                       [&](int idx, int m) { put(b2 + idx, m); });
+  return stage_twiddle_base<L, kFftPlans>();
 }
 
 template <class Put>
@@ -106,6 +107,14 @@ int stage_entries_for(int L, Put put) {
     case 128: return stage_entries<128>(put);
     case 256: return stage_entries<256>(put);
     case 512: return stage_entries<512>(put);
+    case 1024: return stage_entries<1024>(put);
+    case 192: return stage_entries<192>(put);
+    case 384: return stage_entries<384>(put);
+    case 768: return stage_entries<768>(put);
+    case 1536: return stage_entries<1536>(put);
+    case 2048: return stage_entries<2048>(put);
+    case 3072: return stage_entries<3072>(put);
+    case 4096: return stage_entries<4096>(put);
     default: return 0;
   }
 }
@@ -131,7 +140,7 @@ void upload_twiddles(DeviceBuffer& buf, int L) {
 int default_col_tile(int L, size_t cs) {
   // Runs of 128 bytes per global access: 16 FP32 / 8 FP64 complex columns.
   int tc = cs == sizeof(float2) ? 16 : 8;
-  const int tcol = fft_len_fast(L) ? L / fft_len_e(L) : 1;
+  const int tcol = rc_len_ok(L) ? L / fft_len_e(L) : 1;
   while (tc > 1 && (tc * tcol > 1024 || (size_t)L * tc * cs > kLdsBudget)) tc /= 2;
   return tc;
 }
@@ -159,10 +168,10 @@ std::shared_ptr<FftPlan> build_plan(int device, const int shape[3], int prec) {
     const int align = (int)(128 / cs);
     p->ldc = (p->n2h + align - 1) / align * align;
   }
-  p->fast[0] = fft_len_fast(shape[0]);
-  p->fast[1] = fft_len_fast(shape[1]);
-  p->fast[2] = (shape[2] % 2 == 0) && fft_len_fast(shape[2] / 2) && shape[2] / 2 <= 2048;
-  // The direct-DFT fallbacks stage a whole column / row in LDS.
+  p->fast[0] = rc_len_ok(shape[0]);
+  p->fast[1] = rc_len_ok(shape[1]);
+  p->fast[2] = (shape[2] % 2 == 0) && rc_len_ok(shape[2] / 2);
+  // Direct sums stage a whole column / row in LDS.
   for (int i = 0; i < 2; ++i)
     if (!p->fast[i] && (size_t)shape[i] * cs > kLdsBudget)
       fail(FC_ERR_INVALID, "FFT length " + std::to_string(shape[i]) +
@@ -195,8 +204,11 @@ std::shared_ptr<FftPlan> build_plan(int device, const int shape[3], int prec) {
   // cells = 7e7 (80 x 73 x 160) it already halves the whole correlation.
   const int64_t cells = (int64_t)shape[0] * shape[1] * shape[2];
   auto direct = [&](int L) { return gen_radices(L).empty() && (int64_t)L * cells < (1 << 24); };
+  // Columns with a compile-time plan keep the tables too: their tiles' 32-bit
+  // offsets do not reach across spectra above 4 GB.
+  const bool big = (uint64_t)p->nrows() * p->ldc * cs > 0xffffffffull;
   for (int i = 0; i < 3; ++i)
-    if (!p->fast[i] && !direct(shape[i]))
+    if ((!p->fast[i] || (big && i < 2)) && !direct(shape[i]))
       for (int q = 0; q <= i && !p->gen[i]; ++q)  // equal lengths share their tables
         p->gen[i] = q < i ? (shape[q] == shape[i] ? p->gen[q] : nullptr) : make_gen_axis(shape[i]);
   if (prec == FC_FP64) {

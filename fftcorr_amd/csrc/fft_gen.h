@@ -66,8 +66,8 @@ void launch_gen_cols(const GenAxis& ax, const cplx<Tin>* in, cplx<Tout>* out, co
 template <typename Tin, typename Tout, class Loader>
 void launch_gen_r2c(const GenAxis& ax, const Tin* in, int64_t ldi, cplx<Tout>* out, int64_t ldo,
                     int64_t nrows, int64_t grp, Loader ld, hipStream_t s);
-template <typename T>
-void launch_gen_c2r(const GenAxis& ax, const cplx<T>* in, int64_t ldi, T* out, int64_t ldo,
+template <typename T, typename Tout>
+void launch_gen_c2r(const GenAxis& ax, const cplx<T>* in, int64_t ldi, Tout* out, int64_t ldo,
                     int64_t nrows, int64_t grp, int nsel, int offm, hipStream_t s);
 
 }  // namespace fc

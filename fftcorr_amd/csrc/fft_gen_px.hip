@@ -11,7 +11,7 @@ namespace {
 
 template <typename T, typename TI, int MODE, int RM>
 __global__ void __launch_bounds__(512)
-    k_gen_px(GenPx<T> p, int tilesC, int tiles_per_batch, GenDev g) {
+    k_gen_px(PxArgs<T> p, int tilesC, int tiles_per_batch, GenDev g) {
   using C = cplx<T>;
   using CI = cplx<TI>;
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -107,7 +107,7 @@ __global__ void __launch_bounds__(512)
 }  // namespace
 
 template <typename T, typename TI, int MODE>
-void launch_gen_px(const GenAxis& ax, const GenPx<T>& p, hipStream_t s) {
+void launch_gen_px(const GenAxis& ax, const PxArgs<T>& p, hipStream_t s) {
   if (!gen_px_ok(ax)) fail(FC_ERR_RUNTIME, "internal: no fused x pass for this length");
   const size_t cl = sizeof(cplx<TI>) + (MODE == kModeInterlaced ? sizeof(cplx<T>) : 0);
   const int tc = gen_px_tile(ax, cl, sizeof(cplx<T>), 512);
@@ -127,9 +127,9 @@ void launch_gen_px(const GenAxis& ax, const GenPx<T>& p, hipStream_t s) {
 }
 
 #define FC_GEN_PX(T, TI)                                                                       \
-  template void launch_gen_px<T, TI, kModeAuto>(const GenAxis&, const GenPx<T>&, hipStream_t);  \
-  template void launch_gen_px<T, TI, kModeCross>(const GenAxis&, const GenPx<T>&, hipStream_t); \
-  template void launch_gen_px<T, TI, kModeInterlaced>(const GenAxis&, const GenPx<T>&, hipStream_t);
+  template void launch_gen_px<T, TI, kModeAuto>(const GenAxis&, const PxArgs<T>&, hipStream_t);  \
+  template void launch_gen_px<T, TI, kModeCross>(const GenAxis&, const PxArgs<T>&, hipStream_t); \
+  template void launch_gen_px<T, TI, kModeInterlaced>(const GenAxis&, const PxArgs<T>&, hipStream_t);
 FC_GEN_PX(double, double)
 FC_GEN_PX(float, float)
 FC_GEN_PX(float, double)

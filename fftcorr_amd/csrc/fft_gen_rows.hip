@@ -68,9 +68,9 @@ __global__ void __launch_bounds__(gen_max_threads<RM>())
 // sample (o - off) mod n2 at o < nsel (offm = off mod n2).  Every input of a
 // row is read in the first stage, so the real rows may overlay the complex
 // ones.
-template <typename T, bool BLUE, int RM>
+template <typename T, typename Tout, bool BLUE, int RM>
 __global__ void __launch_bounds__(gen_max_threads<RM>())
-    k_gen_c2r(const cplx<T>* in, int64_t ldi, T* out, int64_t ldo, int64_t nrows, int64_t grp,
+    k_gen_c2r(const cplx<T>* in, int64_t ldi, Tout* out, int64_t ldo, int64_t nrows, int64_t grp,
               int rs, int nsel, int offm, GenDev g) {
   using CL = cplx<typename std::conditional<BLUE, double, T>::type>;
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -95,15 +95,15 @@ __global__ void __launch_bounds__(gen_max_threads<RM>())
     if (!okb) b = double2{0.0, 0.0};
     return double2{a.x - b.y, -(a.y + b.x)};
   };
-  T* da = out + r0 * ldo;
+  Tout* da = out + r0 * ldo;
   const int last = nsel == 0 ? L : nsel;
   const int shift = nsel == 0 ? 0 : offm;
   auto put = [&](int r, int u, double2 v) {
     int o = j + r * u + shift;
     if (o >= L) o -= L;
     for (; o < last; o += L) {
-      if (oka) da[o] = T(v.x);
-      if (okb) da[ldo + o] = T(-v.y);
+      if (oka) da[o] = Tout(v.x);
+      if (okb) da[ldo + o] = Tout(-v.y);
     }
   };
   if constexpr (BLUE)
@@ -146,13 +146,13 @@ void launch_gen_r2c(const GenAxis& ax, const Tin* in, int64_t ldi, cplx<Tout>* o
   FC_LAUNCH_CHECK();
 }
 
-template <typename T>
-void launch_gen_c2r(const GenAxis& ax, const cplx<T>* in, int64_t ldi, T* out, int64_t ldo,
+template <typename T, typename Tout>
+void launch_gen_c2r(const GenAxis& ax, const cplx<T>* in, int64_t ldi, Tout* out, int64_t ldo,
                     int64_t nrows, int64_t grp, int nsel, int offm, hipStream_t s) {
   const RowShape r = row_shape(ax, ax.blue ? sizeof(double2) : sizeof(cplx<T>), nrows, grp);
   if (r.nb == 0) return;
   auto go = [&](auto blue, auto rm) {
-    hipLaunchKernelGGL((k_gen_c2r<T, decltype(blue)::value, decltype(rm)::value>), dim3(r.nb),
+    hipLaunchKernelGGL((k_gen_c2r<T, Tout, decltype(blue)::value, decltype(rm)::value>), dim3(r.nb),
                        dim3((unsigned)ax.tcol, (unsigned)r.tr), r.lds, s, in, ldi, out, ldo,
                        nrows, grp, r.rs, nsel, offm, gen_dev(ax));
   };
@@ -173,9 +173,12 @@ FC_GEN_R2C(double, float, LoadYlm)
 FC_GEN_R2C(float, double, LoadYlm)
 FC_GEN_R2C(double, double, LoadYlm)
 #undef FC_GEN_R2C
-template void launch_gen_c2r<float>(const GenAxis&, const float2*, int64_t, float*, int64_t,
-                                    int64_t, int64_t, int, int, hipStream_t);
-template void launch_gen_c2r<double>(const GenAxis&, const double2*, int64_t, double*, int64_t,
-                                     int64_t, int64_t, int, int, hipStream_t);
+#define FC_GEN_C2R(T, Tout)                                                                \
+  template void launch_gen_c2r<T, Tout>(const GenAxis&, const cplx<T>*, int64_t, Tout*,     \
+                                        int64_t, int64_t, int64_t, int, int, hipStream_t);
+FC_GEN_C2R(float, float)
+FC_GEN_C2R(double, double)
+FC_GEN_C2R(float, double)
+#undef FC_GEN_C2R
 
 }  // namespace fc

@@ -12,9 +12,9 @@
 //    complex values; the TC transforms run in LDS with E complex values per
 //    thread in registers between stages.
 //
-// Lengths 2^a (8..4096) and 3*2^a (24..3072) use compile-time radix plans;
-// every other length falls back to a direct O(L^2) DFT per column/row (used
-// for small or unusual test grids).  Forward transforms use sign -1 and no
+// Lengths 2^a (8..4096) and 3*2^a (192..3072) use compile-time radix plans;
+// every other length runs the mixed-radix passes (fft_gen.h) or, where those
+// are slower, a direct O(L^2) DFT per column/row.  Forward transforms use sign -1 and no
 // normalisation, the inverse sign +1 and no 1/N, matching FFTW's r2c/c2r as
 // called by the reference (cc/grid/fft_grid.cc:81-84).
 #pragma once
@@ -85,6 +85,24 @@ __device__ __forceinline__ void st_stream(V* p, V v) {
   e.x = v.x;
   e.y = v.y;
   __builtin_nontemporal_store(e, reinterpret_cast<typename NtVec<V>::type*>(p));
+}
+
+// Streaming hint only for accesses that cover whole 128-byte lines: the narrower
+// row segments of neighbouring tiles share lines, which then have to stay in L2
+// until the other tile has read or written its part.
+template <bool WHOLE, typename V>
+__device__ __forceinline__ V ld_seg(const V* p) {
+  if constexpr (WHOLE)
+    return ld_stream(p);
+  else
+    return *p;
+}
+template <bool WHOLE, typename V>
+__device__ __forceinline__ void st_seg(V* p, V v) {
+  if constexpr (WHOLE)
+    st_stream(p, v);
+  else
+    *p = v;
 }
 
 template <typename C>
@@ -226,6 +244,29 @@ struct Bfly<16, DIR, T> {
   }
 };
 
+// 12 = 4 x 3 without inner twiddles (Good 1958): input n = (3 n1 + 4 n2) mod
+// 12, output k with k = k1 mod 4 and k = k2 mod 3.
+template <int DIR, typename T>
+struct Bfly<12, DIR, T> {
+  using C = cplx<T>;
+  static __host__ __device__ __forceinline__ void run(C* v) {
+    C t[3][4];
+#pragma unroll
+    for (int n2 = 0; n2 < 3; ++n2) {
+#pragma unroll
+      for (int n1 = 0; n1 < 4; ++n1) t[n2][n1] = v[(3 * n1 + 4 * n2) % 12];
+      Bfly<4, DIR, T>::run(t[n2]);
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < 4; ++k1) {
+      C u[3] = {t[0][k1], t[1][k1], t[2][k1]};
+      Bfly<3, DIR, T>::run(u);
+#pragma unroll
+      for (int k2 = 0; k2 < 3; ++k2) v[(9 * k1 + 4 * k2) % 12] = u[k2];
+    }
+  }
+};
+
 template <int DIR, typename T>
 struct Bfly<3, DIR, T> {
   using C = cplx<T>;
@@ -265,23 +306,25 @@ FC_FFT_CFG(128, 8, 8, 8, 2)
 FC_FFT_CFG(256, 8, 8, 8, 4)
 FC_FFT_CFG(512, 8, 8, 8, 8)
 FC_FFT_CFG(1024, 8, 8, 8, 8, 2)
+FC_FFT_CFG(192, 12, 12, 4, 4)
+FC_FFT_CFG(384, 12, 12, 4, 4, 2)
+FC_FFT_CFG(768, 12, 12, 4, 4, 4)
+FC_FFT_CFG(1536, 12, 12, 4, 4, 4, 2)
+FC_FFT_CFG(3072, 12, 12, 4, 4, 4, 4)
 FC_FFT_CFG(2048, 8, 8, 8, 8, 4)
 FC_FFT_CFG(4096, 8, 8, 8, 8, 8)
-FC_FFT_CFG(24, 24, 8, 3)
-FC_FFT_CFG(48, 24, 8, 2, 3)
-FC_FFT_CFG(96, 24, 8, 4, 3)
-FC_FFT_CFG(192, 24, 8, 8, 3)
-FC_FFT_CFG(384, 24, 8, 8, 2, 3)
-FC_FFT_CFG(768, 24, 8, 8, 4, 3)
-FC_FFT_CFG(1536, 24, 8, 8, 8, 3)
-FC_FFT_CFG(3072, 24, 8, 8, 8, 2, 3)
 #undef FC_FFT_CFG
 
-// Plan variants of the register-chained kernels, chosen per pass by the
-// autotuner: 0 is the table above (first radix 8); 1 starts with radix 16
-// (16 values per thread, half the threads per column or row, and for
-// 256 = 16 x 16 one LDS exchange instead of two).
-constexpr int kFftVariants = 2;
+// Plan variants of the register-chained kernels.  0 is the table above and 1
+// starts with radix 16 (16 values per thread, half the threads per column or
+// row, and for 256 = 16 x 16 one LDS exchange instead of two): the autotuner
+// chooses between them per pass.  2 is the plan of the FP32 arithmetic at
+// 3 2^a points: 24 values per thread, radix 8 first and 3 last.  FP32 keeps this
+// order of operations because its rounding of the mean (the sum of a grid of
+// mostly empty cells) is a bias of every lag, and the order decides it; FP64
+// arithmetic takes variant 0, half the registers.
+constexpr int kFftVariants = 2;   // the autotuner's choices
+constexpr int kFftPlans = 3;
 template <int L, int V>
 struct FftCfgV : FftCfg<L> {};
 template <int L>
@@ -299,75 +342,33 @@ FC_FFT_CFG16(128, 16, 8)
 FC_FFT_CFG16(256, 16, 16)
 FC_FFT_CFG16(512, 16, 16, 2)
 #undef FC_FFT_CFG16
-
-// LDS addressing: element e of column c.
-struct LayColFast {  // [e][TC]: columns contiguous (strided y/x passes)
-  int tc;
-  __device__ __forceinline__ int operator()(int c, int e) const { return e * tc + c; }
+template <int L>
+struct FftCfgV<L, 2> {
+  static constexpr bool fast = false;
 };
-struct LayRow {  // [c][rs]: elements contiguous (row / z pass)
-  int rs;
-  __device__ __forceinline__ int operator()(int c, int e) const { return c * rs + e; }
-};
-
-// One Stockham stage of radix R on LDS column c, thread t of L/E.
-// Twiddle table tw[m] = exp(-2 pi i m / L), m < L.
-template <typename T, int L, int E, int R, int NS, int DIR, class Lay>
-__device__ __forceinline__ void stockham_stage(cplx<T>* lds, const cplx<T>* __restrict__ tw,
-                                               int c, int t, Lay lay) {
-  using C = cplx<T>;
-  constexpr int TCOL = L / E;
-  constexpr int NB = E / R;
-  constexpr int LR = L / R;
-  C v[E];
-#pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    const int j = t + b * TCOL;
-#pragma unroll
-    for (int r = 0; r < R; ++r) v[b * R + r] = lds[lay(c, j + r * LR)];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    const int j = t + b * TCOL;
-    const int k = j % NS;
-    if (NS > 1) {
-#pragma unroll
-      for (int r = 1; r < R; ++r) {
-        C w = tw[r * k * (L / (NS * R))];
-        if (DIR > 0) w.y = -w.y;
-        v[b * R + r] = cmul(v[b * R + r], w);
-      }
-    }
-    Bfly<R, DIR, T>::run(&v[b * R]);
-    const int base = (j / NS) * NS * R + k;
-#pragma unroll
-    for (int r = 0; r < R; ++r) lds[lay(c, base + r * NS)] = v[b * R + r];
-  }
-  __syncthreads();
-}
-
-template <typename T, int L, int E, int DIR, int NS, class Lay>
-__device__ __forceinline__ void run_stages(Radices<>, cplx<T>*, const cplx<T>*, int, int, Lay) {}
-
-template <typename T, int L, int E, int DIR, int NS, class Lay, int R, int... Rest>
-__device__ __forceinline__ void run_stages(Radices<R, Rest...>, cplx<T>* lds,
-                                           const cplx<T>* __restrict__ tw, int c, int t,
-                                           Lay lay) {
-  stockham_stage<T, L, E, R, NS, DIR>(lds, tw, c, t, lay);
-  run_stages<T, L, E, DIR, NS * R>(Radices<Rest...>{}, lds, tw, c, t, lay);
-}
-
-template <typename T, int L, int DIR, class Lay>
-__device__ __forceinline__ void fft_lds(cplx<T>* lds, const cplx<T>* __restrict__ tw, int c,
-                                        int t, Lay lay) {
-  run_stages<T, L, FftCfg<L>::E, DIR, 1>(typename FftCfg<L>::radices{}, lds, tw, c, t, lay);
+#define FC_FFT_CFG24(Lv, ...)               \
+  template <>                               \
+  struct FftCfgV<Lv, 2> {                   \
+    static constexpr bool fast = true;      \
+    static constexpr int E = 24;            \
+    using radices = Radices<__VA_ARGS__>;   \
+  };
+FC_FFT_CFG24(192, 8, 8, 3)
+FC_FFT_CFG24(384, 8, 8, 2, 3)
+FC_FFT_CFG24(768, 8, 8, 4, 3)
+FC_FFT_CFG24(1536, 8, 8, 8, 3)
+FC_FFT_CFG24(3072, 8, 8, 8, 2, 3)
+#undef FC_FFT_CFG24
+// The variant of arithmetic A where the autotuner has no say.
+template <typename A, int L>
+constexpr int fft_plan_of() {
+  return sizeof(A) == 4 && FftCfgV<L, 2>::fast ? 2 : 0;
 }
 
 // ---- register-chained Stockham passes -------------------------------------
-// For power-of-two lengths (first radix = E) thread t keeps E values of its
-// column or row in registers: before the first stage slot s holds element
-// t + s L/E, after the last stage (radix Rl) slot s holds element
+// Thread t keeps E values of its column or row in registers: before the first
+// stage slot s holds element t + in_m(s) L/E (t + s L/E when the first radix is
+// E), after the last stage (radix Rl) slot s holds element
 // t + out_m(s) L/E.  The first stage therefore reads global memory directly
 // and the last stage's outputs go straight to global memory (or to the next
 // fused step): two LDS passes fewer than the LDS-staged form above.
@@ -383,9 +384,24 @@ struct RadixInfo<Radices<R, R2, Rest...>> {
 };
 
 __host__ __device__ constexpr bool rc_len_ok(int L) {
-  return L >= 8 && L <= 512 && (L & (L - 1)) == 0;
+  return (L >= 8 && L <= 4096 && (L & (L - 1)) == 0) || L == 192 || L == 384 || L == 768 ||
+         L == 1536 || L == 3072;
 }
 
+// Before the first stage (radix R0) slot s = b R0 + r holds element
+// t + in_m(s) L/E; in_slot is its inverse.
+template <int L, int V = 0>
+__host__ __device__ constexpr int in_m(int s) {
+  constexpr int E = FftCfgV<L, V>::E;
+  constexpr int R0 = RadixInfo<typename FftCfgV<L, V>::radices>::first;
+  return s / R0 + (s % R0) * (E / R0);
+}
+template <int L, int V = 0>
+__host__ __device__ constexpr int in_slot(int m) {
+  constexpr int E = FftCfgV<L, V>::E;
+  constexpr int R0 = RadixInfo<typename FftCfgV<L, V>::radices>::first;
+  return (m % (E / R0)) * R0 + m / (E / R0);
+}
 template <int L, int V = 0>
 __host__ __device__ constexpr int out_m(int s) {
   constexpr int E = FftCfgV<L, V>::E;
@@ -587,24 +603,27 @@ void stage_twiddles_(Radices<R, Rest...>, Put put) {
 // Waves per SIMD a register-chained column kernel is held to when its
 // arithmetic is wider than its LDS tiles (the occupancy of the narrow form).
 // Variant 1 holds twice the values per thread and is sized for half the waves.
-template <typename T, typename To, int V = 0>
+// Plans of 12 values per thread hold half as many more.
+template <typename T, typename To, int V, int L>
 constexpr int rc_wide_waves() {
-  return sizeof(T) > sizeof(To) ? (V == 1 ? 4 : 8) : 1;
+  return sizeof(T) > sizeof(To) ? (V == 1 ? 4 : FftCfgV<L, V>::E > 8 ? 5 : 8) : 1;
 }
 
 template <typename T, int L, int DIR, int TC, typename Tin = T, typename To = T, int V = 0>
 __global__ void __launch_bounds__(TC*(L / FftCfgV<L, V>::E))
-__attribute__((amdgpu_waves_per_eu(rc_wide_waves<T, To, V>())))
+__attribute__((amdgpu_waves_per_eu(rc_wide_waves<T, To, V, L>())))
     k_fft_cols_rc(const cplx<Tin>* in, int64_t inA, int64_t inL, int64_t inG, cplx<To>* out,
                   int64_t outA, int64_t outL, int64_t outG, int B, int tilesB, int G, int nout,
                   int offm, const cplx<T>* __restrict__ tw) {
   using C = cplx<T>;
   constexpr int E = FftCfgV<L, V>::E;
   constexpr int TCOL = L / E;
-  using Rad = typename FftCfgV<L, V>::radices;
-  static_assert(RadixInfo<Rad>::first == E, "first radix must equal E");
+  // Tiles above 64 KB (the longest lengths) are static: dynamic LDS stops there.
+  constexpr size_t kTile = (size_t)L * TC * sizeof(cplx<To>);
+  constexpr bool kStatic = kTile > 65536;
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  cplx<To>* lds = reinterpret_cast<cplx<To>*>(smem_raw);
+  __shared__ __align__(16) unsigned char smem_big[kStatic ? kTile : 16];
+  cplx<To>* lds = reinterpret_cast<cplx<To>*>(kStatic ? smem_big : smem_raw);
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
   const int ag = tile / tilesB;
   const int b0 = (tile - ag * tilesB) * TC;
@@ -628,8 +647,9 @@ __attribute__((amdgpu_waves_per_eu(rc_wide_waves<T, To, V>())))
     cplx<Tin> xs[E];
 #pragma unroll
     for (int s = 0; s < E; ++s)
-      xs[s] = ld_stream(
-          reinterpret_cast<const cplx<Tin>*>(srcb + (cinc + (uint32_t)(t + s * TCOL) * inLb)));
+      xs[s] = ld_seg<TC * sizeof(cplx<Tin>) >= 128>(
+          reinterpret_cast<const cplx<Tin>*>(
+              srcb + (cinc + (uint32_t)(t + in_m<L, V>(s) * TCOL) * inLb)));
 #pragma unroll
     for (int s = 0; s < E; ++s) v[0][s] = colok ? C{T(xs[s].x), T(xs[s].y)} : C{T(0), T(0)};
   }
@@ -640,7 +660,7 @@ __attribute__((amdgpu_waves_per_eu(rc_wide_waves<T, To, V>())))
     int o = t + out_m<L, V>(s) * TCOL + offm;
     if (o >= L) o -= L;
     for (; o < nout; o += L)
-      st_stream(reinterpret_cast<cplx<To>*>(dstb + (cout + (uint32_t)o * outLb)),
+      st_seg<TC * sizeof(cplx<To>) >= 128>(reinterpret_cast<cplx<To>*>(dstb + (cout + (uint32_t)o * outLb)),
                 to_cplx<To>(v[0][s]));
   }
 }
@@ -839,8 +859,6 @@ __global__ void __launch_bounds__(1024)
   constexpr int E = FftCfgV<M, V>::E;
   constexpr int TCOL = M / E;
   constexpr int RS = row_pad_len(M);
-  using Rad = typename FftCfgV<M, V>::radices;
-  static_assert(RadixInfo<Rad>::first == E, "first radix must equal E");
   extern __shared__ __align__(16) unsigned char smem_raw[];
   cplx<To>* lds = reinterpret_cast<cplx<To>*>(smem_raw);
   const LayRowPad lay{RS};
@@ -858,10 +876,10 @@ __global__ void __launch_bounds__(1024)
     const auto lr = ld.row(rowc);
     P pv[E];
 #pragma unroll
-    for (int s = 0; s < E; ++s) pv[s] = ld_stream(src + t + s * TCOL);
+    for (int s = 0; s < E; ++s) pv[s] = ld_stream(src + t + in_m<M, V>(s) * TCOL);
 #pragma unroll
     for (int s = 0; s < E; ++s) {
-      const int e = t + s * TCOL;
+      const int e = t + in_m<M, V>(s) * TCOL;
       const C z{T(lr((double)pv[s].x, 2 * e)), T(lr((double)pv[s].y, 2 * e + 1))};
       v[0][s] = rowok ? z : C{T(0), T(0)};
     }
@@ -925,8 +943,6 @@ __global__ void __launch_bounds__(1024)
   constexpr int E = FftCfgV<M, V>::E;
   constexpr int TCOL = M / E;
   constexpr int RS = row_pad_len(M);
-  using Rad = typename FftCfgV<M, V>::radices;
-  static_assert(RadixInfo<Rad>::first == E, "first radix must equal E");
   extern __shared__ __align__(16) unsigned char smem_raw[];
   C* lds = reinterpret_cast<C*>(smem_raw);
   const LayRowPad lay{RS};
@@ -984,7 +1000,7 @@ __global__ void __launch_bounds__(1024)
   __syncthreads();
   C v[1][E];
 #pragma unroll
-  for (int s = 0; s < E; ++s) v[0][s] = lds[lay(c, t + s * TCOL)];
+  for (int s = 0; s < E; ++s) v[0][s] = lds[lay(c, t + in_m<M, V>(s) * TCOL)];
   __syncthreads();  // every first-stage input is read before the first stage stores
   rstages<T, M, +1, 1, 1, true, V>(v, lds, 0, twM, c, t, lay);
   if (!rowok) return;
@@ -1011,64 +1027,15 @@ __global__ void __launch_bounds__(1024)
   }
 }
 
-// ---- strided column pass ---------------------------------------------------
-// Transforms along L over [A][L][G][B] complex data (G groups of B contiguous
-// columns):
+// ---- direct sums --------------------------------------------------------------
+// Column views [A][L][G][B] (G groups of B contiguous columns):
 //   input  element (a, e, g, b) at a*inA  + e*inL  + g*inG  + b,
 //   output element (a, o, g, b) at a*outA + o*outL + g*outG + b,
 // with o in [0, nout).  off == 0 writes outputs o = e (nout == L: every
 // output); off != 0 writes outputs o < nout holding element e = (o - off)
 // mod L (the pruned inverse: only the lags a separation subgrid needs, off =
 // nout / 2; nout may equal or exceed L).  In place when in == out.
-// grid = (G * tilesB, A), tilesB = ceil(B / tc); block = tc * (L / E);
-// LDS = L * tc complex.
-// The input may be stored in another precision Tin (converted on load).
-template <typename T, int L, int DIR, typename Tin = T>
-__global__ void __launch_bounds__(1024)
-    k_fft_cols(const cplx<Tin>* in, int64_t inA, int64_t inL, int64_t inG, cplx<T>* out,
-               int64_t outA, int64_t outL, int64_t outG, int B, int tilesB, int tc, int nout,
-               int off, const cplx<T>* __restrict__ tw) {
-  using C = cplx<T>;
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  C* lds = reinterpret_cast<C*>(smem_raw);
-  const int g = blockIdx.x / tilesB;
-  const int b0 = (blockIdx.x - g * tilesB) * tc;
-  const int a = blockIdx.y;
-  const cplx<Tin>* src = in + (int64_t)a * inA + (int64_t)g * inG + b0;
-  C* dst = out + (int64_t)a * outA + (int64_t)g * outG + b0;
-  const int nthr = blockDim.x;
-  const int tid = threadIdx.x;
-  const int ncol = min(tc, B - b0);
-  // L * tc elements over tc * (L / E) threads: exactly E per thread, all
-  // loads issued before the first LDS store.
-  constexpr int E = FftCfg<L>::E;
-  {
-    C tmp[E];
-#pragma unroll
-    for (int q = 0; q < E; ++q) {
-      const int idx = tid + q * nthr;
-      const int e = idx / tc, c = idx - e * tc;
-      if (c < ncol) {
-        const cplx<Tin> x = src[e * inL + c];
-        tmp[q] = C{T(x.x), T(x.y)};
-      } else {
-        tmp[q] = C{T(0), T(0)};
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < E; ++q) lds[tid + q * nthr] = tmp[q];
-  }
-  __syncthreads();
-  fft_lds<T, L, DIR>(lds, tw, tid % tc, tid / tc, LayColFast{tc});
-  for (int idx = tid; idx < nout * tc; idx += nthr) {
-    const int o = idx / tc, c = idx - o * tc;
-    const int e = off == 0 ? o : ((o - off) % L + L) % L;
-    if (c < ncol) dst[o * outL + c] = lds[e * tc + c];
-  }
-}
-
-// Direct DFT fallback, one column per block (any L up to LDS capacity); same
-// data layout and pruning as k_fft_cols.  grid = (G * B, A).
+// Direct DFT, one column per block (any L up to LDS capacity).  grid = (G * B, A).
 template <typename T, int DIR, typename Tin = T>
 __global__ void __launch_bounds__(256)
     k_dft_cols(const cplx<Tin>* in, int64_t inA, int64_t inL, int64_t inG, cplx<T>* out,
@@ -1116,159 +1083,7 @@ struct LoadCopy {
   void shift_x(int) {}  // rows restart at a later x slab: nothing to adjust
 };
 
-// block = tr * (M / E) threads, handling rows blockIdx.x*tr ... ; LDS tr*(M+1).
-template <typename T, typename Tin, int M, class Loader>
-__global__ void __launch_bounds__(1024) k_fft_rows_r2c(const Tin* in, int64_t ldi,
-                                                       cplx<T>* out, int64_t ldo,
-                                                       int64_t nrows, int tr,
-                                                       const cplx<T>* __restrict__ twM,
-                                                       const cplx<T>* __restrict__ twN,
-                                                       Loader ld) {
-  using C = cplx<T>;
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  C* lds = reinterpret_cast<C*>(smem_raw);
-  constexpr int RS = M + 1;
-  const int64_t row0 = (int64_t)blockIdx.x * tr;
-  const int nthr = blockDim.x, tid = threadIdx.x;
-  // tr * M samples over tr * (M / E) threads: exactly E pairs per thread.
-  {
-    constexpr int E = FftCfg<M>::E;
-    C tmp[E];
-#pragma unroll
-    for (int q = 0; q < E; ++q) {
-      const int idx = tid + q * nthr;
-      const int c = idx / M, m = idx - c * M;
-      const int64_t row = row0 + c;
-      C z{T(0), T(0)};
-      if (row < nrows) {
-        const Tin* p = in + row * ldi + 2 * m;
-        const auto lr = ld.row(row);
-        z.x = T(lr((double)p[0], 2 * m));
-        z.y = T(lr((double)p[1], 2 * m + 1));
-      }
-      tmp[q] = z;
-    }
-#pragma unroll
-    for (int q = 0; q < E; ++q) {
-      const int idx = tid + q * nthr;
-      const int c = idx / M, m = idx - c * M;
-      lds[c * RS + m] = tmp[q];
-    }
-  }
-  __syncthreads();
-  constexpr int TCOL = M / FftCfg<M>::E;
-  fft_lds<T, M, -1>(lds, twM, tid / TCOL, tid % TCOL, LayRow{RS});
-  // Hermitian half: X[k] = (Z[k] + conj Z[M-k])/2 - i W^k (Z[k] - conj Z[M-k])/2
-  for (int idx = tid; idx < tr * (M + 1); idx += nthr) {
-    const int c = idx / (M + 1), k = idx - c * (M + 1);
-    const int64_t row = row0 + c;
-    if (row >= nrows) continue;
-    const C zk = lds[c * RS + (k == M ? 0 : k)];
-    const C zm = lds[c * RS + (k == 0 ? 0 : M - k)];
-    const T ax = zk.x + zm.x, ay = zk.y - zm.y;
-    const T bx = zk.x - zm.x, by = zk.y + zm.y;
-    const C w = twN[k];
-    const T px = w.x * by + w.y * bx;
-    const T py = -(w.x * bx - w.y * by);
-    out[row * ldo + k] = C{T(0.5) * (ax + px), T(0.5) * (ay + py)};
-  }
-}
-
-// Inverse: Hermitian half rows -> real rows (unnormalised; imaginary parts of
-// the DC and Nyquist terms are ignored, as FFTW's c2r does).
-// nsel == 0 writes the whole real row; nsel > 0 writes only samples
-// n = (o - off) mod 2M for o < nsel (the lags a separation subgrid needs).
-template <typename T, typename Tout, int M>
-__global__ void __launch_bounds__(1024) k_fft_rows_c2r(const cplx<T>* in, int64_t ldi,
-                                                       Tout* out, int64_t ldo,
-                                                       int64_t nrows, int tr,
-                                                       const cplx<T>* __restrict__ twM,
-                                                       const cplx<T>* __restrict__ twN,
-                                                       int nsel, int off) {
-  using C = cplx<T>;
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  C* lds = reinterpret_cast<C*>(smem_raw);
-  constexpr int RS = M + 1;
-  const int64_t row0 = (int64_t)blockIdx.x * tr;
-  const int nthr = blockDim.x, tid = threadIdx.x;
-  {
-    // Elements 0..M-1 of each row: exactly E per thread; element M below.
-    constexpr int E = FftCfg<M>::E;
-    C tmp[E];
-#pragma unroll
-    for (int q = 0; q < E; ++q) {
-      const int idx = tid + q * nthr;
-      const int c = idx / M, k = idx - c * M;
-      const int64_t row = row0 + c;
-      C x{T(0), T(0)};
-      if (row < nrows) x = in[row * ldi + k];
-      if (k == 0) x.y = T(0);
-      tmp[q] = x;
-    }
-#pragma unroll
-    for (int q = 0; q < E; ++q) {
-      const int idx = tid + q * nthr;
-      const int c = idx / M, k = idx - c * M;
-      lds[c * RS + k] = tmp[q];
-    }
-    if (tid < tr) {
-      const int64_t row = row0 + tid;
-      C x{T(0), T(0)};
-      if (row < nrows) x = in[row * ldi + M];
-      x.y = T(0);
-      lds[tid * RS + M] = x;
-    }
-  }
-  __syncthreads();
-  // Z[k] = (X[k] + conj X[M-k]) + i W^-k (X[k] - conj X[M-k]) for k < M,
-  // computed in pairs (p, M-p) so the update can be in place.
-  for (int idx = tid; idx < tr * (M / 2 + 1); idx += nthr) {
-    const int c = idx / (M / 2 + 1), p = idx - c * (M / 2 + 1);
-    const C xp = lds[c * RS + p];
-    const C xq = lds[c * RS + (M - p)];
-    const C wp = twN[p];       // exp(-2 pi i p / N); use conj -> W^-p
-    const C wq = twN[M - p];
-    // Z = A + i conj(w) B with A = X[k] + conj X[M-k], B = X[k] - conj X[M-k];
-    // conj(w) B = (w.x bx + w.y by, w.x by - w.y bx), and i (cx + i cy) = (-cy, cx).
-    {
-      const T ax = xp.x + xq.x, ay = xp.y - xq.y;
-      const T bx = xp.x - xq.x, by = xp.y + xq.y;
-      const T cx = wp.x * bx + wp.y * by, cy = wp.x * by - wp.y * bx;
-      lds[c * RS + p] = C{ax - cy, ay + cx};
-    }
-    if (p != 0 && p != M - p) {
-      const T ax = xq.x + xp.x, ay = xq.y - xp.y;
-      const T bx = xq.x - xp.x, by = xq.y + xp.y;
-      const T cx = wq.x * bx + wq.y * by, cy = wq.x * by - wq.y * bx;
-      lds[c * RS + (M - p)] = C{ax - cy, ay + cx};
-    }
-  }
-  __syncthreads();
-  constexpr int TCOL = M / FftCfg<M>::E;
-  fft_lds<T, M, +1>(lds, twM, tid / TCOL, tid % TCOL, LayRow{RS});
-  if (nsel == 0) {
-    for (int idx = tid; idx < tr * M; idx += nthr) {
-      const int c = idx / M, m = idx - c * M;
-      const int64_t row = row0 + c;
-      if (row >= nrows) continue;
-      const C z = lds[c * RS + m];
-      Tout* p = out + row * ldo + 2 * m;
-      p[0] = Tout(z.x);
-      p[1] = Tout(z.y);
-    }
-  } else {
-    const T* ldr = reinterpret_cast<const T*>(lds);
-    for (int idx = tid; idx < tr * nsel; idx += nthr) {
-      const int c = idx / nsel, o = idx - c * nsel;
-      const int64_t row = row0 + c;
-      if (row >= nrows) continue;
-      const int n = ((o - off) % (2 * M) + 2 * M) % (2 * M);
-      out[row * ldo + o] = Tout(ldr[2 * (c * RS) + n]);
-    }
-  }
-}
-
-// Direct-DFT fallback rows (any n2): one block per row.
+// Direct DFT rows (any n2): one block per row.
 template <typename T, typename Tin, class Loader>
 __global__ void __launch_bounds__(256) k_dft_rows_r2c(const Tin* in, int64_t ldi,
                                                       cplx<T>* out, int64_t ldo,

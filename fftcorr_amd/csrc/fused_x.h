@@ -7,6 +7,7 @@
 // cc/correlate/correlator.h:290-334 with cc/grid/fft_grid.cc:125-257.
 #pragma once
 
+#include "fc_internal.h"
 #include "fft_kernels.h"
 
 namespace fc {
@@ -26,6 +27,28 @@ struct KSlots {
     return ((int64_t)sx * ks1 + sy) * (ks2 / 2 + 1) + c;
   }
 };
+
+// One launch over nb members (member i reads A, B at i a_bstride and writes
+// pk, q at i pk_bstride, q_bstride; B is shared in cross mode).  T: storage of
+// the spectra and pk; TI: combine, inverse and q.
+template <typename T>
+struct PxArgs {
+  const cplx<T>*A, *B;
+  int n1, n2h;
+  int64_t ldc;
+  const double2 *ph0, *ph1, *ph2;
+  T* pk;
+  KSlots ks;
+  void* q;
+  int64_t ldq;
+  int rs, offm, nb;
+  int64_t a_bstride, pk_bstride, q_bstride;
+};
+// Fused x pass of a length with a compile-time plan (n0; tables tw, twi of the
+// axis in T and TI).  False if it does not take the arguments (fused_x.hip).
+template <typename T, typename TI, int MODE>
+bool launch_px_rc(int n0, const PxArgs<T>& p, const cplx<T>* tw, const cplx<TI>* twi,
+                  hipStream_t s);
 
 __device__ __forceinline__ int slot_a(int e, int o) { return e <= o ? e + o : -1; }
 __device__ __forceinline__ int slot_b(int e, int n, int o) {
@@ -56,14 +79,14 @@ __device__ __forceinline__ void put_pk(T* pk, const KSlots& ks, int n0, int n1, 
 // for x2_store_pk.  pyc: the y and z interlacing phases of this column
 // (interlaced mode); ph0: the x phases exp(i pi f / L) of the signed
 // frequencies f, loaded before the first use.
-template <typename T, typename TI, int L, int MODE, int NT, int NG>
-__device__ __forceinline__ void x2_combine(const cplx<T> (&v)[NT][FftCfg<L>::E],
+template <typename T, typename TI, int L, int MODE, int NT, int NG, int V = 0>
+__device__ __forceinline__ void x2_combine(const cplx<T> (&v)[NT][FftCfgV<L, V>::E],
                                            const cplx<T> (&g)[NG],
-                                           cplx<TI> (&u)[1][FftCfg<L>::E],
-                                           T (&pkv)[FftCfg<L>::E], const double2* ph0,
+                                           cplx<TI> (&u)[1][FftCfgV<L, V>::E],
+                                           T (&pkv)[FftCfgV<L, V>::E], const double2* ph0,
                                            double2 pyc, int t) {
   using CI = cplx<TI>;
-  constexpr int E = FftCfg<L>::E;
+  constexpr int E = FftCfgV<L, V>::E;
   constexpr int TCOL = L / E;
   // The x phase of element e = t + m L/E is ph0[t] ph0[m L/E]: with
   // ph0[a] = exp(i pi f(a) / L) for the signed frequency f, f(e) = t + f(m L/E)
@@ -75,7 +98,7 @@ __device__ __forceinline__ void x2_combine(const cplx<T> (&v)[NT][FftCfg<L>::E],
   if (MODE == kModeInterlaced) {
     pt = cmul(ph0[t], pyc);
 #pragma unroll
-    for (int s = 0; s < E; ++s) pm[s] = ph0[out_m<L>(s) * TCOL];
+    for (int s = 0; s < E; ++s) pm[s] = ph0[out_m<L, V>(s) * TCOL];
   }
   {
 #pragma clang fp contract(off)
@@ -96,7 +119,7 @@ __device__ __forceinline__ void x2_combine(const cplx<T> (&v)[NT][FftCfg<L>::E],
       } else {
         p = CI{ax * ax + ay * ay, TI(0)};
       }
-      u[0][out_m<L>(s)] = p;
+      u[0][in_slot<L, V>(out_m<L, V>(s))] = p;
       pkv[s] = (T)p.x;
     }
   }
@@ -105,7 +128,8 @@ __device__ __forceinline__ void x2_combine(const cplx<T> (&v)[NT][FftCfg<L>::E],
 // A uniform value the optimiser cannot see through: offsets built as
 // base + k * step from it stay additions (folding them back into
 // (t + k) * stride would cost a quarter-rate integer multiply per element).
-__device__ __forceinline__ uint32_t opaque_uniform(uint32_t x) {
+template <typename U>
+__device__ __forceinline__ U opaque_uniform(U x) {
   asm volatile("" : "+s"(x));
   return x;
 }
@@ -113,11 +137,11 @@ __device__ __forceinline__ uint32_t opaque_uniform(uint32_t x) {
 // Re P of slot s (pkv, from x2_combine) to every compact k slot that reads
 // element e = t + out_m(s) L/E of row y, column cg.  Issued after the inverse
 // pass, so no load of the pass waits behind these stores.
-template <typename T, int L>
-__device__ __forceinline__ void x2_store_pk(const T (&pkv)[FftCfg<L>::E], T* pk,
+template <typename T, int L, int V = 0>
+__device__ __forceinline__ void x2_store_pk(const T (&pkv)[FftCfgV<L, V>::E], T* pk,
                                             const KSlots& ks, int n1, int y, int cg, bool colok,
                                             int t) {
-  constexpr int E = FftCfg<L>::E;
+  constexpr int E = FftCfgV<L, V>::E;
   constexpr int TCOL = L / E;
   const int oz = ks.oz();
   if (!(colok && cg <= oz)) return;
@@ -140,11 +164,11 @@ __device__ __forceinline__ void x2_store_pk(const T (&pkv)[FftCfg<L>::E], T* pk,
   auto put = [&](uint32_t off, T val) { *reinterpret_cast<T*>(pkb + off) = val; };
 #pragma unroll
   for (int s = 0; s < E; ++s) {
-    const int e = t + out_m<L>(s) * TCOL;
+    const int e = t + out_m<L, V>(s) * TCOL;
     int sx0 = slot_a(e, ox), sx1 = slot_b(e, L, ox);
     if (sx1 == sx0) sx1 = -1;
     const T val = pkv[s];
-    const uint32_t ep = tp + (uint32_t)out_m<L>(s) * step;
+    const uint32_t ep = tp + (uint32_t)out_m<L, V>(s) * step;
     if (sx0 >= 0) {
       const uint32_t r = ep + r0;
       if (sy0 >= 0) put(r + prow0, val);
@@ -160,12 +184,12 @@ __device__ __forceinline__ void x2_store_pk(const T (&pkv)[FftCfg<L>::E], T* pk,
 
 // Pruned store of the inverse x pass: q[sx][y][cg] for every sx < rs holds
 // element (sx - off) mod L (offm = off mod L).
-template <typename TI, int L>
-__device__ __forceinline__ void x2_store_q(const cplx<TI> (&u)[1][FftCfg<L>::E], cplx<TI>* q,
+template <typename TI, int L, int V = 0>
+__device__ __forceinline__ void x2_store_q(const cplx<TI> (&u)[1][FftCfgV<L, V>::E], cplx<TI>* q,
                                            int n1, int y, int64_t ldq, int cg, int rs, int offm,
                                            int t) {
   using CI = cplx<TI>;
-  constexpr int E = FftCfg<L>::E;
+  constexpr int E = FftCfgV<L, V>::E;
   constexpr int TCOL = L / E;
   // Byte offset sx A + (y ldq + cg) |CI| with A = n1 ldq |CI|: one multiply
   // per thread, then uniform steps (32-bit arithmetic throughout).
@@ -179,8 +203,8 @@ __device__ __forceinline__ void x2_store_q(const cplx<TI> (&u)[1][FftCfg<L>::E],
   const uint32_t wrapA = opaque_uniform((uint32_t)L * A);
 #pragma unroll
   for (int s = 0; s < E; ++s) {
-    int sx = base + out_m<L>(s) * TCOL;
-    uint32_t off = o0 + (uint32_t)out_m<L>(s) * stepA;
+    int sx = base + out_m<L, V>(s) * TCOL;
+    uint32_t off = o0 + (uint32_t)out_m<L, V>(s) * stepA;
     if (sx >= L) {
       sx -= L;
       off -= wrapA;
@@ -190,29 +214,51 @@ __device__ __forceinline__ void x2_store_q(const cplx<TI> (&u)[1][FftCfg<L>::E],
 }
 
 // ---- the fused kernel -------------------------------------------------------
-// Columns per workgroup: 64 bytes of each row (8 FP32 or 4 FP64 complex).
-template <typename T>
-constexpr int px_tc() {
-  return 64 / (int)sizeof(cplx<T>);
-}
-// Lengths the fused kernel takes: power-of-two plans whose first radix is E.
+// Lengths the fused kernel takes: plans whose first radix is E.
 __host__ __device__ constexpr bool px_len_ok(int L) { return rc_len_ok(L); }
-template <typename T, int L>
+// LDS of tc columns: the forward tiles hold the storage type T, the inverse
+// tile TI.
+template <typename T, typename TI, int L, int MODE>
+constexpr size_t px_tile_bytes(int tc) {
+  constexpr int tiles = MODE == kModeInterlaced ? 2 : 1;
+  const size_t fwd = tiles * (size_t)L * tc * sizeof(cplx<T>);
+  const size_t inv = (size_t)L * tc * sizeof(cplx<TI>);
+  return fwd > inv ? fwd : inv;
+}
+// Plan variant of the pass (one for both transforms).
+template <typename T, typename TI, int L>
+constexpr int px_plan() {
+  return sizeof(T) == 4 && sizeof(TI) == 4 ? fft_plan_of<float, L>() : 0;
+}
+// Columns per workgroup: 64 bytes of each row (8 FP32 or 4 FP64 complex), or as
+// many as 64 KB of LDS hold (two workgroups per CU).
+template <typename T, typename TI, int L, int MODE>
+constexpr int px_tc() {
+  int tc = 64 / (int)sizeof(cplx<T>);
+  while (tc > 1 && px_tile_bytes<T, TI, L, MODE>(tc) > 65536) tc /= 2;
+  return tc;
+}
+template <typename T, typename TI, int L, int MODE>
 constexpr int px_threads() {
-  return px_tc<T>() * (L / FftCfg<L>::E);
+  return px_tc<T, TI, L, MODE>() * (L / FftCfgV<L, px_plan<T, TI, L>()>::E);
 }
-// Waves per SIMD the register budget is sized for: two workgroups per CU.
-template <typename T>
-constexpr int px_waves() {
-  return sizeof(T) == 4 ? 4 : 2;
-}
-// The forward tiles hold the storage type T; the inverse tile holds TI.
 template <typename T, typename TI, int L, int MODE>
 constexpr size_t px_lds_bytes() {
-  constexpr int tiles = MODE == kModeInterlaced ? 2 : 1;
-  constexpr size_t fwd = tiles * (size_t)L * px_tc<T>() * sizeof(cplx<T>);
-  constexpr size_t inv = (size_t)L * px_tc<T>() * sizeof(cplx<TI>);
-  return fwd > inv ? fwd : inv;
+  return px_tile_bytes<T, TI, L, MODE>(px_tc<T, TI, L, MODE>());
+}
+// Waves per SIMD the register budget is sized for: two workgroups per CU of the
+// plans with 8 or 12 values per thread; the 24 values of the FP32 form's plan
+// at 3 2^a points need the registers of two waves (384 points, cross: 381 us
+// with spills, 196 without).
+template <typename T, typename TI, int L>
+constexpr int px_waves() {
+  return sizeof(T) == 4 && px_plan<T, TI, L>() == 0 ? 4 : 2;
+}
+// Whether the stage twiddles are copied to LDS: not at 1024 points, whose two
+// tables (38 KB in the mixed form) would leave one workgroup per CU.
+template <int L>
+constexpr bool px_tw_lds() {
+  return L <= 768;
 }
 
 // One workgroup per (batch member, y row, tile of TC kz columns) of the work
@@ -228,10 +274,11 @@ constexpr size_t px_lds_bytes() {
 //   as TI): inverse x FFT at element (sx - off) mod L for every sx < rs
 //   (offm = off mod L; rs may exceed L, then elements repeat).
 // Loads, forward FFT (twiddles tw) and pk in T; combine, inverse and q in
-// TI (FP64 for the mixed form), twiddles twi.
-template <typename T, typename TI, int L, int MODE>
-__global__ void __launch_bounds__((px_threads<T, L>()))
-__attribute__((amdgpu_waves_per_eu(px_waves<T>())))
+// TI (FP64 for the mixed form), twiddles twi.  Off: byte offsets into the
+// spectra, 32 bits (one register) while a spectrum is below 4 GB.
+template <typename T, typename TI, int L, int MODE, class Off>
+__global__ void __launch_bounds__((px_threads<T, TI, L, MODE>()))
+__attribute__((amdgpu_waves_per_eu(px_waves<T, TI, L>())))
     k_periodic_x2(const cplx<T>* __restrict__ A, const cplx<T>* __restrict__ B, int n1, int n2h,
                   int64_t ldc, int tilesC, const cplx<T>* __restrict__ tw,
                   const cplx<TI>* __restrict__ twi, const double2* __restrict__ ph0,
@@ -241,13 +288,13 @@ __attribute__((amdgpu_waves_per_eu(px_waves<T>())))
                   int64_t q_bstride) {
   using C = cplx<T>;
   using CI = cplx<TI>;
-  constexpr int E = FftCfg<L>::E;
-  constexpr int TC = px_tc<T>();
+  constexpr int V = px_plan<T, TI, L>();
+  constexpr int E = FftCfgV<L, V>::E;
+  constexpr int TC = px_tc<T, TI, L, MODE>();
   constexpr int TCOL = L / E;
   constexpr int NT = MODE == kModeInterlaced ? 2 : 1;
-  using Rad = typename FftCfg<L>::radices;
-  using Lay = LaySwz<TC>;
-  static_assert(RadixInfo<Rad>::first == E, "first radix must equal E");
+  using Rad = typename FftCfgV<L, V>::radices;
+  using Lay = LaySwz<TC, E>;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   C* lds = reinterpret_cast<C*>(smem_raw);
   CI* ldsi = reinterpret_cast<CI*>(smem_raw);
@@ -255,11 +302,14 @@ __attribute__((amdgpu_waves_per_eu(px_waves<T>())))
   // workgroup in LDS (one table when T and TI agree: the same x length and
   // precision give the same values).  13.8 KB for 512 points in the mixed
   // form, so two workgroups still fit a CU beside their 64 KB tiles.
-  constexpr int SL = stage_twiddle_len<L, 0>();
+  constexpr int SL = stage_twiddle_len<L, V>();
+  constexpr int TB = L + stage_twiddle_base<L, V>();
   constexpr bool kSameTw = std::is_same<T, TI>::value;
-  __shared__ __align__(16) C twf[SL > 0 ? SL : 1];
-  __shared__ __align__(16) CI two[(SL > 0 && !kSameTw) ? SL : 1];
-  const CI* twl = kSameTw ? reinterpret_cast<const CI*>(twf) : two;
+  constexpr bool kTw = px_tw_lds<L>() && SL > 0;
+  __shared__ __align__(16) C twfs[kTw ? SL : 1];
+  __shared__ __align__(16) CI twos[(kTw && !kSameTw) ? SL : 1];
+  const C* twf = kTw ? twfs : tw + TB;
+  const CI* twl = !kTw ? twi + TB : kSameTw ? reinterpret_cast<const CI*>(twfs) : twos;
 
   const int tile_all = xcd_tile(blockIdx.x, gridDim.x);
   const int bat = tile_all / tiles_per_batch;
@@ -274,15 +324,11 @@ __attribute__((amdgpu_waves_per_eu(px_waves<T>())))
   const int c = threadIdx.x % TC, t = threadIdx.x / TC;
   const int cg = c0 + c;
   const bool colok = c < ncol;
-  // Byte offsets stay below 4 GB (checked by the launcher): 32-bit address
-  // arithmetic on a uniform base.
-  const uint32_t sL = (uint32_t)n1 * (uint32_t)ldc * (uint32_t)sizeof(C);
+  const Off sL = (Off)n1 * (Off)ldc * (Off)sizeof(C);
   // Columns past n2h read column c0 (discarded): the loads are unconditional
   // and issue back to back; row offsets are base + s TCOL sL.
-  const uint32_t base =
-      ((uint32_t)y * (uint32_t)ldc + (uint32_t)(colok ? cg : c0)) * (uint32_t)sizeof(C) +
-      (uint32_t)t * sL;
-  const uint32_t stepL = opaque_uniform((uint32_t)TCOL * sL);
+  const Off base = ((Off)y * (Off)ldc + (Off)(colok ? cg : c0)) * (Off)sizeof(C) + (Off)t * sL;
+  const Off stepL = opaque_uniform((Off)TCOL * sL);
   const char* Ab = reinterpret_cast<const char*>(A);
   const char* Bb = reinterpret_cast<const char*>(B);
 
@@ -290,13 +336,13 @@ __attribute__((amdgpu_waves_per_eu(px_waves<T>())))
   C g[MODE == kModeCross ? E : 1];
 #pragma unroll
   for (int s = 0; s < E; ++s) {
-    const uint32_t o = base + (uint32_t)s * stepL;
+    const Off o = base + (Off)in_m<L, V>(s) * stepL;
     // Plain loads: the two tiles of a 128-byte line (64 bytes each) are read
     // by neighbouring workgroups of one XCD, the second from its L2.
     v[0][s] = *reinterpret_cast<const C*>(Ab + o);
     if (NT == 2) v[NT - 1][s] = *reinterpret_cast<const C*>(Bb + o);
     if (MODE == kModeCross)
-      g[s] = *reinterpret_cast<const C*>(Bb + base + (uint32_t)out_m<L>(s) * stepL);
+      g[s] = *reinterpret_cast<const C*>(Bb + base + (Off)out_m<L, V>(s) * stepL);
   }
   if (!colok) {
 #pragma unroll
@@ -309,11 +355,12 @@ __attribute__((amdgpu_waves_per_eu(px_waves<T>())))
   // The twiddle copies wait for their loads, which come after (and so wait
   // for) the input loads the first stage needs anyway; the first stage's
   // closing barrier orders them before any stage reads them.
-  for (int i = threadIdx.x; i < SL; i += blockDim.x) {
-    twf[i] = tw[L + i];
-    if constexpr (!kSameTw) two[i] = twi[L + i];
-  }
-  rstages_<T, L, -1, NT, 1, 0, true, 0, NT, Lay, C, 0, BarWg>(Rad{}, v, lds, L * TC, twf, c, t,
+  if constexpr (kTw)
+    for (int i = threadIdx.x; i < SL; i += blockDim.x) {
+      twfs[i] = tw[TB + i];
+      if constexpr (!kSameTw) twos[i] = twi[TB + i];
+    }
+  rstages_<T, L, -1, NT, 1, 0, true, 0, NT, Lay, C, V, BarWg>(Rad{}, v, lds, L * TC, twf, c, t,
                                                              Lay{});
 
   // Combine: slot s holds element e = t + out_m(s) L/E of both spectra.
@@ -321,11 +368,11 @@ __attribute__((amdgpu_waves_per_eu(px_waves<T>())))
   if (MODE == kModeInterlaced) pyc = cmul(ph1[y], ph2[colok ? cg : 0]);
   CI u[1][E];
   T pkv[E];
-  x2_combine<T, TI, L, MODE, NT, (MODE == kModeCross ? E : 1)>(v, g, u, pkv, ph0, pyc, t);
+  x2_combine<T, TI, L, MODE, NT, (MODE == kModeCross ? E : 1), V>(v, g, u, pkv, ph0, pyc, t);
   __syncthreads();  // the forward pass's last LDS reads precede the inverse's stores
-  rstages_<TI, L, +1, 1, 1, 0, true, 0, 1, Lay, CI, 0, BarWg>(Rad{}, u, ldsi, 0, twl, c, t, Lay{});
-  x2_store_pk<T, L>(pkv, pk, ks, n1, y, cg, colok, t);
-  if (colok) x2_store_q<TI, L>(u, q, n1, y, ldq, cg, rs, offm, t);
+  rstages_<TI, L, +1, 1, 1, 0, true, 0, 1, Lay, CI, V, BarWg>(Rad{}, u, ldsi, 0, twl, c, t, Lay{});
+  x2_store_pk<T, L, V>(pkv, pk, ks, n1, y, cg, colok, t);
+  if (colok) x2_store_q<TI, L, V>(u, q, n1, y, ldq, cg, rs, offm, t);
 }
 
 // ---- persistent cross-mode fused x pass with direct-to-LDS prefetch ---------
@@ -354,14 +401,14 @@ __global__ void __launch_bounds__(8 * (L / 8))
   using C = cplx<T>;
   using CI = cplx<TI>;
   constexpr int E = FftCfg<L>::E;
-  constexpr int TC = px_tc<T>();
+  constexpr int TC = 8;
   constexpr int TCOL = L / E;
   constexpr int SL = stage_twiddle_len<L, 0>();
   constexpr size_t RAW = 2 * (size_t)L * TC * sizeof(C);  // rows of A, then of B
   constexpr size_t INV = (size_t)L * TC * sizeof(CI);
   constexpr size_t BUF = RAW > INV ? RAW : INV;
   using Rad = typename FftCfg<L>::radices;
-  using Lay = LaySwz<TC>;
+  using Lay = LaySwz<TC, E>;
   static_assert(E == 8 && TC * sizeof(C) == 64, "64-byte rows of 8 FP32 columns");
   __shared__ __align__(16) unsigned char bufA[BUF];
   __shared__ __align__(16) unsigned char bufB[BUF];
