@@ -12,42 +12,32 @@
 //      at most 8 bits over the bits the largest key needs): within a key
 //      cell the particles keep their input order;
 //   3. k_permute      records in sorted order;
-//   4. k_cell_runs    per occupied key cell, its run {first sorted particle,
-//                     count} (one 8-byte entry) and its bit in an occupancy
-//                     bitmap (cleared first; the run table is read only where
-//                     the bit is set, so it needs no clearing);
-//   5. k_ma_tile      one workgroup per 4 x 4 x 32 tile of target cells lists
+//   4. k_row_bounds   per grid row (x, y), the sorted particles at the borders
+//                     of its z tiles (binary searches);
+//   5. k_ma_tile      one wave per 8 x 32 tile of target cells of an x plane:
 //                     the particles of every key cell whose stencil reaches
-//                     the tile, in key-cell order; each wave takes a contiguous
-//                     quarter of the list, 64 particles at a time, forms their
-//                     stencil weights and sums them per key cell with a
-//                     segmented scan across lanes (a fixed tree).  The last
-//                     lane of each key cell's segment adds the sums to the
-//                     wave's own FP64 copy of the tile in LDS (distinct key
-//                     cells, so no two lanes hit one target cell in a step);
-//                     the four copies are added in wave order and each touched
-//                     grid cell is read and written once.
-// No floating-point atomics and no order that depends on scheduling: repeated
-// runs give identical bits.  Each particle record is read by the tiles its
-// stencil reaches (1.3-1.5x on average), never once per target cell.
+//                     the tile, an equal share per lane, summed in registers
+//                     and then in an FP64 copy of the tile in LDS; each
+//                     touched grid cell is read and written once.
+// (The D12 wavelet's gather finds its particles per key cell instead, by
+// k_cell_runs.)
+// No floating-point atomics on memory and no order that depends on
+// scheduling: repeated runs give identical bits.
 
 #include <mutex>
 #include <vector>
 
 #include "fc_objects.h"
 #include "radix_sort.h"
+#include "xcd.h"
 
 namespace fc {
 namespace {
 
 constexpr int kPrepThreads = 256;
-#ifndef FC_MA_TILE_Y
-#define FC_MA_TILE_Y 4
-#endif
-constexpr int TX = 4, TY = FC_MA_TILE_Y, TZ = 32;  // target tile of k_ma_tile
-constexpr int kTileCells = TX * TY * TZ;
+constexpr int TY = 8, TZ = 32;  // target tile of one wave of k_ma_tile, in one x plane
 constexpr int kTileThreads = 256;
-constexpr int kTileWaves = kTileThreads / kWave;
+constexpr int kTileWaves = kTileThreads / kWave;  // consecutive x planes of a workgroup
 
 struct GridGeom {
   int n0, n1, n2;
@@ -71,6 +61,13 @@ __device__ __forceinline__ bool to_grid(double p, double pmin, double cell, int 
   return true;
 }
 
+// Orders a wave's LDS accesses across its lanes (they execute in order; this
+// keeps the compiler from moving them).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Key cell and offset along one axis: a = floor(x - anchor), wrapped into
 // [0, n), and r = (x - anchor) - floor(x - anchor) in [0, 1).  anchor is 0
 // (NGP, TSC, D12: the cell holding the particle) or 1/2 (CIC: the lower of the
@@ -90,7 +87,8 @@ __device__ __forceinline__ int key_axis(double x, double anchor, int n, double* 
 __global__ void __launch_bounds__(kPrepThreads)
     k_ma_prepare(const double* __restrict__ pos, int64_t n, int ncol,
                  const double* __restrict__ weights, double w_scalar, GridGeom g, int wrap,
-                 double shift, double anchor, uint32_t sentinel, uint32_t* __restrict__ keys,
+                 double shift, double anchor, bool keep_z, uint32_t sentinel,
+                 uint32_t* __restrict__ keys,
                  uint32_t* __restrict__ idx, double4* __restrict__ rec,
                  double* __restrict__ part_w, unsigned long long* __restrict__ part_n) {
 #pragma clang fp contract(off)
@@ -127,7 +125,7 @@ __global__ void __launch_bounds__(kPrepThreads)
     const int iy = key_axis(y, anchor, g.n1, &ry);
     const int iz = key_axis(z, anchor, g.n2, &rz);
     keys[i] = (uint32_t)(((uint64_t)ix * g.n1 + iy) * g.n2 + iz);
-    rec[i] = make_double4(rx, ry, rz, w);
+    rec[i] = make_double4(rx, ry, keep_z ? z - anchor : rz, w);
     tw += w;
     tw2 += w * w;
     added += 1;
@@ -259,193 +257,241 @@ struct Stencil<3> {  // CIC about cell centres: key cell a <= x - 1/2 < a + 1
   }
 };
 
+// First sorted particle at the z borders of the planes' tiles, per grid row
+// (x, y): entries 2b and 2b + 1 bound the key cells that reach tile b from
+// inside the row, entry 2 ntz starts the row's last key cell and entry
+// 2 ntz + 1 ends its first one (the ranges that reach the row's other end
+// through the periodic wrap).
+__host__ __device__ inline int row_bounds(int n2) { return 2 * ((n2 + TZ - 1) / TZ) + 2; }
+
+template <int SCHEME>
+__global__ void k_row_bounds(const uint32_t* __restrict__ keys,
+                             const unsigned long long* __restrict__ nvalid_p, int64_t nrows,
+                             int n2, int32_t* __restrict__ bounds) {
+  using S = Stencil<SCHEME>;
+  const int nb = row_bounds(n2), ntz = nb / 2 - 1;
+  const int nvalid = (int)*nvalid_p;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nrows * nb;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t row = i / nb;
+    const int j = (int)(i - row * nb), b = j >> 1;
+    int z;
+    if (b < ntz)
+      z = (j & 1) ? min(b * TZ + TZ - S::OMIN, n2) : max(b * TZ - S::OMAX, 0);
+    else
+      z = (j & 1) ? 1 : n2 - 1;
+    const uint32_t key = (uint32_t)(row * n2 + z);
+    int lo = 0, hi = nvalid;  // keys[lo - 1] < key <= keys[hi]
+    while (lo < hi) {
+      const int mid = lo + (hi - lo) / 2;
+      if (keys[mid] < key)
+        lo = mid + 1;
+      else
+        hi = mid;
+    }
+    bounds[i] = lo;
+  }
+}
+
+// One wave per TY x TZ tile of target cells of one x plane, without any
+// barrier.  The key cells that reach the tile are W RY rows, each up to three
+// ranges of the sorted particles (inside the row, and through the wrap from
+// either end).  Lane l takes the l-th of 64 equal shares of the concatenated
+// ranges and walks it in order, summing the W x W weights of one key cell in
+// registers; when the key cell changes it adds them to the wave's FP64 copies
+// of the tile in LDS, one per plane of key cells.  Two lanes never hit one
+// address in one instruction: key cells of one plane differ in their targets
+// for each of the W x W offsets, and a key cell spread over several lanes ends
+// inside the share of one of them only, the others hold it at the end of their
+// share and add it after the loop, one lane after the other.  So each target
+// cell is summed in an order that the input alone decides.
+//
+// Bound by the latency of a tile's chain (bounds, records, LDS adds) and by
+// the lanes a sparse tile leaves idle, not by memory: hence no barrier, grid
+// cells requested first, and the wave order of the XCDs, which lets the tiles
+// that share rows meet in one L2.  20 million particles CIC into 512^3 FP32
+// 0.77 ms (2.06 ms with a workgroup per 4 x 4 x 32 tile and a segmented scan
+// across lanes); 3 million clustered particles TSC into 256^3 FP64 0.21 ms
+// (0.80 ms).  Four rows instead of eight: 0.79 and 0.24 ms.
 template <typename Tg, int SCHEME>
 __global__ void __launch_bounds__(kTileThreads)
-    k_ma_tile(Tg* __restrict__ grid, GridGeom g, const int2* __restrict__ runs,
-              const uint32_t* __restrict__ occ, const double4* __restrict__ srec, int tiles_y,
-              int tiles_z) {
+    k_ma_tile(Tg* __restrict__ grid, GridGeom g, const int32_t* __restrict__ bounds,
+              const double4* __restrict__ srec, int tiles_y, int tiles_z) {
 #pragma clang fp contract(off)
   using S = Stencil<SCHEME>;
   constexpr int W = S::OMAX - S::OMIN + 1;
-  // Key cells whose stencil reaches the tile: [t0 - OMAX, t0 + T - 1 - OMIN].
-  constexpr int RX = TX + W - 1, RY = TY + W - 1, RZ = TZ + W - 1;
-  constexpr int RC = RX * RY * RZ;
-  constexpr int kPer = (RC + kTileThreads - 1) / kTileThreads;
-  __shared__ int32_t pre[RC + 1];  // counts, then their exclusive prefix sums
-  __shared__ int32_t bg[RC];
-  __shared__ double acc[kTileWaves][kTileCells];
-  __shared__ uint32_t touched[kTileCells / 32];
-  __shared__ int32_t wtot[kTileWaves];
+  constexpr int RY = TY + W - 1;                   // key rows that reach the tile, per key plane
+  constexpr int PY = TY + 2 * (W - 1), PZ = TZ + 2 * (W - 1);  // tile with the stencils' margin
+  constexpr int NROW = W * RY, NKIND = W, NQ = NROW * NKIND;
+  constexpr int kChunks = (NQ + kWave - 1) / kWave;
+  __shared__ double acc_s[kTileWaves][W * PY * PZ];  // one copy per key plane
+  __shared__ int32_t first_s[kTileWaves][kChunks * kWave];    // first particle of each range
+  __shared__ int32_t pre_s[kTileWaves][kChunks * kWave + 1];  // exclusive prefix of their lengths
 
-  int b = blockIdx.x;
+  int b = xcd_tile((int)blockIdx.x, (int)gridDim.x);
   const int bz = b % tiles_z;
   b /= tiles_z;
   const int by = b % tiles_y;
   const int bx = b / tiles_y;
-  const int x0 = bx * TX, y0 = by * TY, z0 = bz * TZ;
-  const int tid = threadIdx.x, lane = tid % kWave, wv = tid / kWave;
+  const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave;
+  const int x = bx * kTileWaves + wv, y0 = by * TY, z0 = bz * TZ;
+  if (x >= g.n0) return;
+  double* acc = acc_s[wv];
+  int32_t* first = first_s[wv];
+  int32_t* pre = pre_s[wv];
+  const int nb = row_bounds(g.n2);
 
-  // Run tables of the key cells: every occupancy word is requested before the
-  // first is used, then the runs of the occupied cells, so a thread waits for
-  // two rounds of loads rather than one per cell.
-  {
-    int64_t cell[kPer];
-    uint32_t word[kPer];
+  int begin[kChunks], len[kChunks];
 #pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      const int rc = tid + q * kTileThreads;
-      cell[q] = -1;
-      word[q] = 0u;
-      if (rc < RC) {
-        const int rz = rc % RZ, ry = (rc / RZ) % RY, rx = rc / (RZ * RY);
-        const int gx = wrap_index(x0 - S::OMAX + rx, g.n0);
-        const int gy = wrap_index(y0 - S::OMAX + ry, g.n1);
-        const int gz = wrap_index(z0 - S::OMAX + rz, g.n2);
-        cell[q] = ((int64_t)gx * g.n1 + gy) * g.n2 + gz;
-        word[q] = occ[cell[q] >> 5];
-      }
+  for (int c = 0; c < kChunks; ++c) {
+    const int q = c * kWave + lane;
+    const int kind = q / NROW, row = q % NROW;
+    const int y = y0 - S::OMAX + row % RY;
+    bool on = q < NQ && y < g.n1 - S::OMIN;
+    int lo = 2 * bz, hi = 2 * bz + 1;
+    if (kind == 1) {  // the last key cell of the row reaches its first target cell
+      on = on && bz == 0;
+      lo = nb - 2;
+      hi = nb - 3;
+    } else if (kind == 2) {  // the first key cell reaches the last target cell
+      on = on && bz == tiles_z - 1;
+      lo = 0;
+      hi = nb - 1;
     }
-    int2 run[kPer];
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      const bool on = cell[q] >= 0 && ((word[q] >> (cell[q] & 31)) & 1u);
-      run[q] = on ? runs[cell[q]] : make_int2(0, 0);
-    }
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      const int rc = tid + q * kTileThreads;
-      if (rc < RC) {
-        pre[rc] = run[q].y;
-        bg[rc] = run[q].x;
-      }
+    begin[c] = len[c] = 0;
+    if (on) {
+      const int gx = wrap_index(x - S::OMAX + row / RY, g.n0);
+      const int32_t* t = bounds + ((int64_t)gx * g.n1 + wrap_index(y, g.n1)) * nb;
+      begin[c] = t[lo];
+      len[c] = t[hi] - begin[c];
     }
   }
-  __syncthreads();
-  // Exclusive scan of the counts: thread t owns entries [t kPer, (t+1) kPer).
-  int loc[kPer];
-  int s = 0;
+  int total = 0;
 #pragma unroll
-  for (int q = 0; q < kPer; ++q) {
-    const int i = tid * kPer + q;
-    loc[q] = i < RC ? pre[i] : 0;
-    s += loc[q];
-  }
-  int incl = s;
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const int t = __shfl_up(incl, d, kWave);
-    if (lane >= d) incl += t;
-  }
-  if (lane == kWave - 1) wtot[wv] = incl;
-  __syncthreads();
-  int run = incl - s, total = 0;
-#pragma unroll
-  for (int w = 0; w < kTileWaves; ++w) {
-    if (w < wv) run += wtot[w];
-    total += wtot[w];
-  }
-#pragma unroll
-  for (int q = 0; q < kPer; ++q) {
-    const int i = tid * kPer + q;
-    if (i < RC) pre[i] = run;
-    run += loc[q];
-  }
-  if (tid == 0) pre[RC] = total;
-  if (total == 0) return;  // uniform: no particle reaches this tile
-  for (int i = tid; i < kTileWaves * kTileCells; i += kTileThreads) (&acc[0][0])[i] = 0.0;
-  for (int i = tid; i < kTileCells / 32; i += kTileThreads) touched[i] = 0u;
-  __syncthreads();
-
-  // Wave wv sums list entries [p0, p1) into its copy acc[wv].
-  const int p0 = (int)((int64_t)total * wv / kTileWaves);
-  const int p1 = (int)((int64_t)total * (wv + 1) / kTileWaves);
-  double* mine = acc[wv];
-  for (int base = p0; base < p1; base += kWave) {
-    const int p = base + lane;
-    const bool valid = p < p1;
-    int rc = -1;
-    double wx[W], wy[W], wz[W];
-#pragma unroll
-    for (int o = 0; o < W; ++o) wx[o] = wy[o] = wz[o] = 0.0;
-    if (valid) {
-      int lo = 0, hi = RC;  // pre[lo] <= p < pre[hi]
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (pre[mid] <= p)
-          lo = mid;
-        else
-          hi = mid;
-      }
-      rc = lo;
-      const double4 q = srec[bg[rc] + (p - pre[rc])];
-      S::weights(q.x, wx);
-      S::weights(q.y, wy);
-      S::weights(q.z, wz);
-#pragma unroll
-      for (int o = 0; o < W; ++o) wx[o] = wx[o] * q.w;  // weight folded into x, as the reference
-    }
-    // Segments: runs of lanes with the same key cell (rc); sstart = first lane.
-    const int prev = __shfl_up(rc, 1, kWave);
-    const int next = __shfl_down(rc, 1, kWave);
-    const bool head = lane == 0 || prev != rc;
-    const bool tail = valid && (lane == kWave - 1 || next != rc);
-    int sstart = head ? lane : 0;
+  for (int c = 0; c < kChunks; ++c) {
+    int incl = len[c];
 #pragma unroll
     for (int d = 1; d < kWave; d <<= 1) {
-      const int t = __shfl_up(sstart, d, kWave);
-      if (lane >= d) sstart = max(sstart, t);
+      const int t = __shfl_up(incl, d, kWave);
+      if (lane >= d) incl += t;
     }
-    const bool singles = __ballot(valid && !head) == 0ull;  // wave-uniform
-    const int rz = rc % RZ, ry = (rc / RZ) % RY, rx = rc / (RZ * RY);
-#pragma unroll
-    for (int a = 0; a < W; ++a) {
-      const int tx = rx + a - (W - 1);
-#pragma unroll
-      for (int bb = 0; bb < W; ++bb) {
-        const int ty = ry + bb - (W - 1);
-        const double vxy = wx[a] * wy[bb];
-#pragma unroll
-        for (int c = 0; c < W; ++c) {
-          const int tz = rz + c - (W - 1);
-          double v = vxy * wz[c];
-          if (!singles) {
-#pragma unroll
-            for (int d = 1; d < kWave; d <<= 1) {
-              const double t = __shfl_up(v, d, kWave);
-              if (lane - d >= sstart) v += t;
-            }
-          }
-          if (tail && tx >= 0 && tx < TX && ty >= 0 && ty < TY && tz >= 0 && tz < TZ &&
-              x0 + tx < g.n0 && y0 + ty < g.n1 && z0 + tz < g.n2) {
-            const int t = (tx * TY + ty) * TZ + tz;
-            mine[t] += v;
-            atomicOr(&touched[t >> 5], 1u << (t & 31));
-          }
-        }
-      }
-    }
+    first[c * kWave + lane] = begin[c];
+    pre[c * kWave + lane] = total + incl - len[c];
+    total += __shfl(incl, kWave - 1, kWave);
   }
-  __syncthreads();
-  // Each thread's touched cells: all grid loads first, then the stores.
-  constexpr int kOut = kTileCells / kTileThreads;
+  if (total == 0) return;  // no particle reaches this tile
+  if (lane == 0) pre[kChunks * kWave] = total;
+  for (int i = lane; i < W * PY * PZ; i += kWave) acc[i] = -0.0;  // -0 + v == v; see the store
+  // The tile's own grid cells, requested before the particles.
+  constexpr int kOut = TY * TZ / kWave;
   Tg old[kOut];
   Tg* dst[kOut];
 #pragma unroll
   for (int q = 0; q < kOut; ++q) {
-    const int t = tid + q * kTileThreads;
-    const int tz = t % TZ, ty = (t / TZ) % TY, tx = t / (TZ * TY);
-    const bool on = (touched[t >> 5] >> (t & 31)) & 1u;
-    dst[q] = on ? grid + ((int64_t)(x0 + tx) * g.n1 + (y0 + ty)) * g.n2 + (z0 + tz) : nullptr;
-    old[q] = on ? *dst[q] : Tg(0);
+    const int tz = lane % TZ, ty = (lane + q * kWave) / TZ;
+    dst[q] = y0 + ty < g.n1 && z0 + tz < g.n2
+                 ? grid + ((int64_t)x * g.n1 + (y0 + ty)) * g.n2 + (z0 + tz)
+                 : nullptr;
+    old[q] = dst[q] ? *dst[q] : Tg(0);
   }
+  wave_lds_fence();
+
+  const int share = (total - 1) / kWave + 1;
+  const int64_t p0 = (int64_t)lane * share;
+  int left = (int)(p0 >= total ? 0 : total - p0 < share ? total - p0 : share);
+  int q = 0, idx = 0, in_range = 0;
+  double4 next = make_double4(0, 0, 0, 0);
+  if (left > 0) {
+    int hi = kChunks * kWave;  // pre[q] <= p0 < pre[hi]
+    while (hi - q > 1) {
+      const int mid = (q + hi) >> 1;
+      if (pre[mid] <= p0)
+        q = mid;
+      else
+        hi = mid;
+    }
+    idx = first[q] + (int)(p0 - pre[q]);
+    in_range = pre[q + 1] - (int)p0;
+    next = srec[idx];
+  }
+  const bool any = left > 0;
+  double v[W][W];
+#pragma unroll
+  for (int bb = 0; bb < W; ++bb)
+#pragma unroll
+    for (int c = 0; c < W; ++c) v[bb][c] = 0.0;
+  int held = -1;  // key cell of v: its corner target in its plane's copy
+  auto flush = [&] {
+    double* t = acc + held;
+#pragma unroll
+    for (int bb = 0; bb < W; ++bb)
+#pragma unroll
+      for (int c = 0; c < W; ++c)
+        __hip_atomic_fetch_add(t + bb * PZ + c, v[bb][c], __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  for (int j = 0; j < share; ++j) {
+    if (left > 0) {
+      const double4 p = next;
+      const int kind = q / NROW, row = q % NROW, rx = row / RY, ry = row % RY;
+      // Advance; the next record is on its way while this one is summed.
+      ++idx;
+      if (--left > 0) {
+        if (--in_range == 0) {
+          do {
+            ++q;
+            in_range = pre[q + 1] - pre[q];
+          } while (in_range == 0);
+          idx = first[q];
+        }
+        next = srec[idx];
+      }
+      const double fz = floor(p.z);
+      int iz = (int)fz;
+      if (iz < 0) iz += g.n2;
+      const int rz = iz + S::OMAX - (kind == 0 ? z0 : kind == 1 ? g.n2 : z0 - g.n2);
+      const int cell = (rx * PY + ry) * PZ + rz;
+      double wx[W], wy[W], wz[W];
+      S::weights(p.x, wx);
+      S::weights(p.y, wy);
+      S::weights(p.z - fz, wz);
+      double wa = wx[W - 1];  // the key plane x - OMAX + rx adds with weight W - 1 - rx
+#pragma unroll
+      for (int o = 1; o < W; ++o) wa = rx == o ? wx[W - 1 - o] : wa;
+      wa = wa * p.w;  // weight folded into x, as the reference
+      if (cell != held) {
+        if (held >= 0) flush();
+        held = cell;
+#pragma unroll
+        for (int bb = 0; bb < W; ++bb)
+#pragma unroll
+          for (int c = 0; c < W; ++c) v[bb][c] = 0.0;
+      }
+#pragma unroll
+      for (int bb = 0; bb < W; ++bb) {
+        const double vxy = wa * wy[bb];
+#pragma unroll
+        for (int c = 0; c < W; ++c) v[bb][c] += vxy * wz[c];
+      }
+    }
+  }
+  // What each lane still holds: equal key cells sit in neighbouring lanes.
+  const int prev = __shfl_up(held, 1, kWave);
+  const unsigned long long heads = __ballot(lane == 0 || prev != held);
+  const unsigned long long upto = heads & (~0ull >> (kWave - 1 - lane));
+  const int rank = any ? lane - (kWave - 1 - __clzll((long long)upto)) : -1;
+  for (int r = 0; __ballot(rank >= r) != 0ull; ++r)
+    if (rank == r) flush();
+  wave_lds_fence();
+  // A sum that is still -0 had no particle: adding it would change nothing.
 #pragma unroll
   for (int q = 0; q < kOut; ++q) {
-    if (!dst[q]) continue;
-    const int t = tid + q * kTileThreads;
-    double sum = acc[0][t];
+    const int tz = lane % TZ, ty = (lane + q * kWave) / TZ;
+    double add = acc[(ty + W - 1) * PZ + tz + W - 1];
 #pragma unroll
-    for (int w = 1; w < kTileWaves; ++w) sum += acc[w][t];
-    *dst[q] = (Tg)((double)old[q] + sum);
+    for (int c = 1; c < W; ++c) add += acc[(c * PY + ty + W - 1) * PZ + tz + W - 1];
+    if (dst[q] && __double_as_longlong(add) != (long long)0x8000000000000000ull)
+      *dst[q] = (Tg)((double)old[q] + add);
   }
 }
 
@@ -533,30 +579,35 @@ const double* wavelet_on_device(fc_ctx* ctx) {
 }
 
 template <typename Tg>
-void launch_gather(int scheme, Tg* grid, const GridGeom& gg, const int2* runs,
-                   const uint32_t* occ, const double4* srec, hipStream_t s,
-                   const double* table = nullptr) {
-  const bool wav = scheme == 2;
-  const int bx = wav ? WTX : TX, by = wav ? WTY : TY, bz = wav ? WTZ : TZ;
-  const int tx = (gg.n0 + bx - 1) / bx, ty = (gg.n1 + by - 1) / by, tz = (gg.n2 + bz - 1) / bz;
+void launch_wavelet(Tg* grid, const GridGeom& gg, const int2* runs, const uint32_t* occ,
+                    const double4* srec, hipStream_t s, const double* table) {
+  const int tx = (gg.n0 + WTX - 1) / WTX, ty = (gg.n1 + WTY - 1) / WTY,
+            tz = (gg.n2 + WTZ - 1) / WTZ;
   const uint64_t nb = (uint64_t)tx * ty * tz;
   if (nb > 0x7fffffffULL) fail(FC_ERR_INVALID, "grid too large for mass assignment");
-  dim3 grd((unsigned)nb), blk(wav ? WTX * WTY * WTZ : kTileThreads);
-  switch (scheme) {
-    case 0:
-      hipLaunchKernelGGL((k_ma_tile<Tg, 0>), grd, blk, 0, s, grid, gg, runs, occ, srec, ty, tz);
-      break;
-    case 1:
-      hipLaunchKernelGGL((k_ma_tile<Tg, 1>), grd, blk, 0, s, grid, gg, runs, occ, srec, ty, tz);
-      break;
-    case 3:
-      hipLaunchKernelGGL((k_ma_tile<Tg, 3>), grd, blk, 0, s, grid, gg, runs, occ, srec, ty, tz);
-      break;
-    case 2:
-      hipLaunchKernelGGL((k_ma_gather_wavelet<Tg>), grd, blk, 0, s, grid, gg, runs, occ, srec,
-                         table, ty, tz);
-      break;
-  }
+  hipLaunchKernelGGL((k_ma_gather_wavelet<Tg>), dim3((unsigned)nb), dim3(WTX * WTY * WTZ), 0, s,
+                     grid, gg, runs, occ, srec, table, ty, tz);
+  FC_LAUNCH_CHECK();
+}
+
+template <int SCHEME>
+void launch_tiles(fc_grid* grid, const GridGeom& gg, const uint32_t* skeys,
+                  const unsigned long long* nvalid, int32_t* bounds, const double4* srec,
+                  hipStream_t s, hipEvent_t sorted) {
+  const int64_t nrows = (int64_t)gg.n0 * gg.n1;
+  const int ty = (gg.n1 + TY - 1) / TY, tz = (gg.n2 + TZ - 1) / TZ;
+  const uint64_t nb = (uint64_t)((gg.n0 + kTileWaves - 1) / kTileWaves) * ty * tz;
+  if (nb > 0x7fffffffULL) fail(FC_ERR_INVALID, "grid too large for mass assignment");
+  hipLaunchKernelGGL((k_row_bounds<SCHEME>), dim3(grid1d(nrows * row_bounds(gg.n2), 256)),
+                     dim3(256), 0, s, skeys, nvalid, nrows, gg.n2, bounds);
+  FC_LAUNCH_CHECK();
+  FC_HIP(hipEventRecord(sorted, s));
+  if (grid->prec == FC_FP64)
+    hipLaunchKernelGGL((k_ma_tile<double, SCHEME>), dim3((unsigned)nb), dim3(kTileThreads), 0, s,
+                       grid->data.as<double>(), gg, bounds, srec, ty, tz);
+  else
+    hipLaunchKernelGGL((k_ma_tile<float, SCHEME>), dim3((unsigned)nb), dim3(kTileThreads), 0, s,
+                       grid->data.as<float>(), gg, bounds, srec, ty, tz);
   FC_LAUNCH_CHECK();
 }
 
@@ -565,6 +616,17 @@ int key_bits(uint64_t sentinel) {
   while (b < 64 && (sentinel >> b) != 0) ++b;
   return b;
 }
+
+// Bytes of the table that finds the sorted particles of a key cell: row
+// bounds, or (D12 wavelet) a run per cell and the occupancy bits.
+struct RunScratch {
+  size_t runs, occ = 0;
+  RunScratch(const int* shape, bool wavelet) {
+    const size_t rows = (size_t)shape[0] * shape[1], cells = rows * shape[2];
+    runs = wavelet ? sizeof(int2) * cells : sizeof(int32_t) * rows * row_bounds(shape[2]);
+    if (wavelet) occ = sizeof(uint32_t) * ((cells + 31) / 32);
+  }
+};
 
 void mass_assign(fc_grid* grid, const double* pos_dev, int64_t n, int ncol,
                  const double* w_dev, double w_scalar, int scheme, int wrap, double shift,
@@ -610,15 +672,15 @@ void mass_assign(fc_grid* grid, const double* pos_dev, int64_t n, int ncol,
   sc[6].reserve(sizeof(double4) * n);
   sc[7].reserve(sizeof(double) * 2 * (nbp + 1));
   sc[8].reserve(sizeof(unsigned long long) * (nbp + 1));
-  const uint64_t nwords = (ncells + 31) / 32;
-  sc[9].reserve(sizeof(int2) * ncells);
-  sc[11].reserve(sizeof(uint32_t) * nwords);
+  const RunScratch rs(grid->shape, scheme == 2);
+  sc[9].reserve(rs.runs);
+  sc[11].reserve(rs.occ);
   DeviceBuffer &keys = sc[1], &keys2 = sc[2], &idx = sc[3], &idx2 = sc[4], &rec = sc[5],
                &srec = sc[6], &partw = sc[7], &partn = sc[8], &runs = sc[9], &occ = sc[11];
   const double anchor = scheme == 3 ? 0.5 : 0.0;  // CIC keys by its 2x2x2 block
 
   hipLaunchKernelGGL(k_ma_prepare, dim3(nbp), dim3(kPrepThreads), 0, s, pos_dev, n, ncol, w_dev,
-                     w_scalar, gg, wrap, shift, anchor, (uint32_t)sentinel, keys.as<uint32_t>(),
+                     w_scalar, gg, wrap, shift, anchor, scheme != 2, (uint32_t)sentinel, keys.as<uint32_t>(),
                      idx.as<uint32_t>(), rec.as<double4>(), partw.as<double>(),
                      partn.as<unsigned long long>());
   FC_LAUNCH_CHECK();
@@ -638,19 +700,28 @@ void mass_assign(fc_grid* grid, const double* pos_dev, int64_t n, int ncol,
   hipLaunchKernelGGL(k_permute, dim3(grid1d(n, 256, 65536)), dim3(256), 0, s, sidx,
                      rec.as<double4>(), srec.as<double4>(), n);
   FC_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_zero_i32, dim3(grid1d(nwords, 256, 65536)), dim3(256), 0, s,
-                     occ.as<int32_t>(), (int64_t)nwords);
-  FC_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_cell_runs, dim3(grid1d(n, 256, 65536)), dim3(256), 0, s, skeys,
-                     partn.as<unsigned long long>() + nbp, runs.as<int2>(), occ.as<uint32_t>());
-  FC_LAUNCH_CHECK();
-  FC_HIP(hipEventRecord(ev[1], s));
-  if (grid->prec == FC_FP64)
-    launch_gather<double>(scheme, grid->data.as<double>(), gg, runs.as<int2>(),
-                          occ.as<uint32_t>(), srec.as<double4>(), s, wtab);
-  else
-    launch_gather<float>(scheme, grid->data.as<float>(), gg, runs.as<int2>(),
-                         occ.as<uint32_t>(), srec.as<double4>(), s, wtab);
+  const unsigned long long* nvalid = partn.as<unsigned long long>() + nbp;
+  if (scheme == 2) {
+    const int64_t nwords = (int64_t)(rs.occ / sizeof(uint32_t));
+    hipLaunchKernelGGL(k_zero_i32, dim3(grid1d(nwords, 256, 65536)), dim3(256), 0, s,
+                       occ.as<int32_t>(), nwords);
+    FC_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_cell_runs, dim3(grid1d(n, 256, 65536)), dim3(256), 0, s, skeys, nvalid,
+                       runs.as<int2>(), occ.as<uint32_t>());
+    FC_LAUNCH_CHECK();
+    FC_HIP(hipEventRecord(ev[1], s));
+    if (grid->prec == FC_FP64)
+      launch_wavelet(grid->data.as<double>(), gg, runs.as<int2>(), occ.as<uint32_t>(),
+                     srec.as<double4>(), s, wtab);
+    else
+      launch_wavelet(grid->data.as<float>(), gg, runs.as<int2>(), occ.as<uint32_t>(),
+                     srec.as<double4>(), s, wtab);
+  } else {
+    const auto launch = scheme == 0   ? launch_tiles<0>
+                        : scheme == 1 ? launch_tiles<1>
+                                      : launch_tiles<3>;
+    launch(grid, gg, skeys, nvalid, runs.as<int32_t>(), srec.as<double4>(), s, ev[1]);
+  }
   FC_HIP(hipEventRecord(ev[2], s));
 
   double wsum[2];
@@ -711,6 +782,7 @@ int fc_mass_assign_footprint(fc_grid* grid, int64_t n, int ncol, int has_weights
       const uint64_t ncells = grid->size();
       const int nbp = (int)std::min<int64_t>(1024, (n + fc::kPrepThreads - 1) / fc::kPrepThreads);
       const size_t temp = fc::radix_plan(n, fc::key_bits(ncells)).scratch_bytes();
+      const fc::RunScratch tiles(grid->shape, false), wavelet(grid->shape, true);
       const size_t want[12] = {temp,
                                sizeof(uint32_t) * n,
                                sizeof(uint32_t) * n,
@@ -720,9 +792,9 @@ int fc_mass_assign_footprint(fc_grid* grid, int64_t n, int ncol, int has_weights
                                sizeof(double4) * n,
                                sizeof(double) * 2 * (nbp + 1),
                                sizeof(unsigned long long) * (nbp + 1),
-                               sizeof(int2) * ncells,
+                               std::max(tiles.runs, wavelet.runs),
                                0,
-                               sizeof(uint32_t) * ((ncells + 31) / 32)};
+                               wavelet.occ};
       for (int i = 0; i < 12; ++i)
         if (want[i] > ctx->scratch[i].bytes()) g += want[i] - ctx->scratch[i].bytes();
     }
