@@ -37,14 +37,6 @@ int fft_radices(int L, int var, int* out) {
     case 128: return radices_of<128>(var, out);
     case 256: return radices_of<256>(var, out);
     case 512: return radices_of<512>(var, out);
-    case 1024: return radices_of<1024>(var, out);
-    case 192: return radices_of<192>(var, out);
-    case 384: return radices_of<384>(var, out);
-    case 768: return radices_of<768>(var, out);
-    case 1536: return radices_of<1536>(var, out);
-    case 2048: return radices_of<2048>(var, out);
-    case 3072: return radices_of<3072>(var, out);
-    case 4096: return radices_of<4096>(var, out);
     default: return 0;
   }
 }
