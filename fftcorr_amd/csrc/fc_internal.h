@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "../../include/fftcorr_hip.h"
+#include "host_copy.h"
 
 namespace fc {
 
@@ -150,6 +151,7 @@ struct fc_ctx {
   hipStream_t stream = nullptr;
   // Scratch reused across calls on this context (sort temp storage, staging).
   fc::DeviceBuffer scratch[12];  // per-context work buffers, grown on demand
+  std::unique_ptr<fc::HostCopier> copier;  // staged copies of host arrays, on first use
   fc::DeviceBuffer wavelet;       // D12 sample table on this device
   uint64_t wavelet_ver = 0;       // version of the process-wide table it holds
   int arch_cus = 0;

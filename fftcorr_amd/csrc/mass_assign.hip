@@ -670,7 +670,7 @@ void mass_assign(fc_grid* grid, const double* pos_dev, int64_t n, int ncol,
   sc[4].reserve(sizeof(uint32_t) * n);
   sc[5].reserve(sizeof(double4) * n);
   sc[6].reserve(sizeof(double4) * n);
-  sc[7].reserve(sizeof(double) * 2 * (nbp + 1));
+  sc[7].reserve(sizeof(double) * 2 * (nbp + 2));
   sc[8].reserve(sizeof(unsigned long long) * (nbp + 1));
   const RunScratch rs(grid->shape, scheme == 2);
   sc[9].reserve(rs.runs);
@@ -684,9 +684,11 @@ void mass_assign(fc_grid* grid, const double* pos_dev, int64_t n, int ncol,
                      idx.as<uint32_t>(), rec.as<double4>(), partw.as<double>(),
                      partn.as<unsigned long long>());
   FC_LAUNCH_CHECK();
+  // The sums of w and w^2 and the number of particles on the grid, read back as one.
+  unsigned long long* nvalid =
+      reinterpret_cast<unsigned long long*>(partw.as<double>() + 2 * nbp + 2);
   hipLaunchKernelGGL(k_ma_finish_stats, dim3(1), dim3(64), 0, s, partw.as<double>(),
-                     partn.as<unsigned long long>(), nbp, partw.as<double>() + 2 * nbp,
-                     partn.as<unsigned long long>() + nbp);
+                     partn.as<unsigned long long>(), nbp, partw.as<double>() + 2 * nbp, nvalid);
   FC_LAUNCH_CHECK();
 
   FC_HIP(hipEventRecord(ev[0], s));
@@ -700,7 +702,6 @@ void mass_assign(fc_grid* grid, const double* pos_dev, int64_t n, int ncol,
   hipLaunchKernelGGL(k_permute, dim3(grid1d(n, 256, 65536)), dim3(256), 0, s, sidx,
                      rec.as<double4>(), srec.as<double4>(), n);
   FC_LAUNCH_CHECK();
-  const unsigned long long* nvalid = partn.as<unsigned long long>() + nbp;
   if (scheme == 2) {
     const int64_t nwords = (int64_t)(rs.occ / sizeof(uint32_t));
     hipLaunchKernelGGL(k_zero_i32, dim3(grid1d(nwords, 256, 65536)), dim3(256), 0, s,
@@ -724,13 +725,12 @@ void mass_assign(fc_grid* grid, const double* pos_dev, int64_t n, int ncol,
   }
   FC_HIP(hipEventRecord(ev[2], s));
 
-  double wsum[2];
-  unsigned long long nadd = 0;
+  double wsum[3];
   FC_HIP(hipMemcpyAsync(wsum, partw.as<double>() + 2 * nbp, sizeof(wsum),
                         hipMemcpyDeviceToHost, s));
-  FC_HIP(hipMemcpyAsync(&nadd, partn.as<unsigned long long>() + nbp, sizeof(nadd),
-                        hipMemcpyDeviceToHost, s));
   FC_HIP(hipStreamSynchronize(s));
+  unsigned long long nadd = 0;
+  std::memcpy(&nadd, &wsum[2], sizeof(nadd));
   float t_sort = 0, t_win = 0;
   FC_HIP(hipEventElapsedTime(&t_sort, ev[0], ev[1]));
   FC_HIP(hipEventElapsedTime(&t_win, ev[1], ev[2]));
@@ -790,19 +790,16 @@ int fc_mass_assign_footprint(fc_grid* grid, int64_t n, int ncol, int has_weights
                                sizeof(uint32_t) * n,
                                sizeof(double4) * n,
                                sizeof(double4) * n,
-                               sizeof(double) * 2 * (nbp + 1),
+                               sizeof(double) * 2 * (nbp + 2),
                                sizeof(unsigned long long) * (nbp + 1),
                                std::max(tiles.runs, wavelet.runs),
-                               0,
+                               host_input ? sizeof(double) * n * (ncol + (has_weights ? 1 : 0)) : 0,
                                wavelet.occ};
       for (int i = 0; i < 12; ++i)
         if (want[i] > ctx->scratch[i].bytes()) g += want[i] - ctx->scratch[i].bytes();
     }
     if (grow) *grow = g;
-    if (transient)
-      *transient = host_input && n > 0
-                       ? sizeof(double) * (size_t)n * (ncol + (has_weights ? 1 : 0))
-                       : 0;
+    if (transient) *transient = 0;
   });
 }
 
@@ -827,15 +824,14 @@ int fc_mass_assign(fc_grid* grid, const double* pos, int64_t n, int ncol,
     if (n <= 0) return;
     fc::DeviceGuard dg(grid->ctx->device);
     hipStream_t s = grid->ctx->stream;
-    fc::DeviceBuffer dpos(sizeof(double) * n * ncol);
-    fc::DeviceBuffer dw(weights ? sizeof(double) * n : 0);
-    FC_HIP(hipMemcpyAsync(dpos.as<void>(), pos, sizeof(double) * n * ncol,
-                          hipMemcpyHostToDevice, s));
-    if (weights)
-      FC_HIP(hipMemcpyAsync(dw.as<void>(), weights, sizeof(double) * n, hipMemcpyHostToDevice,
-                            s));
-    fc::mass_assign(grid, dpos.as<double>(), n, ncol, weights ? dw.as<double>() : nullptr,
-                    w_scalar, scheme, periodic_wrap, shift, stats);
+    fc_ctx* ctx = grid->ctx;
+    ctx->scratch[10].reserve(sizeof(double) * n * (ncol + (weights ? 1 : 0)));
+    double* dpos = ctx->scratch[10].as<double>();
+    double* dw = weights ? dpos + n * ncol : nullptr;
+    if (!ctx->copier) ctx->copier.reset(new fc::HostCopier(ctx->device));
+    FC_HIP(ctx->copier->copy(dpos, pos, sizeof(double) * n * ncol, s));
+    if (weights) FC_HIP(ctx->copier->copy(dw, weights, sizeof(double) * n, s));
+    fc::mass_assign(grid, dpos, n, ncol, dw, w_scalar, scheme, periodic_wrap, shift, stats);
   });
 }
 

@@ -90,6 +90,7 @@ int fc_ctx_destroy(fc_ctx* ctx) {
     if (!ctx) return;
     fc::DeviceGuard g(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
+    ctx->copier.reset();
     for (auto& b : ctx->scratch) b.release();
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;

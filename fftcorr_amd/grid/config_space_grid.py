@@ -114,6 +114,7 @@ class ConfigSpaceGrid:
         self._host_refs = sys.getrefcount(self._host)
         self._dev = None
         self._host_valid = True
+        self._cleared = False  # the device copy is known to hold zeros
         self._dev_valid = False
         _log.info("grid %s, cell %.6g, posmin %s, posmax %s", self._shape, cell, lo.tolist(),
                   hi.tolist())
@@ -141,13 +142,16 @@ class ConfigSpaceGrid:
     def _device_modified(self):
         """Called after device work changed the grid."""
         self._dev_valid = True
-        self._host_valid = False
+        self._host_valid = self._cleared = False
         if self._view_held():
             self._sync_host()
 
     def _sync_host(self):
         if not self._host_valid:
-            self._dev.download(self._host)
+            if self._cleared:
+                self._host.fill(0.0)
+            else:
+                self._dev.download(self._host)
             self._host_valid = True
 
     # ---- reference API -----------------------------------------------------
@@ -203,11 +207,17 @@ class ConfigSpaceGrid:
         return "fp64" if self._precision == _lib.FC_FP64 else "fp32"
 
     def clear(self):
-        self._host.fill(0.0)
-        self._host_valid = True
-        if self._dev is not None:
+        if self._dev is None:
+            self._host.fill(0.0)
+            self._host_valid = True
+        else:
+            # The host copy is written when it is read next, unless device
+            # work has changed the grid by then.
             self._dev.clear()
-            self._dev_valid = True
+            self._dev_valid = self._cleared = True
+            self._host_valid = False
+            if self._view_held():
+                self._sync_host()
         self._metadata.clear()
 
     def sum(self):
@@ -259,7 +269,8 @@ class ConfigSpaceGrid:
 
     # ---- in-place arithmetic ---------------------------------------------------
     def _inplace(self, other, op, dev_op):
-        device_current = self._dev is not None and self._dev_valid and not self._host_valid
+        device_current = self._dev is not None and self._dev_valid and not (
+            self._host_valid or self._cleared)
         if np.isscalar(other) and dev_op is not None and device_current \
                 and not self._view_held():
             dev_op(float(other))

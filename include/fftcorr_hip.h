@@ -128,8 +128,9 @@ int fc_mass_assign(fc_grid* grid, const double* pos, int64_t n, int ncol,
                    int periodic_wrap, double shift, fc_ma_stats* stats);
 /* Device memory a call of n particles on this grid needs beyond what its
  * context holds: *grow = growth of the context's reused work buffers (kept
- * after the call), *transient = staging of host inputs (host_input = 1, as
- * fc_mass_assign; freed on return).  No reference counterpart. */
+ * after the call; host_input = 1, as fc_mass_assign, counts the device copy of
+ * the host inputs), *transient = buffers freed on return (none).  No reference
+ * counterpart. */
 int fc_mass_assign_footprint(fc_grid* grid, int64_t n, int ncol, int has_weights,
                              int host_input, size_t* grow, size_t* transient);
 /* Same, with pos/weights already in device memory (HBM-resident catalogs). */
