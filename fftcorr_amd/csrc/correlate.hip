@@ -67,6 +67,7 @@ struct fc_corr {
   fc::DeviceBuffer rsub, ksub;  // FP64 subgrids (Yamamoto accumulation)
   fc::DeviceBuffer ph[3];       // interlacing phase per axis
   // Outputs.
+  fc::DeviceBuffer outputs;  // one allocation, see OutLayout; the next are views of it
   fc::DeviceBuffer r_counts, r_hist, k_counts, k_hist, zerolag;
   fc::HistScratch hs;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -410,19 +411,29 @@ void fill(V* p, int64_t n, V v, hipStream_t s) {
   FC_LAUNCH_CHECK();
 }
 
-// Zeroes up to 5 arrays of 32-bit words in one launch (the per-correlation
-// histogram outputs), block y = array.
-struct ZeroSegs {
-  uint32_t* p[5];
-  int64_t n[5];
+// The outputs of one correlation as one run of doubles, cleared by one launch
+// and read back by one copy: r histogram, k histogram, zero lag, then the
+// int32 counts (r, k).
+struct OutLayout {
+  int64_t nr, nk;
+  explicit OutLayout(const fc_corr* c)
+      : nr((int64_t)c->nell * c->nrbins), nk((int64_t)c->nell * c->nkbins) {}
+  int64_t k_hist() const { return nr; }
+  int64_t zerolag() const { return nr + nk; }
+  int64_t r_counts() const { return nr + nk + 1; }  // nr + nk int32 from here
+  int64_t doubles() const { return r_counts() + (nr + nk + 1) / 2; }
+  // Copies the wanted outputs out of a run read back.
+  void unpack(const char* run, double* r_hist, int* r_cnt, double* k_hst, int* k_cnt,
+              double* zero) const {
+    const double* d = reinterpret_cast<const double*>(run);
+    const int* n = reinterpret_cast<const int*>(d + r_counts());
+    if (r_hist) std::copy(d, d + nr, r_hist);
+    if (k_hst) std::copy(d + k_hist(), d + k_hist() + nk, k_hst);
+    if (zero) *zero = d[zerolag()];
+    if (r_cnt) std::copy(n, n + nr, r_cnt);
+    if (k_cnt) std::copy(n + nr, n + nr + nk, k_cnt);
+  }
 };
-__global__ void k_zero_segs(ZeroSegs z) {
-  uint32_t* p = z.p[blockIdx.y];
-  const int64_t n = z.n[blockIdx.y];
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = 0u;
-}
 
 // ---- host orchestration -----------------------------------------------------
 // Reads back the events of finished stages into the per-stage totals.
@@ -599,21 +610,18 @@ void setup_geometry(fc_corr* c) {
   upload(c->wx, w[0]);
   upload(c->wy, w[1]);
   upload(c->wz, w[2]);
-  c->r_counts.allocate(sizeof(int) * c->nell * c->nrbins);
-  c->r_hist.allocate(sizeof(double) * c->nell * c->nrbins);
-  c->k_counts.allocate(sizeof(int) * c->nell * c->nkbins);
-  c->k_hist.allocate(sizeof(double) * c->nell * c->nkbins);
-  c->zerolag.allocate(sizeof(double));
+  const OutLayout lay(c);
+  c->outputs.allocate(sizeof(double) * lay.doubles());
+  double* out = c->outputs.as<double>();
+  c->r_hist.wrap(out, sizeof(double) * lay.nr);
+  c->k_hist.wrap(out + lay.k_hist(), sizeof(double) * lay.nk);
+  c->zerolag.wrap(out + lay.zerolag(), sizeof(double));
+  c->r_counts.wrap(out + lay.r_counts(), sizeof(int) * lay.nr);
+  c->k_counts.wrap(c->r_counts.as<int>() + lay.nr, sizeof(int) * lay.nk);
 }
 
 void reset_hists(fc_corr* c, hipStream_t s) {
-  const int64_t nr = (int64_t)c->nell * c->nrbins, nk = (int64_t)c->nell * c->nkbins;
-  ZeroSegs z{{c->r_counts.as<uint32_t>(), c->r_hist.as<uint32_t>(), c->k_counts.as<uint32_t>(),
-              c->k_hist.as<uint32_t>(), c->zerolag.as<uint32_t>()},
-             {nr, 2 * nr, nk, 2 * nk, 2}};
-  const int64_t most = std::max<int64_t>(2 * std::max(nr, nk), 2);
-  hipLaunchKernelGGL(k_zero_segs, dim3(grid1d(most, 256, 4096), 5), dim3(256), 0, s, z);
-  FC_LAUNCH_CHECK();
+  fill<double>(c->outputs.as<double>(), OutLayout(c).doubles(), 0.0, s);
 }
 
 // Orders the correlator's stream after all work queued on the grid's stream.
@@ -1503,24 +1511,13 @@ int fc_corr_results(fc_corr* c, double* r_mid, int* r_counts, double* r_hist, do
   return fc::guard([&] {
     if (!c) fc::fail(FC_ERR_INVALID, "null correlator");
     fc::DeviceGuard dg(c->ctx->device);
-    hipStream_t s = c->ctx->stream;
-    const size_t nr = (size_t)c->nell * c->nrbins, nk = (size_t)c->nell * c->nkbins;
-    if (r_counts)
-      FC_HIP(hipMemcpyAsync(r_counts, c->r_counts.as<void>(), sizeof(int) * nr,
-                            hipMemcpyDeviceToHost, s));
-    if (r_hist)
-      FC_HIP(hipMemcpyAsync(r_hist, c->r_hist.as<void>(), sizeof(double) * nr,
-                            hipMemcpyDeviceToHost, s));
-    if (k_counts)
-      FC_HIP(hipMemcpyAsync(k_counts, c->k_counts.as<void>(), sizeof(int) * nk,
-                            hipMemcpyDeviceToHost, s));
-    if (k_hist)
-      FC_HIP(hipMemcpyAsync(k_hist, c->k_hist.as<void>(), sizeof(double) * nk,
-                            hipMemcpyDeviceToHost, s));
-    if (zerolag)
-      FC_HIP(hipMemcpyAsync(zerolag, c->zerolag.as<void>(), sizeof(double),
-                            hipMemcpyDeviceToHost, s));
-    FC_HIP(hipStreamSynchronize(s));
+    if (r_counts || r_hist || k_counts || k_hist || zerolag) {
+      const fc::OutLayout o(c);
+      fc::read_back(c->ctx, c->outputs.as<void>(), sizeof(double) * o.doubles(),
+                    [&](const char* p) { o.unpack(p, r_hist, r_counts, k_hist, k_counts, zerolag); });
+    } else {
+      FC_HIP(hipStreamSynchronize(c->ctx->stream));
+    }
     if (r_mid) std::copy(c->rbins.begin(), c->rbins.end(), r_mid);
     if (k_mid) std::copy(c->kbins.begin(), c->kbins.end(), k_mid);
   });
@@ -1589,7 +1586,7 @@ struct fc_batch {
   fc::DeviceBuffer input;  // [nb][n0][n1][n2] grid storage
   std::vector<fc_grid*> grids;
   fc::DeviceBuffer work, pk, q1, q2, xisub, part;
-  fc::DeviceBuffer r_hist, r_counts, k_hist, k_counts, zerolag;
+  fc::DeviceBuffer outputs;  // [nb] OutLayout
   int64_t npk = 0, nq1 = 0, nq2 = 0, nxs = 0;
   bool use_graph = false;
   hipGraph_t graph = nullptr;
@@ -1618,12 +1615,11 @@ void batch_sequence(fc_batch* bt, int n) {
   const FftPlan& pi = *c->plan_inv;
   const int rs = c->rshape, o = rs / 2;
   const int64_t ldq = pi.ldc;
-  const int64_t hk = (int64_t)c->nell * c->nkbins, hr = (int64_t)c->nell * c->nrbins;
-  fill<int>(bt->r_counts.as<int>(), hr * n, 0, s);
-  fill<double>(bt->r_hist.as<double>(), hr * n, 0.0, s);
-  fill<int>(bt->k_counts.as<int>(), hk * n, 0, s);
-  fill<double>(bt->k_hist.as<double>(), hk * n, 0.0, s);
-  fill<double>(bt->zerolag.as<double>(), n, 0.0, s);
+  const OutLayout ol(c);
+  double* out = bt->outputs.as<double>();
+  int* r_counts = reinterpret_cast<int*>(out + ol.r_counts());
+  int* k_counts = r_counts + ol.nr;
+  fill<double>(out, ol.doubles() * n, 0.0, s);
   cplx<T>* w = bt->work.as<cplx<T>>();
   const int64_t rows = (int64_t)n * p.n[0] * p.n[1];
   // Forward z and y in the arithmetic of TI (FP64 for the mixed form),
@@ -1673,21 +1669,21 @@ void batch_sequence(fc_batch* bt, int n) {
   launch_rows_c2r<TI, TI>(pi, bt->q2.as<cplx<TI>>(), ldq, bt->xisub.as<TI>(), rs, s,
                           (int64_t)n * rs * rs, rs, o, (int64_t)rs * rs);
   if (c->khalf_ok) {
-    run_hist_khalf<T, NV>(c, bt->pk.as<T>(), bt->npk, bt->part, bt->k_hist.as<double>(),
-                          bt->k_counts.as<int>(), 0, 0, NV, s, n, hk);
+    run_hist_khalf<T, NV>(c, bt->pk.as<T>(), bt->npk, bt->part, out + ol.k_hist(),
+                          k_counts, 0, 0, NV, s, n, ol.doubles());
   } else {
     KEntry<T, NV> ke{c->kbin.cells.as<uint32_t>(), bt->pk.as<T>(), kslots(c),
                      FastDiv((uint32_t)c->kshape[2]), FastDiv((uint32_t)c->kshape[1]),
                      c->kx.as<double>(), c->ky.as<double>(), c->kz.as<double>(),
                      c->wx.as<double>(), c->wy.as<double>(), c->wz.as<double>(), {}, bt->npk};
     for (int q = 0; q < NV; ++q) ke.coef[q] = c->kcoef[q];
-    run_hist_seg<NV>(ke, c->kbin, bt->part, bt->k_hist.as<double>(), bt->k_counts.as<int>(), 0,
-                     0, NV, s, -1, nullptr, n, hk);
+    run_hist_seg<NV>(ke, c->kbin, bt->part, out + ol.k_hist(), k_counts, 0, 0, NV, s, -1,
+                     nullptr, n, ol.doubles());
   }
   WEntry<TI, NV> we{bt->xisub.as<TI>(), c->rbin.cells.as<uint32_t>(), c->rw.as<double>(),
                     c->rbin.n, bt->nxs};
-  run_hist_seg<NV>(we, c->rbin, bt->part, bt->r_hist.as<double>(), bt->r_counts.as<int>(), 0, 0,
-                   NV, s, c->rbin.tracked_pos, bt->zerolag.as<double>(), n, hr);
+  run_hist_seg<NV>(we, c->rbin, bt->part, out, r_counts, 0, 0, NV, s, c->rbin.tracked_pos,
+                   out + ol.zerolag(), n, ol.doubles());
 }
 
 template <typename T, typename TI>
@@ -1756,12 +1752,7 @@ int fc_batch_create(fc_ctx* ctx, const int shape[3], double cell_size, int windo
     b->q1.allocate(csi * b->nq1 * nbatch);
     b->q2.allocate(csi * b->nq2 * nbatch);
     b->xisub.allocate(tsi * b->nxs * nbatch);
-    const int64_t hk = (int64_t)c->nell * c->nkbins, hr = (int64_t)c->nell * c->nrbins;
-    b->k_hist.allocate(sizeof(double) * hk * nbatch);
-    b->k_counts.allocate(sizeof(int) * hk * nbatch);
-    b->r_hist.allocate(sizeof(double) * hr * nbatch);
-    b->r_counts.allocate(sizeof(int) * hr * nbatch);
-    b->zerolag.allocate(sizeof(double) * nbatch);
+    b->outputs.allocate(sizeof(double) * fc::OutLayout(c).doubles() * nbatch);
     b->part.allocate(sizeof(double) * 3 *
                      (size_t)std::max({c->kbin.nchunks, c->rbin.nchunks, c->khalf.nchunks}) *
                      nbatch);
@@ -1860,24 +1851,14 @@ int fc_batch_results(fc_batch* b, int i, double* r_hist, int* r_counts, double* 
     if (i < 0 || i >= b->nb) fc::fail(FC_ERR_RANGE, "batch member out of range");
     fc_corr* c = b->corr;
     fc::DeviceGuard dg(c->ctx->device);
-    hipStream_t s = c->ctx->stream;
-    const size_t hk = (size_t)c->nell * c->nkbins, hr = (size_t)c->nell * c->nrbins;
-    if (r_hist)
-      FC_HIP(hipMemcpyAsync(r_hist, b->r_hist.as<double>() + hr * i, sizeof(double) * hr,
-                            hipMemcpyDeviceToHost, s));
-    if (r_counts)
-      FC_HIP(hipMemcpyAsync(r_counts, b->r_counts.as<int>() + hr * i, sizeof(int) * hr,
-                            hipMemcpyDeviceToHost, s));
-    if (k_hist)
-      FC_HIP(hipMemcpyAsync(k_hist, b->k_hist.as<double>() + hk * i, sizeof(double) * hk,
-                            hipMemcpyDeviceToHost, s));
-    if (k_counts)
-      FC_HIP(hipMemcpyAsync(k_counts, b->k_counts.as<int>() + hk * i, sizeof(int) * hk,
-                            hipMemcpyDeviceToHost, s));
-    if (zerolag)
-      FC_HIP(hipMemcpyAsync(zerolag, b->zerolag.as<double>() + i, sizeof(double),
-                            hipMemcpyDeviceToHost, s));
-    FC_HIP(hipStreamSynchronize(s));
+    if (r_counts || r_hist || k_counts || k_hist || zerolag) {
+      const fc::OutLayout o(c);
+      fc::read_back(c->ctx, b->outputs.as<double>() + o.doubles() * i,
+                    sizeof(double) * o.doubles(),
+                    [&](const char* p) { o.unpack(p, r_hist, r_counts, k_hist, k_counts, zerolag); });
+    } else {
+      FC_HIP(hipStreamSynchronize(c->ctx->stream));
+    }
   });
 }
 

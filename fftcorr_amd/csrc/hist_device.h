@@ -160,15 +160,16 @@ struct FastDiv {
 // fixed tree over lanes and waves) into part[b][NV].  When pos == zpos the
 // first value is also stored to *zval (the zero-lag cell).  blockIdx.y is
 // the batch member: g.offset(m) selects its values, and its partials and
-// zero-lag value go to part[m][nchunks][NV] and zval[m].
+// zero-lag value go to part[m][nchunks][NV] and zval[m * out_bstride].
 template <int NV, class G>
 __global__ void __launch_bounds__(kSegThreads)
     k_hist_seg(G g, const int4* __restrict__ chunks, const int* __restrict__ order,
-               double* __restrict__ part, int64_t zpos, double* __restrict__ zval) {
+               double* __restrict__ part, int64_t zpos, double* __restrict__ zval,
+               int64_t out_bstride) {
   __shared__ double sw[kSegThreads / kWave][NV];
   g.offset(blockIdx.y);
   part += (size_t)blockIdx.y * gridDim.x * NV;
-  if (zval) zval += blockIdx.y;
+  if (zval) zval += blockIdx.y * out_bstride;
   const int cid = order[xcd_tile(blockIdx.x, gridDim.x)];
   const int4 ch = chunks[cid];
   double acc[NV];
@@ -208,7 +209,7 @@ __global__ void __launch_bounds__(kWave)
   const int i = blockIdx.x;
   part += (size_t)blockIdx.y * nchunks * NV;
   hist += blockIdx.y * out_bstride;
-  counts += blockIdx.y * out_bstride;
+  counts += blockIdx.y * 2 * out_bstride;
   const int lane = threadIdx.x;
   if (i < NV * nbins) {
     const int q = i / nbins, bin = i - q * nbins;
@@ -267,8 +268,8 @@ struct HistScratch {
   }
 };
 
-// nb batch members: member m's histogram rows start at hist + m * out_bstride
-// (counts likewise).
+// nb batch members: member m's outputs (histogram rows, counts, zero lag) lie
+// m * out_bstride doubles behind the first member's.
 // bin_counts (optional): the counts added per bin, instead of bc's own.
 template <int NV, class G>
 void run_hist_seg(G g, const BinnedCells& bc, DeviceBuffer& part, double* hist, int* counts,
@@ -279,7 +280,7 @@ void run_hist_seg(G g, const BinnedCells& bc, DeviceBuffer& part, double* hist, 
   if (bc.nchunks > 0) {
     part.reserve(sizeof(double) * (size_t)bc.nchunks * NV * nb);
     hipLaunchKernelGGL((k_hist_seg<NV, G>), dim3(bc.nchunks, nb), dim3(kSegThreads), 0, s, g,
-                       bc.chunks.as<int4>(), bc.order.as<int>(), part.as<double>(), zpos, zval);
+                       bc.chunks.as<int4>(), bc.order.as<int>(), part.as<double>(), zpos, zval, out_bstride);
     FC_LAUNCH_CHECK();
   }
   const int tot = NV * nbins > nbins ? NV * nbins : nbins;

@@ -725,12 +725,12 @@ void mass_assign(fc_grid* grid, const double* pos_dev, int64_t n, int ncol,
   }
   FC_HIP(hipEventRecord(ev[2], s));
 
-  double wsum[3];
-  FC_HIP(hipMemcpyAsync(wsum, partw.as<double>() + 2 * nbp, sizeof(wsum),
-                        hipMemcpyDeviceToHost, s));
-  FC_HIP(hipStreamSynchronize(s));
+  double wsum[2];
   unsigned long long nadd = 0;
-  std::memcpy(&nadd, &wsum[2], sizeof(nadd));
+  read_back(ctx, partw.as<double>() + 2 * nbp, sizeof(wsum) + sizeof(nadd), [&](const char* p) {
+    std::memcpy(wsum, p, sizeof(wsum));
+    std::memcpy(&nadd, p + sizeof(wsum), sizeof(nadd));
+  });
   float t_sort = 0, t_win = 0;
   FC_HIP(hipEventElapsedTime(&t_sort, ev[0], ev[1]));
   FC_HIP(hipEventElapsedTime(&t_win, ev[1], ev[2]));
