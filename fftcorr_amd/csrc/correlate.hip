@@ -76,6 +76,10 @@ struct fc_corr {
   // priority) beside the pruned inverse; created on first use.
   hipStream_t side = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  // Yamamoto correlations run the pruned inverse of a transform on a third
+  // stream, beside the forward passes of the next one.
+  hipStream_t inv = nullptr;
+  hipEvent_t ev_inv = nullptr;
   fc::DeviceBuffer part_k;  // the k histogram's partials (the r histogram's are hs.part_seg)
   // Per-stage profiling: event pairs recorded during the last call(s).
   bool profile = false;
@@ -356,10 +360,11 @@ __global__ void k_acc_k(double* __restrict__ ksub, const T* __restrict__ pk, KSl
 }
 
 // Yamamoto accumulation into the r subgrid (correlator.h:477-483) from the
-// pruned inverse: rsub += Y_lm(r) 4 pi / N xi.
+// pruned inverse: rsub += Y_lm(r) 4 pi / N xi (the first m of a multipole
+// sets it).
 template <typename T>
 __global__ void k_acc_r(double* __restrict__ rsub, const T* __restrict__ xi, int rs,
-                        const double* __restrict__ rx, int ell, int m, double c) {
+                        const double* __restrict__ rx, int ell, int m, double c, bool first) {
 #pragma clang fp contract(off)
   const int64_t n = (int64_t)rs * rs * rs;
   for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < n;
@@ -368,7 +373,7 @@ __global__ void k_acc_r(double* __restrict__ rsub, const T* __restrict__ xi, int
     const int64_t t = idx / rs;
     const int j = (int)(t % rs), i = (int)(t / rs);
     const double y = ylm_eval(ell, m, rx[i], rx[j], rx[k], c, 1.0);
-    rsub[idx] += y * (double)xi[idx];
+    rsub[idx] = (first ? 0.0 : rsub[idx]) + y * (double)xi[idx];
   }
 }
 
@@ -730,6 +735,19 @@ void forward_fft(fc_corr* c, fc_grid* g, cplx<T>* dst, Loader ld) {
   forward_x<T, A>(c, dst);
 }
 
+// The x pass of the y-transformed grid w into the FFT of grid 2; w stays.
+template <typename T, typename A>
+void store_grid2(fc_corr* c, const cplx<T>* w) {
+  const FftPlan& p = *c->plan;
+  c->grid2_fft.reserve(p.complex_bytes());
+  Stage st(c, FC_STAGE_FFT_X_FWD);
+  ColView<T> v = x_view<T>(p, c->grid2_fft.as<cplx<T>>());
+  v.in = w;
+  launch_cols_wide<T, -1, A>(p.n[0], v, p.tile[0], c->plan_inv->tw0.as<cplx<A>>(),
+                             p.tw0.as<cplx<T>>(), c->ctx->stream, p.gen[0].get(), p.var[0]);
+  c->have_grid2 = true;
+}
+
 // exp(i pi f / n) for the signed frequency f of every index along each axis
 // (numpy.fft.fftfreq convention), for interlacing.
 void ensure_phase_tables(fc_corr* c) {
@@ -888,10 +906,9 @@ void power_x(fc_corr* c, cplx<T>* w, const cplx<T>* b, int mode) {
   }
 }
 
-// Pruned inverse y and z passes: q1 -> q2 -> the r subgrid xisub.
+// Pruned inverse y and z passes: q1 -> q2 -> the r subgrid xisub, on stream s.
 template <typename T, typename TI>
-void pruned_inverse_yz(fc_corr* c) {
-  hipStream_t s = c->ctx->stream;
+void pruned_inverse_yz(fc_corr* c, hipStream_t s) {
   const FftPlan& pi = *c->plan_inv;
   const int64_t ldq = pi.ldc;
   const int rs = c->rshape, o = rs / 2;
@@ -913,7 +930,7 @@ void pruned_inverse_yz(fc_corr* c) {
 template <typename T, typename TI>
 void power_and_pruned_inverse(fc_corr* c, cplx<T>* w, const cplx<T>* b, int mode) {
   power_x<T, TI>(c, w, b, mode);
-  pruned_inverse_yz<T, TI>(c);
+  pruned_inverse_yz<T, TI>(c, c->ctx->stream);
 }
 
 // Builds the periodic histogram coefficients and r weights once per correlator.
@@ -979,6 +996,15 @@ hipStream_t side_stream(fc_corr* c) {
   return c->side;
 }
 
+// The stream of the Yamamoto correlations' pruned inverse (likewise).
+hipStream_t inverse_stream(fc_corr* c) {
+  if (!c->inv) {
+    FC_HIP(hipStreamCreateWithFlags(&c->inv, hipStreamNonBlocking));
+    FC_HIP(hipEventCreateWithFlags(&c->ev_inv, hipEventDisableTiming));
+  }
+  return c->inv;
+}
+
 // After the forward passes: power spectrum and pruned inverse x, then the k
 // histogram (which reads only pk) on the side stream while the pruned
 // inverse y and z passes and the r histogram run on the correlator's
@@ -992,7 +1018,7 @@ void periodic_tail(fc_corr* c, cplx<T>* w, const cplx<T>* b, int mode) {
   power_x<T, TI>(c, w, b, mode);
   if (c->profile) {
     periodic_k_hist<T, NV>(c, s, c->part_k);
-    pruned_inverse_yz<T, TI>(c);
+    pruned_inverse_yz<T, TI>(c, c->ctx->stream);
     periodic_r_hist<TI, NV>(c);
     return;
   }
@@ -1001,7 +1027,7 @@ void periodic_tail(fc_corr* c, cplx<T>* w, const cplx<T>* b, int mode) {
   FC_HIP(hipStreamWaitEvent(hs, c->ev_fork, 0));
   periodic_k_hist<T, NV>(c, hs, c->part_k);
   FC_HIP(hipEventRecord(c->ev_join, hs));
-  pruned_inverse_yz<T, TI>(c);
+  pruned_inverse_yz<T, TI>(c, c->ctx->stream);
   periodic_r_hist<TI, NV>(c);
   FC_HIP(hipStreamWaitEvent(s, c->ev_join, 0));
 }
@@ -1092,8 +1118,7 @@ void plain_r_multipole(fc_corr* c, const T* xr, int ell, int m, double coef, boo
   FC_LAUNCH_CHECK();
 }
 
-void hist_subgrids(fc_corr* c, int ell, bool k_side, bool r_side) {
-  hipStream_t s = c->ctx->stream;
+void hist_subgrids(fc_corr* c, int ell, bool k_side, bool r_side, hipStream_t s) {
   if (r_side) {
     Stage st(c, FC_STAGE_HIST_R);
     run_hist_seg<1>(GEntry<double>{c->rsub.as<double>(), c->rbin.cells.as<uint32_t>()}, c->rbin,
@@ -1144,13 +1169,13 @@ void periodic_plain(fc_corr* c, fc_grid* g1, int mode, fc_grid* gb) {
   const double r_rescale = (1.0 / ncells / ncells);
   for (int ell = 0; ell <= c->maxell; ell += 2) {
     plain_k_multipole<T>(c, ell, 0, std::sqrt((4.0 * M_PI) * (2 * ell + 1)) * k_rescale, false);
-    hist_subgrids(c, ell, true, false);
+    hist_subgrids(c, ell, true, false, c->ctx->stream);
   }
   const T* xr = full_inverse<T>(c, w);
   for (int ell = 0; ell <= c->maxell; ell += 2) {
     plain_r_multipole<T>(c, xr, ell, 0, std::sqrt((4.0 * M_PI) * (2 * ell + 1)) * r_rescale,
                          false);
-    hist_subgrids(c, ell, false, true);
+    hist_subgrids(c, ell, false, true, c->ctx->stream);
   }
 }
 
@@ -1174,12 +1199,15 @@ void yamamoto_plain(fc_corr* c, fc_grid* g1) {
       const T* xr = full_inverse<T>(c, w);
       plain_r_multipole<T>(c, xr, ell, m, 4.0 * M_PI / ncells, m != -ell);
     }
-    hist_subgrids(c, ell, true, true);
+    hist_subgrids(c, ell, true, true, c->ctx->stream);
   }
 }
 
+// own: the grid is its own grid 2 (autocorrelation).  Its spectrum is then
+// taken from the one plain z and y transform that serves l = 0 as well: Y_00
+// is a constant, so that multipole's product is |F|^2 with Y_00 in the weights.
 template <typename T, typename TI>
-void yamamoto_correlate(fc_corr* c, fc_grid* g1) {
+void yamamoto_correlate(fc_corr* c, fc_grid* g1, bool own) {
   hipStream_t s = c->ctx->stream;
   const FftPlan& p = *c->plan;
   cplx<T>* w = c->work.as<cplx<T>>();
@@ -1193,63 +1221,86 @@ void yamamoto_correlate(fc_corr* c, fc_grid* g1) {
   for (int i = 0; i < 3; ++i) start[i] = 0.5 - (-c->posmin[i] / c->cell);
   const int rs = c->rshape;
   const int64_t nr = (int64_t)rs * rs * rs;
-  // Each transform's k histogram runs on the side stream (unless stage
-  // profiling is on) beside its pruned inverse and the next transform's
-  // forward passes; the next power pass, which rewrites pk, waits for it.
+  // Beside a transform's power pass and the next one's forward passes run
+  // (unless stage profiling is on) its k histogram, which reads pk, on the side
+  // stream and its pruned inverse, which reads q1, on another; the next power
+  // pass, which rewrites both, waits for them.
   const bool par = !c->profile;
   hipStream_t ks = par ? side_stream(c) : s;
-  DeviceBuffer& kpart = par ? c->part_k : c->hs.part_seg;
+  hipStream_t is = par ? inverse_stream(c) : s;
+  const BinnedCells& kcells = c->khalf_ok ? c->khalf : c->kbin;
+  c->part_k.reserve(sizeof(double) * (size_t)std::max(kcells.nchunks, 1) * (2 * c->maxell + 1));
   bool pending = false;
   for (int ell = 0; ell <= c->maxell; ell += 2) {
+    const int row = ell / 2;
     for (int m = -ell; m <= ell; ++m) {
-      LoadYlm ld{ell, m, p.n[1], ylm_coeff(ell, m, 1.0), start[0], start[1], start[2]};
-      forward_zy<T, TI>(c, g1, w, ld);
-      if (pending) FC_HIP(hipStreamWaitEvent(s, c->ev_join, 0));
-      power_x<T, TI>(c, w, c->grid2_fft.as<cplx<T>>(), kModeCross);
+      const bool plain = own && ell == 0;
+      const double y00 = plain ? ylm_coeff(0, 0, 1.0) : 1.0;
+      if (plain) {
+        forward_zy<T, TI>(c, g1, w, LoadCopy{});
+        store_grid2<T, TI>(c, w);
+        power_x<T, TI>(c, w, nullptr, kModeAuto);
+      } else {
+        LoadYlm ld{ell, m, p.n[1], ylm_coeff(ell, m, 1.0), start[0], start[1], start[2]};
+        forward_zy<T, TI>(c, g1, w, ld);
+        if (pending) {
+          FC_HIP(hipStreamWaitEvent(s, c->ev_join, 0));
+          FC_HIP(hipStreamWaitEvent(s, c->ev_inv, 0));
+        }
+        power_x<T, TI>(c, w, c->grid2_fft.as<cplx<T>>(), kModeCross);
+      }
       if (par) {
         FC_HIP(hipEventRecord(c->ev_fork, s));
         FC_HIP(hipStreamWaitEvent(ks, c->ev_fork, 0));
+        FC_HIP(hipStreamWaitEvent(is, c->ev_fork, 0));
       }
       {
         // k-space multipole l: this transform's share, straight from the
-        // compact k values (counts once per l).
+        // compact k values; the shares are summed once per l.
         Stage st(c, FC_STAGE_HIST_K);
-        const int row = ell / 2;
+        double* part = c->part_k.as<double>() + (size_t)(m + ell) * kcells.nchunks;
+        const double coef = ylm_coeff(ell, m, 4.0 * M_PI) * y00;
         if (c->khalf_ok) {
           const int nz = c->kshape[2] / 2 + 1, oz = c->kshape[2] / 2;
           KEntryHalfLm<T> ke{c->khalf.cells.as<uint32_t>(), c->pk.as<T>(),
                              FastDiv((uint32_t)nz), FastDiv((uint32_t)c->kshape[1]), nz,
                              c->kshape[1], c->kx.as<double>(), c->ky.as<double>(),
                              c->kz.as<double>() + oz, c->wx.as<double>(), c->wy.as<double>(),
-                             c->wz.as<double>() + oz, ell, m, ylm_coeff(ell, m, 4.0 * M_PI)};
-          run_hist_seg<1>(ke, c->khalf, kpart, c->k_hist.as<double>(), c->k_counts.as<int>(),
-                          row, row, m == -ell ? row + 1 : row, ks, -1, nullptr, 1, 0,
-                          c->kbin.counts.as<int>());
+                             c->wz.as<double>() + oz, ell, m, coef};
+          hist_seg_partials<1>(ke, kcells, part, ks);
         } else {
           KEntryLm<T> ke{c->kbin.cells.as<uint32_t>(), c->pk.as<T>(), kslots(c),
                          FastDiv((uint32_t)c->kshape[2]), FastDiv((uint32_t)c->kshape[1]),
                          c->kx.as<double>(), c->ky.as<double>(), c->kz.as<double>(),
                          c->wx.as<double>(), c->wy.as<double>(), c->wz.as<double>(), ell, m,
-                         ylm_coeff(ell, m, 4.0 * M_PI)};
-          run_hist_seg<1>(ke, c->kbin, kpart, c->k_hist.as<double>(), c->k_counts.as<int>(),
-                          row, row, m == -ell ? row + 1 : row, ks);
+                         coef};
+          hist_seg_partials<1>(ke, kcells, part, ks);
         }
+        if (m == ell)
+          hist_seg_sum<1>(kcells, c->part_k.as<double>(), 2 * ell + 1, c->k_hist.as<double>(),
+                          c->k_counts.as<int>(), row, row, row + 1, ks, 1, 0,
+                          c->kbin.counts.as<int>());
       }
+      pruned_inverse_yz<T, TI>(c, is);
+      {
+        Stage st(c, FC_STAGE_SUBGRID);
+        hipLaunchKernelGGL(k_acc_r<TI>, dim3(grid1d(nr, 256, 65536)), dim3(256), 0, is,
+                           c->rsub.as<double>(), c->xisub.as<TI>(), rs, c->rx.as<double>(), ell,
+                           m, ylm_coeff(ell, m, 4.0 * M_PI / ncells) * y00, m == -ell);
+        FC_LAUNCH_CHECK();
+      }
+      if (m == ell) hist_subgrids(c, ell, false, true, is);
       if (par) {
         FC_HIP(hipEventRecord(c->ev_join, ks));
+        FC_HIP(hipEventRecord(c->ev_inv, is));
         pending = true;
       }
-      pruned_inverse_yz<T, TI>(c);
-      Stage st(c, FC_STAGE_SUBGRID);
-      if (m == -ell) fill<double>(c->rsub.as<double>(), nr, 0.0, s);
-      hipLaunchKernelGGL(k_acc_r<TI>, dim3(grid1d(nr, 256, 65536)), dim3(256), 0, s,
-                         c->rsub.as<double>(), c->xisub.as<TI>(), rs, c->rx.as<double>(), ell,
-                         m, ylm_coeff(ell, m, 4.0 * M_PI / ncells));
-      FC_LAUNCH_CHECK();
     }
-    hist_subgrids(c, ell, false, true);
   }
-  if (pending) FC_HIP(hipStreamWaitEvent(s, c->ev_join, 0));
+  if (pending) {
+    FC_HIP(hipStreamWaitEvent(s, c->ev_join, 0));
+    FC_HIP(hipStreamWaitEvent(s, c->ev_inv, 0));
+  }
 }
 
 void ensure_work(fc_corr* c) { c->work.reserve(c->plan->complex_bytes()); }
@@ -1273,7 +1324,7 @@ void run_kind(fc_corr* c, fc_grid* g1, fc_grid* gb, int mode) {
     if constexpr (std::is_same<T, TI>::value) {
       if (plain) return yamamoto_plain<T>(c, g1);
     }
-    yamamoto_correlate<T, TI>(c, g1);
+    yamamoto_correlate<T, TI>(c, g1, mode == kModeAuto);
   } else {
     if constexpr (std::is_same<T, TI>::value) {
       if (plain) return periodic_plain<T>(c, g1, mode, gb);
@@ -1302,8 +1353,9 @@ void correlate(fc_corr* c, fc_grid* g1, fc_grid* gb, int mode) {
   FC_HIP(hipEventRecord(c->ev0, s));
   reset_hists(c, s);
   if (c->kind == FC_YAMAMOTO) {
-    if (mode == kModeAuto) set_grid2_device(c, g1);  // Correlator::autocorrelate = cross(grid, grid)
-    if (!c->have_grid2) fail(FC_ERR_RUNTIME, "grid2 FFT not set: call set_grid2 first");
+    // Correlator::autocorrelate = cross(grid, grid)
+    if (mode == kModeAuto && c->algo == FC_ALGO_PLAIN) set_grid2_device(c, g1);
+    if (mode == kModeCross && !c->have_grid2) fail(FC_ERR_RUNTIME, "grid2 FFT not set: call set_grid2 first");
   }
   if (c->prec == FC_FP64)
     run_kind<double, double>(c, g1, gb, mode);
@@ -1371,6 +1423,11 @@ int fc_corr_destroy(fc_corr* corr) {
       (void)hipStreamSynchronize(corr->side);
       (void)hipStreamDestroy(corr->side);
     }
+    if (corr->inv) {
+      (void)hipStreamSynchronize(corr->inv);
+      (void)hipStreamDestroy(corr->inv);
+    }
+    if (corr->ev_inv) (void)hipEventDestroy(corr->ev_inv);
     if (corr->ev_fork) (void)hipEventDestroy(corr->ev_fork);
     if (corr->ev_join) (void)hipEventDestroy(corr->ev_join);
     for (auto e : corr->ev_pool) (void)hipEventDestroy(e);
@@ -1425,7 +1482,8 @@ int fc_corr_footprint(fc_corr* c, int interlaced, size_t* held, size_t* full) {
     add(c->rw, 8 * nv * (size_t)std::max<int64_t>(c->rbin.n, 1));
     add(c->hs.part_seg,
         8 * nv * (size_t)std::max({c->kbin.nchunks, c->rbin.nchunks, c->khalf.nchunks}));
-    add(c->part_k, 8 * nv * (size_t)(c->khalf_ok ? c->khalf.nchunks : c->kbin.nchunks));
+    const size_t ksets = c->kind == FC_YAMAMOTO ? 2 * (size_t)c->maxell + 1 : nv;
+    add(c->part_k, 8 * ksets * (size_t)(c->khalf_ok ? c->khalf.nchunks : c->kbin.nchunks));
     for (int d = 0; d < 3; ++d)
       add(c->ph[d], sizeof(double2) * (size_t)(d == 2 ? p.ldc : c->shape[d]));
     if (held) *held = now;

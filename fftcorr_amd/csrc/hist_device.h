@@ -199,13 +199,14 @@ __global__ void __launch_bounds__(kSegThreads)
 
 // One wave per (multipole, bin): hist[row0 + q][bin] += the chunk partials
 // of the bin (lane l sums chunks l, l + 64, ... in order, then a fixed xor
-// tree); counts rows [crow0, crow1) += counts of the bin.
+// tree); counts rows [crow0, crow1) += counts of the bin.  nsets sets of
+// partials, one behind the other, are summed in turn.
 template <int NV>
 __global__ void __launch_bounds__(kWave)
     k_hist_seg_final(const double* __restrict__ part, const int* __restrict__ chunk_first,
                      const int* __restrict__ bin_counts, int nbins, double* __restrict__ hist,
                      int* __restrict__ counts, int row0, int crow0, int crow1, int nchunks,
-                     int64_t out_bstride) {
+                     int64_t out_bstride, int nsets) {
   const int i = blockIdx.x;
   part += (size_t)blockIdx.y * nchunks * NV;
   hist += blockIdx.y * out_bstride;
@@ -213,11 +214,14 @@ __global__ void __launch_bounds__(kWave)
   const int lane = threadIdx.x;
   if (i < NV * nbins) {
     const int q = i / nbins, bin = i - q * nbins;
-    double s = 0.0;
-    for (int c = chunk_first[bin] + lane; c < chunk_first[bin + 1]; c += kWave)
-      s += part[(size_t)c * NV + q];
-    s = wave_sum(s);
-    if (lane == 0) hist[(size_t)(row0 + q) * nbins + bin] += s;
+    const int c0 = chunk_first[bin] + lane, c1 = chunk_first[bin + 1];
+    double sum = 0.0;
+    for (int t = 0; t < nsets; ++t) {
+      double s = 0.0;
+      for (int c = c0; c < c1; c += kWave) s += part[((size_t)t * nchunks + c) * NV + q];
+      sum += wave_sum(s);
+    }
+    if (lane == 0) hist[(size_t)(row0 + q) * nbins + bin] += sum;
   }
   if (i < nbins && lane == 0)
     for (int r = crow0; r < crow1; ++r) counts[(size_t)r * nbins + i] += bin_counts[i];
@@ -272,23 +276,35 @@ struct HistScratch {
 // m * out_bstride doubles behind the first member's.
 // bin_counts (optional): the counts added per bin, instead of bc's own.
 template <int NV, class G>
+void hist_seg_partials(G g, const BinnedCells& bc, double* part, hipStream_t s,
+                       int64_t zpos = -1, double* zval = nullptr, int nb = 1,
+                       int64_t out_bstride = 0) {
+  if (bc.nchunks == 0) return;
+  hipLaunchKernelGGL((k_hist_seg<NV, G>), dim3(bc.nchunks, nb), dim3(kSegThreads), 0, s, g,
+                     bc.chunks.as<int4>(), bc.order.as<int>(), part, zpos, zval, out_bstride);
+  FC_LAUNCH_CHECK();
+}
+
+template <int NV>
+void hist_seg_sum(const BinnedCells& bc, const double* part, int nsets, double* hist,
+                  int* counts, int row0, int crow0, int crow1, hipStream_t s, int nb = 1,
+                  int64_t out_bstride = 0, const int* bin_counts = nullptr) {
+  const int tot = NV * bc.nbins;
+  hipLaunchKernelGGL((k_hist_seg_final<NV>), dim3(tot, nb), dim3(kWave), 0, s, part,
+                     bc.chunk_first.as<int>(), bin_counts ? bin_counts : bc.counts.as<int>(),
+                     bc.nbins, hist, counts, row0, crow0, crow1, bc.nchunks, out_bstride, nsets);
+  FC_LAUNCH_CHECK();
+}
+
+template <int NV, class G>
 void run_hist_seg(G g, const BinnedCells& bc, DeviceBuffer& part, double* hist, int* counts,
                   int row0, int crow0, int crow1, hipStream_t s, int64_t zpos = -1,
                   double* zval = nullptr, int nb = 1, int64_t out_bstride = 0,
                   const int* bin_counts = nullptr) {
-  const int nbins = bc.nbins;
-  if (bc.nchunks > 0) {
-    part.reserve(sizeof(double) * (size_t)bc.nchunks * NV * nb);
-    hipLaunchKernelGGL((k_hist_seg<NV, G>), dim3(bc.nchunks, nb), dim3(kSegThreads), 0, s, g,
-                       bc.chunks.as<int4>(), bc.order.as<int>(), part.as<double>(), zpos, zval, out_bstride);
-    FC_LAUNCH_CHECK();
-  }
-  const int tot = NV * nbins > nbins ? NV * nbins : nbins;
-  hipLaunchKernelGGL((k_hist_seg_final<NV>), dim3(tot, nb), dim3(kWave), 0, s,
-                     part.as<double>(), bc.chunk_first.as<int>(),
-                     bin_counts ? bin_counts : bc.counts.as<int>(), nbins,
-                     hist, counts, row0, crow0, crow1, bc.nchunks, out_bstride);
-  FC_LAUNCH_CHECK();
+  if (bc.nchunks > 0) part.reserve(sizeof(double) * (size_t)bc.nchunks * NV * nb);
+  hist_seg_partials<NV>(g, bc, part.as<double>(), s, zpos, zval, nb, out_bstride);
+  hist_seg_sum<NV>(bc, part.as<double>(), 1, hist, counts, row0, crow0, crow1, s, nb,
+                   out_bstride, bin_counts);
 }
 
 template <int NV, class F>
