@@ -212,8 +212,13 @@ struct KEntryLm {
   FastDiv d2, d1;  // division by ks2 and ks1
   const double *kx, *ky, *kz, *wx, *wy, *wz;
   int ell, m;
-  double coef;
-  __device__ __forceinline__ void offset(int) {}
+  double coef0, coef;  // of m = 0 and of the others
+  int64_t bstride;     // pk elements per transform; member i is m + i
+  __device__ __forceinline__ void offset(int i) {
+    pk += i * bstride;
+    m += i;
+    if (m == 0) coef = coef0;
+  }
   __device__ __forceinline__ void operator()(int64_t pos, double* v) const {
 #pragma clang fp contract(off)
     const uint32_t cell = cells[pos];
@@ -274,8 +279,13 @@ struct KEntryHalfLm {
   int nz, ks1;
   const double *kx, *ky, *kz, *wx, *wy, *wz;  // kz, wz from the kz = 0 plane on
   int ell, m;
-  double coef;
-  __device__ __forceinline__ void offset(int) {}
+  double coef0, coef;
+  int64_t bstride;
+  __device__ __forceinline__ void offset(int i) {
+    pk += i * bstride;
+    m += i;
+    if (m == 0) coef = coef0;
+  }
   __device__ __forceinline__ void operator()(int64_t pos, double* v) const {
 #pragma clang fp contract(off)
     const uint32_t e = cells[pos];
@@ -360,11 +370,12 @@ __global__ void k_acc_k(double* __restrict__ ksub, const T* __restrict__ pk, KSl
 }
 
 // Yamamoto accumulation into the r subgrid (correlator.h:477-483) from the
-// pruned inverse: rsub += Y_lm(r) 4 pi / N xi (the first m of a multipole
-// sets it).
+// pruned inverses of nm transforms m, m + 1, ..: rsub += Y_lm(r) 4 pi / N xi
+// (the first m of a multipole sets it).  c0: normalisation of m = 0.
 template <typename T>
 __global__ void k_acc_r(double* __restrict__ rsub, const T* __restrict__ xi, int rs,
-                        const double* __restrict__ rx, int ell, int m, double c, bool first) {
+                        const double* __restrict__ rx, int ell, int m, int nm, double c0,
+                        double c, bool first) {
 #pragma clang fp contract(off)
   const int64_t n = (int64_t)rs * rs * rs;
   for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < n;
@@ -372,8 +383,12 @@ __global__ void k_acc_r(double* __restrict__ rsub, const T* __restrict__ xi, int
     const int k = (int)(idx % rs);
     const int64_t t = idx / rs;
     const int j = (int)(t % rs), i = (int)(t / rs);
-    const double y = ylm_eval(ell, m, rx[i], rx[j], rx[k], c, 1.0);
-    rsub[idx] = (first ? 0.0 : rsub[idx]) + y * (double)xi[idx];
+    double sum = first ? 0.0 : rsub[idx];
+    for (int g = 0; g < nm; ++g) {
+      const double y = ylm_eval(ell, m + g, rx[i], rx[j], rx[k], m + g == 0 ? c0 : c, 1.0);
+      sum += y * (double)xi[g * n + idx];
+    }
+    rsub[idx] = sum;
   }
 }
 
@@ -652,15 +667,17 @@ void check_grid_shape(fc_corr* c, fc_grid* g) {
 // then takes its twiddles from the FP64 plan plan_inv).  The grid is
 // processed in chunks of x slabs (plan zy_chunk) so that each chunk's y pass
 // reads the z pass's output from the last-level cache.
+// nb > 1: the loader's transforms of the grid, one behind the other (no
+// chunks).
 template <typename T, typename A = T, class Loader>
-void forward_zy(fc_corr* c, fc_grid* g, cplx<T>* dst, Loader ld) {
+void forward_zy(fc_corr* c, fc_grid* g, cplx<T>* dst, Loader ld, int nb = 1) {
   const FftPlan& p = *c->plan;
   const FftPlan& pa = *c->plan_inv;
   hipStream_t s = c->ctx->stream;
   const int X = p.zy_chunk > 0 ? p.zy_chunk : p.n[0];
   for (int x0 = 0; x0 < p.n[0]; x0 += X) {
     const int nx = std::min(X, p.n[0] - x0);
-    const int64_t rows = (int64_t)nx * p.n[1];
+    const int64_t rows = (int64_t)nb * nx * p.n[1];
     cplx<T>* d = dst + (int64_t)x0 * p.n[1] * p.ldc;
     Loader lc = ld;
     lc.shift_x(x0);
@@ -676,7 +693,7 @@ void forward_zy(fc_corr* c, fc_grid* g, cplx<T>* dst, Loader ld) {
     }
     Stage st(c, FC_STAGE_FFT_Y_FWD);
     ColView<T> v = y_view<T>(p, d);
-    v.A = nx;
+    v.A = nb * nx;
     launch_cols_wide<T, -1, A>(p.n[1], v, p.tile[1], pa.tw1.as<cplx<A>>(), p.tw1.as<cplx<T>>(),
                                s, p.gen[1].get(), p.var[1]);
   }
@@ -787,15 +804,41 @@ void run_hist_khalf(fc_corr* c, const T* pk, int64_t bstride, DeviceBuffer& part
                    out_bstride, c->kbin.counts.as<int>());
 }
 
+int64_t pk_elems(const fc_corr* c) {
+  return (int64_t)c->kshape[0] * c->kshape[1] * (c->kshape[2] / 2 + 1);
+}
+
+// nb: transforms that share their launches.
 template <typename T, typename TI>
-void ensure_periodic_buffers(fc_corr* c) {
+void ensure_periodic_buffers(fc_corr* c, int nb = 1) {
   const FftPlan& pi = *c->plan_inv;
   const int rs = c->rshape;
-  const int oz = c->kshape[2] / 2;
-  c->pk.reserve(sizeof(T) * (size_t)c->kshape[0] * c->kshape[1] * (oz + 1));
-  c->q1.reserve(sizeof(cplx<TI>) * (size_t)rs * pi.n[1] * pi.ldc);
-  c->q2.reserve(sizeof(cplx<TI>) * (size_t)rs * rs * pi.ldc);
-  c->xisub.reserve(sizeof(TI) * (size_t)rs * rs * rs);
+  c->pk.reserve(sizeof(T) * nb * (size_t)pk_elems(c));
+  c->q1.reserve(sizeof(cplx<TI>) * nb * (size_t)rs * pi.n[1] * pi.ldc);
+  c->q2.reserve(sizeof(cplx<TI>) * nb * (size_t)rs * rs * pi.ldc);
+  c->xisub.reserve(sizeof(TI) * nb * (size_t)rs * rs * rs);
+}
+
+// Transforms of multipole ell that share their launches: as many as keep the
+// spectra within kGroupBytes.  Small grids are bound by their launches and by
+// the chip they leave idle (64^3 FP64 l <= 4: 1060 us one by one, 290 in
+// groups; 128^3 1140 and 515), large ones by the small passes of the pruned
+// inverse (256^3 2990 and 2680, 360 x 300 x 200 6090 and 5420).  Beyond 1 GB
+// (0.35% of the memory) another 1% is left.
+constexpr size_t kGroupBytes = size_t(1) << 30;
+int yamamoto_group(const fc_corr* c, int ell) {
+  const int all = 2 * ell + 1;
+  const FftPlan& p = *c->plan;
+  if (p.zy_chunk > 0) return 1;
+  const int most = (int)std::min<size_t>(all, std::max<size_t>(1, kGroupBytes / p.complex_bytes()));
+  const int groups = (all + most - 1) / most;
+  return (all + groups - 1) / groups;  // of about equal size
+}
+// The largest group of a correlation (what its buffers are sized for).
+int yamamoto_most(const fc_corr* c) {
+  int most = 1;
+  for (int ell = 0; ell <= c->maxell; ell += 2) most = std::max(most, yamamoto_group(c, ell));
+  return most;
 }
 
 // Outputs of one fused x launch: nb batch members, member i reading its
@@ -863,26 +906,29 @@ void full_power(fc_corr* c, cplx<T>* w, const cplx<T>* b, int mode) {
 }
 
 template <typename T>
-void gather_pk(fc_corr* c, const cplx<T>* P) {
+void gather_pk(fc_corr* c, const cplx<T>* P, int member = 0) {
   const FftPlan& p = *c->plan;
   const KSlots ks = kslots(c);
-  const int64_t npk = (int64_t)ks.ks0 * ks.ks1 * (ks.ks2 / 2 + 1);
+  const int64_t npk = pk_elems(c);
   hipLaunchKernelGGL(k_gather_pk<T>, dim3(grid1d(npk, 256, 65536)), dim3(256), 0,
-                     c->ctx->stream, c->pk.as<T>(), P, ks, p.n[0], p.n[1], (int64_t)p.ldc);
+                     c->ctx->stream, c->pk.as<T>() + member * npk, P, ks, p.n[0], p.n[1],
+                     (int64_t)p.ldc);
   FC_LAUNCH_CHECK();
 }
 
 // |F|^2 (or F conj(G)) -> compact k values pk, then the pruned inverse
 // (x lags in the fused kernel, then y and z, in the inverse precision TI)
-// -> r subgrid xisub.
+// -> r subgrid xisub.  nb transforms in w, one behind the other (auto and cross
+// modes).
 template <typename T, typename TI>
-void power_x(fc_corr* c, cplx<T>* w, const cplx<T>* b, int mode) {
+void power_x(fc_corr* c, cplx<T>* w, const cplx<T>* b, int mode, int nb = 1) {
   hipStream_t s = c->ctx->stream;
   const FftPlan& p = *c->plan;
   const FftPlan& pi = *c->plan_inv;
   const int64_t ldq = pi.ldc;
   const int rs = c->rshape, o = rs / 2;
-  const PxOut po{c->pk.as<void>(), c->q1.as<void>()};
+  const int64_t nw = p.nrows() * p.ldc, nq = (int64_t)rs * pi.n[1] * ldq;
+  const PxOut po{c->pk.as<void>(), c->q1.as<void>(), nb, nw, pk_elems(c), nq};
   bool fused;
   {
     Stage st(c, FC_STAGE_COMBINE);
@@ -897,18 +943,22 @@ void power_x(fc_corr* c, cplx<T>* w, const cplx<T>* b, int mode) {
   if (!fused) {
     // Other x lengths: separate x pass, combine, gather, pruned inverse x
     // (reading the power grid in T, transforming in TI).
-    full_power<T, TI>(c, w, b, mode);
-    gather_pk<T>(c, w);
-    Stage st(c, FC_STAGE_FFT_X_INV);
-    ColView<TI, T> v{w, 0, (int64_t)p.n[1] * p.ldc, (int64_t)p.ldc, c->q1.as<cplx<TI>>(), 0,
-                     (int64_t)p.n[1] * ldq, ldq, 1, p.n[1], p.n2h, rs, o};
-    launch_cols<TI, +1, T>(p.n[0], v, pi.tile[0], pi.tw0.as<cplx<TI>>(), s, pi.gen[0].get());
+    for (int i = 0; i < nb; ++i) {
+      cplx<T>* wi = w + i * nw;
+      full_power<T, TI>(c, wi, b, mode);
+      gather_pk<T>(c, wi, i);
+      Stage st(c, FC_STAGE_FFT_X_INV);
+      ColView<TI, T> v{wi, 0, (int64_t)p.n[1] * p.ldc, (int64_t)p.ldc,
+                       c->q1.as<cplx<TI>>() + i * nq, 0, (int64_t)p.n[1] * ldq, ldq, 1, p.n[1],
+                       p.n2h, rs, o};
+      launch_cols<TI, +1, T>(p.n[0], v, pi.tile[0], pi.tw0.as<cplx<TI>>(), s, pi.gen[0].get());
+    }
   }
 }
 
 // Pruned inverse y and z passes: q1 -> q2 -> the r subgrid xisub, on stream s.
 template <typename T, typename TI>
-void pruned_inverse_yz(fc_corr* c, hipStream_t s) {
+void pruned_inverse_yz(fc_corr* c, hipStream_t s, int nb = 1) {
   const FftPlan& pi = *c->plan_inv;
   const int64_t ldq = pi.ldc;
   const int rs = c->rshape, o = rs / 2;
@@ -916,13 +966,13 @@ void pruned_inverse_yz(fc_corr* c, hipStream_t s) {
   {
     Stage st(c, FC_STAGE_FFT_Y_INV);
     ColView<TI> v{c->q1.as<cplx<TI>>(), (int64_t)pi.n[1] * ldq, ldq, 0, c->q2.as<cplx<TI>>(),
-                  (int64_t)rs * ldq, ldq, 0, rs, 1, pi.n2h, rs, o};
+                  (int64_t)rs * ldq, ldq, 0, nb * rs, 1, pi.n2h, rs, o};
     launch_cols<TI, +1>(pi.n[1], v, pi.tile[1], pi.tw1.as<cplx<TI>>(), s, pi.gen[1].get());
   }
   // Pruned z C2R: rows of q2 -> r subgrid rows xi[sx][sy][sz].
   Stage st(c, FC_STAGE_FFT_Z_INV);
   launch_rows_c2r<TI, TI>(pi, c->q2.as<cplx<TI>>(), ldq, c->xisub.as<TI>(), rs, s,
-                          (int64_t)rs * rs, rs, o);
+                          (int64_t)nb * rs * rs, rs, o, (int64_t)rs * rs);
 }
 
 // Power spectrum with its compact k values (pk) and pruned inverse x (q1),
@@ -1191,7 +1241,8 @@ void yamamoto_plain(fc_corr* c, fc_grid* g1) {
   for (int i = 0; i < 3; ++i) start[i] = 0.5 - (-c->posmin[i] / c->cell);
   for (int ell = 0; ell <= c->maxell; ell += 2) {
     for (int m = -ell; m <= ell; ++m) {
-      LoadYlm ld{ell, m, p.n[1], ylm_coeff(ell, m, 1.0), start[0], start[1], start[2]};
+      LoadYlm ld{ell, m, p.n[1], ylm_coeff(ell, 0, 1.0), ylm_coeff(ell, 1, 1.0), start[0],
+                 start[1], start[2], (uint32_t)p.nrows()};
       forward_zy<T>(c, g1, w, ld);
       full_power<T>(c, w, c->grid2_fft.as<cplx<T>>(), kModeCross);
       gather_pk<T>(c, w);
@@ -1210,9 +1261,11 @@ template <typename T, typename TI>
 void yamamoto_correlate(fc_corr* c, fc_grid* g1, bool own) {
   hipStream_t s = c->ctx->stream;
   const FftPlan& p = *c->plan;
+  const int most = yamamoto_most(c);
+  c->work.reserve(most * p.complex_bytes());
   cplx<T>* w = c->work.as<cplx<T>>();
   const uint64_t ncells = (uint64_t)c->shape[0] * c->shape[1] * c->shape[2];
-  ensure_periodic_buffers<T, TI>(c);
+  ensure_periodic_buffers<T, TI>(c, most);
   ensure_phase_tables(c);
   ensure_subgrids(c, false);
   // Observer at the survey origin; cell centres 0.5 - observer + i
@@ -1232,8 +1285,10 @@ void yamamoto_correlate(fc_corr* c, fc_grid* g1, bool own) {
   c->part_k.reserve(sizeof(double) * (size_t)std::max(kcells.nchunks, 1) * (2 * c->maxell + 1));
   bool pending = false;
   for (int ell = 0; ell <= c->maxell; ell += 2) {
-    const int row = ell / 2;
-    for (int m = -ell; m <= ell; ++m) {
+    const int row = ell / 2, group = yamamoto_group(c, ell);
+    for (int m = -ell, nm; m <= ell; m += nm) {
+      nm = std::min(group, ell - m + 1);
+      const bool last = m + nm > ell;
       const bool plain = own && ell == 0;
       const double y00 = plain ? ylm_coeff(0, 0, 1.0) : 1.0;
       if (plain) {
@@ -1241,13 +1296,14 @@ void yamamoto_correlate(fc_corr* c, fc_grid* g1, bool own) {
         store_grid2<T, TI>(c, w);
         power_x<T, TI>(c, w, nullptr, kModeAuto);
       } else {
-        LoadYlm ld{ell, m, p.n[1], ylm_coeff(ell, m, 1.0), start[0], start[1], start[2]};
-        forward_zy<T, TI>(c, g1, w, ld);
+        LoadYlm ld{ell, m, p.n[1], ylm_coeff(ell, 0, 1.0), ylm_coeff(ell, 1, 1.0), start[0],
+                   start[1], start[2], (uint32_t)p.nrows()};
+        forward_zy<T, TI>(c, g1, w, ld, nm);
         if (pending) {
           FC_HIP(hipStreamWaitEvent(s, c->ev_join, 0));
           FC_HIP(hipStreamWaitEvent(s, c->ev_inv, 0));
         }
-        power_x<T, TI>(c, w, c->grid2_fft.as<cplx<T>>(), kModeCross);
+        power_x<T, TI>(c, w, c->grid2_fft.as<cplx<T>>(), kModeCross, nm);
       }
       if (par) {
         FC_HIP(hipEventRecord(c->ev_fork, s));
@@ -1259,37 +1315,39 @@ void yamamoto_correlate(fc_corr* c, fc_grid* g1, bool own) {
         // compact k values; the shares are summed once per l.
         Stage st(c, FC_STAGE_HIST_K);
         double* part = c->part_k.as<double>() + (size_t)(m + ell) * kcells.nchunks;
-        const double coef = ylm_coeff(ell, m, 4.0 * M_PI) * y00;
+        const double coef0 = ylm_coeff(ell, 0, 4.0 * M_PI) * y00;
+        const double coef = ylm_coeff(ell, 1, 4.0 * M_PI) * y00;
         if (c->khalf_ok) {
           const int nz = c->kshape[2] / 2 + 1, oz = c->kshape[2] / 2;
           KEntryHalfLm<T> ke{c->khalf.cells.as<uint32_t>(), c->pk.as<T>(),
                              FastDiv((uint32_t)nz), FastDiv((uint32_t)c->kshape[1]), nz,
                              c->kshape[1], c->kx.as<double>(), c->ky.as<double>(),
                              c->kz.as<double>() + oz, c->wx.as<double>(), c->wy.as<double>(),
-                             c->wz.as<double>() + oz, ell, m, coef};
-          hist_seg_partials<1>(ke, kcells, part, ks);
+                             c->wz.as<double>() + oz, ell, m, coef0, coef, pk_elems(c)};
+          hist_seg_partials<1>(ke, kcells, part, ks, -1, nullptr, nm);
         } else {
           KEntryLm<T> ke{c->kbin.cells.as<uint32_t>(), c->pk.as<T>(), kslots(c),
                          FastDiv((uint32_t)c->kshape[2]), FastDiv((uint32_t)c->kshape[1]),
                          c->kx.as<double>(), c->ky.as<double>(), c->kz.as<double>(),
                          c->wx.as<double>(), c->wy.as<double>(), c->wz.as<double>(), ell, m,
-                         coef};
-          hist_seg_partials<1>(ke, kcells, part, ks);
+                         coef0, coef, pk_elems(c)};
+          hist_seg_partials<1>(ke, kcells, part, ks, -1, nullptr, nm);
         }
-        if (m == ell)
+        if (last)
           hist_seg_sum<1>(kcells, c->part_k.as<double>(), 2 * ell + 1, c->k_hist.as<double>(),
                           c->k_counts.as<int>(), row, row, row + 1, ks, 1, 0,
                           c->kbin.counts.as<int>());
       }
-      pruned_inverse_yz<T, TI>(c, is);
+      pruned_inverse_yz<T, TI>(c, is, nm);
       {
         Stage st(c, FC_STAGE_SUBGRID);
         hipLaunchKernelGGL(k_acc_r<TI>, dim3(grid1d(nr, 256, 65536)), dim3(256), 0, is,
                            c->rsub.as<double>(), c->xisub.as<TI>(), rs, c->rx.as<double>(), ell,
-                           m, ylm_coeff(ell, m, 4.0 * M_PI / ncells) * y00, m == -ell);
+                           m, nm, ylm_coeff(ell, 0, 4.0 * M_PI / ncells) * y00,
+                           ylm_coeff(ell, 1, 4.0 * M_PI / ncells) * y00, m == -ell);
         FC_LAUNCH_CHECK();
       }
-      if (m == ell) hist_subgrids(c, ell, false, true, is);
+      if (last) hist_subgrids(c, ell, false, true, is);
       if (par) {
         FC_HIP(hipEventRecord(c->ev_join, ks));
         FC_HIP(hipEventRecord(c->ev_inv, is));
@@ -1470,13 +1528,14 @@ int fc_corr_footprint(fc_corr* c, int interlaced, size_t* held, size_t* full) {
     // spectra in work, otherwise the second sits in work_b (grids of two
     // precisions take that path too: then this is an upper bound).
     const bool pair = interlaced && c->algo != FC_ALGO_PLAIN && fc::forward_pair_plan_ok(c);
-    add(c->work, pair ? 2 * cb : cb);
+    const size_t nb = c->kind == FC_YAMAMOTO ? fc::yamamoto_most(c) : 1;
+    add(c->work, std::max<size_t>(pair ? 2 : 1, nb) * cb);
     add(c->work_b, interlaced && !pair ? cb : 0);
     add(c->grid2_fft, c->kind == FC_YAMAMOTO || c->have_grid2 ? cb : 0);
-    add(c->pk, ts * (size_t)c->kshape[0] * c->kshape[1] * (c->kshape[2] / 2 + 1));
-    add(c->q1, 2 * tsi * rs * pi.n[1] * pi.ldc);
-    add(c->q2, 2 * tsi * rs * rs * pi.ldc);
-    add(c->xisub, tsi * rs * rs * rs);
+    add(c->pk, ts * nb * (size_t)fc::pk_elems(c));
+    add(c->q1, 2 * tsi * nb * rs * pi.n[1] * pi.ldc);
+    add(c->q2, 2 * tsi * nb * rs * rs * pi.ldc);
+    add(c->xisub, tsi * nb * rs * rs * rs);
     add(c->rsub, c->kind == FC_YAMAMOTO || c->algo == FC_ALGO_PLAIN ? 8 * rs * rs * rs : 0);
     add(c->ksub, c->algo == FC_ALGO_PLAIN ? 8 * K : 0);
     add(c->rw, 8 * nv * (size_t)std::max<int64_t>(c->rbin.n, 1));

@@ -35,8 +35,8 @@ __global__ void __launch_bounds__(gen_max_threads<RM>())
   const int64_t rb = two ? r0 + 1 : 0;
   const auto la = ld.row(ra);
   const auto lb = ld.row(rb);
-  const Tin* pa = in + ra * ldi + j;
-  const Tin* pb = in + rb * ldi + j;
+  const Tin* pa = in + ld.src(ra) * ldi + j;
+  const Tin* pb = in + ld.src(rb) * ldi + j;
   // A row without a partner is paired with zeros: a partner's values would
   // enter its rounding.
   auto load = [&](int r, int u) {

@@ -872,7 +872,7 @@ __global__ void __launch_bounds__(1024)
     using P = typename PairOf<Tin>::type;
     const int64_t rowc = rowok ? row : 0;
     const P* src = reinterpret_cast<const P*>(
-        in2 && rowc >= nrows1 ? in2 + (rowc - nrows1) * ldi : in + rowc * ldi);
+        in2 && rowc >= nrows1 ? in2 + (rowc - nrows1) * ldi : in + ld.src(rowc) * ldi);
     const auto lr = ld.row(rowc);
     P pv[E];
 #pragma unroll
@@ -1080,6 +1080,8 @@ struct LoadCopy {
     __device__ __forceinline__ double operator()(double v, int) const { return v; }
   };
   __device__ __forceinline__ Row row(int64_t) const { return Row{}; }
+  // Input row of output row r.
+  __device__ __forceinline__ int64_t src(int64_t r) const { return r; }
   void shift_x(int) {}  // rows restart at a later x slab: nothing to adjust
 };
 
@@ -1094,8 +1096,9 @@ __global__ void __launch_bounds__(256) k_dft_rows_r2c(const Tin* in, int64_t ldi
   T* x = reinterpret_cast<T*>(smem_raw);
   const int64_t row = blockIdx.x;
   const auto lr = ld.row(row);
+  const int64_t irow = ld.src(row);
   for (int n = threadIdx.x; n < n2; n += blockDim.x)
-    x[n] = T(lr((double)in[row * ldi + n], n));
+    x[n] = T(lr((double)in[irow * ldi + n], n));
   __syncthreads();
   // Every global read of the row happened before the barrier above, so the
   // output row may alias the input row (in-place transform).
