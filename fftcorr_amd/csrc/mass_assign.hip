@@ -6,12 +6,13 @@
 // particle's 27 weights into the grid slab by slab.  Here:
 //   1. k_ma_prepare   grid coordinates / skip test (config_space_grid.h:31-46),
 //                     the key cell (the cell holding the particle; for CIC the
-//                     lower corner of its 2x2x2 block of target cells), the
-//                     offsets from it and FP64 weight sums per block;
+//                     lower corner of its 2x2x2 block of target cells) and FP64
+//                     weight sums per block;
 //   2. stable radix sort of (key, particle index) (radix_sort.h: passes of
 //      at most 8 bits over the bits the largest key needs): within a key
 //      cell the particles keep their input order;
-//   3. k_permute      records in sorted order;
+//   3. k_records      records (offsets from the key cell, weight) in sorted
+//                     order, from the particles again;
 //   4. k_row_bounds   per grid row (x, y), the sorted particles at the borders
 //                     of its z tiles (binary searches);
 //   5. k_ma_tile      one wave per 8 x 32 tile of target cells of an x plane:
@@ -28,6 +29,7 @@
 #include <vector>
 
 #include "fc_objects.h"
+#include "philox.h"
 #include "radix_sort.h"
 #include "xcd.h"
 
@@ -82,36 +84,47 @@ __device__ __forceinline__ int key_axis(double x, double anchor, int n, double* 
   return a;
 }
 
-// Particles: pos [n, ncol] (ncol 3 or 4), weights [n] or null.  Skipped
-// particles get the key `sentinel` (sorted after every cell).
-__global__ void __launch_bounds__(kPrepThreads)
-    k_ma_prepare(const double* __restrict__ pos, int64_t n, int ncol,
-                 const double* __restrict__ weights, double w_scalar, GridGeom g, int wrap,
-                 double shift, double anchor, bool keep_z, uint32_t sentinel,
-                 uint32_t* __restrict__ keys,
-                 uint32_t* __restrict__ idx, double4* __restrict__ rec,
-                 double* __restrict__ part_w, unsigned long long* __restrict__ part_n) {
-#pragma clang fp contract(off)
-  __shared__ double sd[kPrepThreads / kWave];
-  __shared__ unsigned long long su[kPrepThreads / kWave];
-  const int64_t chunk = (n + gridDim.x - 1) / gridDim.x;
-  const int64_t lo = (int64_t)blockIdx.x * chunk;
-  const int64_t hi = lo + chunk < n ? lo + chunk : n;
-  double tw = 0.0, tw2 = 0.0;
-  unsigned long long added = 0;
-  for (int64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) {
+// Where the particles come from: an array pos [n, ncol] (ncol 3 or 4) with
+// weights [n] or null, or the random generator.  Each particle is asked for
+// twice, for its key and, in sorted order, for its record: cheaper than
+// keeping 32 bytes per particle in input order in between.
+struct ArraySource {
+  const double* pos;
+  int ncol;
+  const double* weights;
+  double w_scalar;
+  __device__ __forceinline__ double4 operator()(int64_t i) const {
     const double* p = pos + i * ncol;
-    const double w = ncol == 4 ? p[3] : (weights ? weights[i] : w_scalar);
+    return make_double4(p[0], p[1], p[2],
+                        ncol == 4 ? p[3] : (weights ? weights[i] : w_scalar));
+  }
+};
+struct UniformSource {
+  double3 lo, span;
+  uint64_t seed, first;
+  double weight;
+  __device__ __forceinline__ double4 operator()(int64_t i) const {
+    const double3 p = random_uniform(lo, span, seed, first + (uint64_t)i);
+    return make_double4(p.x, p.y, p.z, weight);
+  }
+};
+
+// Key and record (offsets from the key cell, weight) of particle p; false if
+// it is skipped.  The record's z is the position itself unless cell_z (the
+// key cell along z is found from it again).
+struct Locator {
+  GridGeom g;
+  int wrap;
+  double shift, anchor;
+  bool cell_z;
+  __device__ __forceinline__ bool operator()(const double4& p, uint32_t* key,
+                                             double4* rec) const {
+#pragma clang fp contract(off)
     double x, y, z;
-    const bool ok = to_grid(p[0], g.p0, g.cell, g.n0, wrap, &x) &&
-                    to_grid(p[1], g.p1, g.cell, g.n1, wrap, &y) &&
-                    to_grid(p[2], g.p2, g.cell, g.n2, wrap, &z);
-    idx[i] = (uint32_t)i;
-    if (!ok) {
-      keys[i] = sentinel;
-      rec[i] = make_double4(0, 0, 0, 0);
-      continue;
-    }
+    if (!(to_grid(p.x, g.p0, g.cell, g.n0, wrap, &x) &&
+          to_grid(p.y, g.p1, g.cell, g.n1, wrap, &y) &&
+          to_grid(p.z, g.p2, g.cell, g.n2, wrap, &z)))
+      return false;
     if (shift != 0.0) {  // interlaced grid: displace by `shift` cells, wrap
       x += shift;
       y += shift;
@@ -124,11 +137,37 @@ __global__ void __launch_bounds__(kPrepThreads)
     const int ix = key_axis(x, anchor, g.n0, &rx);
     const int iy = key_axis(y, anchor, g.n1, &ry);
     const int iz = key_axis(z, anchor, g.n2, &rz);
-    keys[i] = (uint32_t)(((uint64_t)ix * g.n1 + iy) * g.n2 + iz);
-    rec[i] = make_double4(rx, ry, keep_z ? z - anchor : rz, w);
-    tw += w;
-    tw2 += w * w;
-    added += 1;
+    *key = (uint32_t)(((uint64_t)ix * g.n1 + iy) * g.n2 + iz);
+    *rec = make_double4(rx, ry, cell_z ? rz : z - anchor, p.w);
+    return true;
+  }
+};
+
+// Keys (skipped particles get `sentinel`, sorted after every cell) and the
+// weight sums per block.
+template <class Source>
+__global__ void __launch_bounds__(kPrepThreads)
+    k_ma_prepare(Source src, int64_t n, Locator loc, uint32_t sentinel,
+                 uint32_t* __restrict__ keys, double* __restrict__ part_w,
+                 unsigned long long* __restrict__ part_n) {
+#pragma clang fp contract(off)
+  __shared__ double sd[kPrepThreads / kWave];
+  __shared__ unsigned long long su[kPrepThreads / kWave];
+  const int64_t chunk = (n + gridDim.x - 1) / gridDim.x;
+  const int64_t lo = (int64_t)blockIdx.x * chunk;
+  const int64_t hi = lo + chunk < n ? lo + chunk : n;
+  double tw = 0.0, tw2 = 0.0;
+  unsigned long long added = 0;
+  for (int64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) {
+    const double4 p = src(i);
+    uint32_t key = sentinel;
+    double4 rec;
+    if (loc(p, &key, &rec)) {
+      tw += p.w;
+      tw2 += p.w * p.w;
+      added += 1;
+    }
+    keys[i] = key;
   }
   tw = block_sum(tw, sd);
   tw2 = block_sum(tw2, sd);
@@ -167,11 +206,19 @@ __global__ void __launch_bounds__(kWave)
   }
 }
 
-__global__ void k_permute(const uint32_t* __restrict__ order, const double4* __restrict__ rec,
-                          double4* __restrict__ out, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    out[i] = rec[order[i]];
+// The records of the particles on the grid, in sorted order.
+template <class Source>
+__global__ void k_records(const uint32_t* __restrict__ order, Source src, Locator loc,
+                          const unsigned long long* __restrict__ nvalid_p,
+                          double4* __restrict__ out) {
+  const int64_t nvalid = (int64_t)*nvalid_p;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nvalid;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    uint32_t key;
+    double4 rec = make_double4(0, 0, 0, 0);
+    loc(src(order[i]), &key, &rec);
+    out[i] = rec;
+  }
 }
 
 __global__ void k_zero_i32(int32_t* __restrict__ p, int64_t n) {
@@ -628,12 +675,11 @@ struct RunScratch {
   }
 };
 
-void mass_assign(fc_grid* grid, const double* pos_dev, int64_t n, int ncol,
-                 const double* w_dev, double w_scalar, int scheme, int wrap, double shift,
+template <class Source>
+void mass_assign(fc_grid* grid, const Source& src, int64_t n, int scheme, int wrap, double shift,
                  fc_ma_stats* stats) {
   if (scheme < 0 || scheme > 3)
     fail(FC_ERR_INVALID, "unknown distribution scheme " + std::to_string(scheme));
-  if (ncol != 3 && ncol != 4) fail(FC_ERR_INVALID, "Rows must be 3D or 4D.");
   if (n < 0) fail(FC_ERR_INVALID, "negative particle count");
   if (n > 0x7fffffffLL) fail(FC_ERR_INVALID, "more than 2^31-1 particles in one call");
   if (!(shift >= 0.0 && shift < 1.0)) fail(FC_ERR_INVALID, "shift must be in [0, 1)");
@@ -668,20 +714,19 @@ void mass_assign(fc_grid* grid, const double* pos_dev, int64_t n, int ncol,
   sc[2].reserve(sizeof(uint32_t) * n);
   sc[3].reserve(sizeof(uint32_t) * n);
   sc[4].reserve(sizeof(uint32_t) * n);
-  sc[5].reserve(sizeof(double4) * n);
   sc[6].reserve(sizeof(double4) * n);
   sc[7].reserve(sizeof(double) * 2 * (nbp + 2));
   sc[8].reserve(sizeof(unsigned long long) * (nbp + 1));
   const RunScratch rs(grid->shape, scheme == 2);
   sc[9].reserve(rs.runs);
   sc[11].reserve(rs.occ);
-  DeviceBuffer &keys = sc[1], &keys2 = sc[2], &idx = sc[3], &idx2 = sc[4], &rec = sc[5],
-               &srec = sc[6], &partw = sc[7], &partn = sc[8], &runs = sc[9], &occ = sc[11];
+  DeviceBuffer &keys = sc[1], &keys2 = sc[2], &idx = sc[3], &idx2 = sc[4], &srec = sc[6],
+               &partw = sc[7], &partn = sc[8], &runs = sc[9], &occ = sc[11];
   const double anchor = scheme == 3 ? 0.5 : 0.0;  // CIC keys by its 2x2x2 block
 
-  hipLaunchKernelGGL(k_ma_prepare, dim3(nbp), dim3(kPrepThreads), 0, s, pos_dev, n, ncol, w_dev,
-                     w_scalar, gg, wrap, shift, anchor, scheme != 2, (uint32_t)sentinel, keys.as<uint32_t>(),
-                     idx.as<uint32_t>(), rec.as<double4>(), partw.as<double>(),
+  const Locator loc{gg, wrap, shift, anchor, scheme == 2};
+  hipLaunchKernelGGL(k_ma_prepare<Source>, dim3(nbp), dim3(kPrepThreads), 0, s, src, n, loc,
+                     (uint32_t)sentinel, keys.as<uint32_t>(), partw.as<double>(),
                      partn.as<unsigned long long>());
   FC_LAUNCH_CHECK();
   // The sums of w and w^2 and the number of particles on the grid, read back as one.
@@ -699,8 +744,8 @@ void mass_assign(fc_grid* grid, const double* pos_dev, int64_t n, int ncol,
                                        ctx->scratch[0].as<void>(), s);
   const uint32_t* skeys = second ? keys2.as<uint32_t>() : keys.as<uint32_t>();
   const uint32_t* sidx = second ? idx2.as<uint32_t>() : idx.as<uint32_t>();
-  hipLaunchKernelGGL(k_permute, dim3(grid1d(n, 256, 65536)), dim3(256), 0, s, sidx,
-                     rec.as<double4>(), srec.as<double4>(), n);
+  hipLaunchKernelGGL(k_records<Source>, dim3(grid1d(n, 256, 65536)), dim3(256), 0, s, sidx, src,
+                     loc, nvalid, srec.as<double4>());
   FC_LAUNCH_CHECK();
   if (scheme == 2) {
     const int64_t nwords = (int64_t)(rs.occ / sizeof(uint32_t));
@@ -749,7 +794,15 @@ void mass_assign(fc_grid* grid, const double* pos_dev, int64_t n, int ncol,
 void mass_assign_device(fc_grid* grid, const double* pos_dev, int64_t n, int ncol,
                         const double* w_dev, double w_scalar, int scheme, int wrap, double shift,
                         fc_ma_stats* stats) {
-  mass_assign(grid, pos_dev, n, ncol, w_dev, w_scalar, scheme, wrap, shift, stats);
+  if (ncol != 3 && ncol != 4) fail(FC_ERR_INVALID, "Rows must be 3D or 4D.");
+  mass_assign(grid, ArraySource{pos_dev, ncol, w_dev, w_scalar}, n, scheme, wrap, shift, stats);
+}
+
+// n particles of the random generator, uniform in [lo, lo + span).
+void mass_assign_uniform(fc_grid* grid, int64_t n, double3 lo, double3 span, uint64_t seed,
+                         uint64_t first, double weight, int scheme, int wrap,
+                         fc_ma_stats* stats) {
+  mass_assign(grid, UniformSource{lo, span, seed, first, weight}, n, scheme, wrap, 0.0, stats);
 }
 
 }  // namespace fc
@@ -788,7 +841,7 @@ int fc_mass_assign_footprint(fc_grid* grid, int64_t n, int ncol, int has_weights
                                sizeof(uint32_t) * n,
                                sizeof(uint32_t) * n,
                                sizeof(uint32_t) * n,
-                               sizeof(double4) * n,
+                               0,
                                sizeof(double4) * n,
                                sizeof(double) * 2 * (nbp + 2),
                                sizeof(unsigned long long) * (nbp + 1),
@@ -809,8 +862,8 @@ int fc_mass_assign_device(fc_grid* grid, const double* pos_dev, int64_t n, int n
   return fc::guard([&] {
     fc::check_grid(grid);
     if (n > 0 && !pos_dev) fc::fail(FC_ERR_INVALID, "null positions");
-    fc::mass_assign(grid, pos_dev, n, ncol, weights_dev, w_scalar, scheme, periodic_wrap,
-                    shift, stats);
+    fc::mass_assign_device(grid, pos_dev, n, ncol, weights_dev, w_scalar, scheme, periodic_wrap,
+                           shift, stats);
   });
 }
 
@@ -831,7 +884,7 @@ int fc_mass_assign(fc_grid* grid, const double* pos, int64_t n, int ncol,
     if (!ctx->copier) ctx->copier.reset(new fc::HostCopier(ctx->device));
     FC_HIP(ctx->copier->copy(dpos, pos, sizeof(double) * n * ncol, s));
     if (weights) FC_HIP(ctx->copier->copy(dw, weights, sizeof(double) * n, s));
-    fc::mass_assign(grid, dpos, n, ncol, dw, w_scalar, scheme, periodic_wrap, shift, stats);
+    fc::mass_assign_device(grid, dpos, n, ncol, dw, w_scalar, scheme, periodic_wrap, shift, stats);
   });
 }
 

@@ -155,7 +155,7 @@ __global__ void __launch_bounds__(kRsThreads)
   for (int r = 0; r < kRsRounds; ++r) {
     const int64_t k = wk0 + r * 64 + lane;
     key[r] = k < n ? kin[k] : 0u;
-    val[r] = k < n ? vin[k] : 0u;
+    val[r] = k >= n ? 0u : vin ? vin[k] : (uint32_t)k;
   }
   const unsigned long long below = (1ull << lane) - 1ull;
 #pragma unroll
@@ -210,8 +210,8 @@ __global__ void __launch_bounds__(kRsThreads)
   }
 }
 
-// Sorts n pairs (k1, v1) by the low `bits` key bits with (k2, v2) as the
-// second buffer and scratch (RadixPlan::scratch_bytes) for the counts.
+// Sorts n pairs (k1[i], i) by the low `bits` key bits, with (k2, v2) as the
+// second buffer (the first pass reads no values) and scratch (RadixPlan::scratch_bytes) for the counts.
 // Returns true when the result is in (k2, v2), false when in (k1, v1).
 inline bool radix_sort_pairs(uint32_t* k1, uint32_t* k2, uint32_t* v1, uint32_t* v2, int64_t n,
                              int bits, void* scratch, hipStream_t s) {
@@ -222,7 +222,7 @@ inline bool radix_sort_pairs(uint32_t* k1, uint32_t* k2, uint32_t* v1, uint32_t*
   if (p.tiles > INT32_MAX / kRsMaxDigits) fail(FC_ERR_INVALID, "too many particles for one sort");
   int32_t* counts = static_cast<int32_t*>(scratch);
   int32_t* totals = counts + (size_t)p.tiles * p.nb;
-  uint32_t *ki = k1, *ko = k2, *vi = v1, *vo = v2;
+  uint32_t *ki = k1, *ko = k2, *vi = nullptr, *vo = v2;
   for (int q = 0; q < p.passes; ++q) {
     const int shift = q * p.dbits;
     hipLaunchKernelGGL(k_rs_count, dim3((unsigned)p.tiles), dim3(kRsThreads), 0, s, ki, n, shift,
@@ -235,7 +235,8 @@ inline bool radix_sort_pairs(uint32_t* k1, uint32_t* k2, uint32_t* v1, uint32_t*
                        vo, n, shift, p.dbits, counts, totals);
     FC_LAUNCH_CHECK();
     std::swap(ki, ko);
-    std::swap(vi, vo);
+    vi = vo;
+    vo = vi == v2 ? v1 : v2;
   }
   return p.passes % 2 == 1;
 }

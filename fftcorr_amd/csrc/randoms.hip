@@ -1,48 +1,10 @@
 // Random catalogues and displacement fields on the device
 // (fftcorr/catalog/random_catalog.py:8-87, fftcorr/grid/utils.pyx:19-55).
-//
-// Randoms come from a counter-based generator, Philox4x32-10 (Salmon,
-// Moraes, Dror and Shaw, "Parallel random numbers: as easy as 1, 2, 3",
-// SC 2011): 10 rounds of two 32x32->64-bit multiplies with the key bumped by
-// the Weyl constants between rounds.  Particle i of stream `seed` uses the
-// counters (i, 0, 0) and (i, 1, 0) -- two 4-word draws, six words -> three
-// 53-bit uniforms -- so any range of particles can be generated
-// independently and the catalogue is the same however it is batched.
 #include "fc_objects.h"
+#include "philox.h"
 
 namespace fc {
 namespace {
-
-struct Philox {
-  uint32_t c[4];
-};
-
-__host__ __device__ inline void mulhilo(uint32_t a, uint32_t b, uint32_t* hi, uint32_t* lo) {
-  const uint64_t p = (uint64_t)a * b;
-  *hi = (uint32_t)(p >> 32);
-  *lo = (uint32_t)p;
-}
-
-__host__ __device__ inline Philox philox4x32_10(Philox x, uint32_t k0, uint32_t k1) {
-  const uint32_t M0 = 0xD2511F53u, M1 = 0xCD9E8D57u;
-  const uint32_t W0 = 0x9E3779B9u, W1 = 0xBB67AE85u;
-  for (int r = 0; r < 10; ++r) {
-    if (r > 0) {
-      k0 += W0;
-      k1 += W1;
-    }
-    uint32_t hi0, lo0, hi1, lo1;
-    mulhilo(M0, x.c[0], &hi0, &lo0);
-    mulhilo(M1, x.c[2], &hi1, &lo1);
-    x = Philox{{hi1 ^ x.c[1] ^ k0, lo1, hi0 ^ x.c[3] ^ k1, lo0}};
-  }
-  return x;
-}
-
-// Uniform in [0, 1) from two words: 27 + 26 bits (53 in all).
-__device__ __forceinline__ double u53(uint32_t a, uint32_t b) {
-  return ((double)(a >> 5) * 67108864.0 + (double)(b >> 6)) * (1.0 / 9007199254740992.0);
-}
 
 __global__ void k_random_raw(uint32_t* __restrict__ out, int64_t n, uint64_t seed,
                              uint64_t first, uint32_t w2, uint32_t w3) {
@@ -61,14 +23,10 @@ __global__ void k_random_uniform(double* __restrict__ pos, int64_t n, double3 lo
 #pragma clang fp contract(off)
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
-    const uint64_t ctr = first + (uint64_t)i;
-    const uint32_t c0 = (uint32_t)ctr, c1 = (uint32_t)(ctr >> 32);
-    const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
-    const Philox a = philox4x32_10(Philox{{c0, c1, 0u, 0u}}, k0, k1);
-    const Philox b = philox4x32_10(Philox{{c0, c1, 1u, 0u}}, k0, k1);
-    pos[3 * i + 0] = lo.x + u53(a.c[0], a.c[1]) * span.x;
-    pos[3 * i + 1] = lo.y + u53(a.c[2], a.c[3]) * span.y;
-    pos[3 * i + 2] = lo.z + u53(b.c[0], b.c[1]) * span.z;
+    const double3 p = random_uniform(lo, span, seed, first + (uint64_t)i);
+    pos[3 * i + 0] = p.x;
+    pos[3 * i + 1] = p.y;
+    pos[3 * i + 2] = p.z;
   }
 }
 
@@ -117,6 +75,9 @@ __global__ void k_apply_disp(const double* __restrict__ pos, int64_t n,
 void mass_assign_device(fc_grid* grid, const double* pos_dev, int64_t n, int ncol,
                         const double* w_dev, double w_scalar, int scheme, int wrap, double shift,
                         fc_ma_stats* stats);
+void mass_assign_uniform(fc_grid* grid, int64_t n, double3 lo, double3 span, uint64_t seed,
+                         uint64_t first, double weight, int scheme, int wrap,
+                         fc_ma_stats* stats);
 
 }  // namespace fc
 
@@ -227,12 +188,13 @@ int fc_add_random_particles(fc_grid* grid, int64_t n, double weight, int scheme,
     fc::DeviceGuard dg(ctx->device);
     hipStream_t s = ctx->stream;
     const int64_t nb = std::min<int64_t>(n, batch);
-    fc::DeviceBuffer pos(sizeof(double) * 3 * nb), moved, ddisp, bad;
+    fc::DeviceBuffer pos, moved, ddisp, bad;
     const double lo[3] = {grid->posmin[0], grid->posmin[1], grid->posmin[2]};
     double3 span = make_double3(grid->cell * grid->shape[0], grid->cell * grid->shape[1],
                                 grid->cell * grid->shape[2]);
     if (disp) {
       const size_t nd = (size_t)grid->size() * 3;
+      pos.allocate(sizeof(double) * 3 * nb);
       ddisp.allocate(sizeof(double) * nd);
       moved.allocate(sizeof(double) * 3 * nb);
       bad.allocate(sizeof(unsigned long long));
@@ -242,21 +204,22 @@ int fc_add_random_particles(fc_grid* grid, int64_t n, double weight, int scheme,
     }
     for (int64_t first = 0; first < n; first += nb) {
       const int64_t m = std::min(nb, n - first);
+      if (!disp) {  // drawn where they are assigned: no positions in memory
+        fc::mass_assign_uniform(grid, m, make_double3(lo[0], lo[1], lo[2]), span, seed,
+                                (uint64_t)first, weight, scheme, periodic_wrap, stats);
+        continue;
+      }
       hipLaunchKernelGGL(fc::k_random_uniform, dim3(fc::grid1d(m, 256, 65536)), dim3(256), 0, s,
                          pos.as<double>(), m, make_double3(lo[0], lo[1], lo[2]), span, seed,
                          (uint64_t)first);
       FC_LAUNCH_CHECK();
-      const double* p = pos.as<double>();
-      if (disp) {
-        hipLaunchKernelGGL(fc::k_apply_disp, dim3(fc::grid1d(m, 256, 65536)), dim3(256), 0, s,
-                           pos.as<double>(), m, ddisp.as<double>(), grid->shape[0],
-                           grid->shape[1], grid->shape[2], grid->posmin[0], grid->posmin[1],
-                           grid->posmin[2], grid->cell, periodic_wrap, moved.as<double>(),
-                           bad.as<unsigned long long>());
-        FC_LAUNCH_CHECK();
-        p = moved.as<double>();
-      }
-      fc::mass_assign_device(grid, p, m, 3, nullptr, weight, scheme, periodic_wrap, 0.0, stats);
+      hipLaunchKernelGGL(fc::k_apply_disp, dim3(fc::grid1d(m, 256, 65536)), dim3(256), 0, s,
+                         pos.as<double>(), m, ddisp.as<double>(), grid->shape[0], grid->shape[1],
+                         grid->shape[2], grid->posmin[0], grid->posmin[1], grid->posmin[2],
+                         grid->cell, periodic_wrap, moved.as<double>(),
+                         bad.as<unsigned long long>());
+      FC_LAUNCH_CHECK();
+      fc::mass_assign_device(grid, moved.as<double>(), m, 3, nullptr, weight, scheme, periodic_wrap, 0.0, stats);
     }
     if (disp) {
       unsigned long long nbad = 0;
