@@ -1242,7 +1242,7 @@ void yamamoto_plain(fc_corr* c, fc_grid* g1) {
   for (int ell = 0; ell <= c->maxell; ell += 2) {
     for (int m = -ell; m <= ell; ++m) {
       LoadYlm ld{ell, m, p.n[1], ylm_coeff(ell, 0, 1.0), ylm_coeff(ell, 1, 1.0), start[0],
-                 start[1], start[2], (uint32_t)p.nrows()};
+                 start[1], start[2], (uint32_t)p.nrows(), 1};
       forward_zy<T>(c, g1, w, ld);
       full_power<T>(c, w, c->grid2_fft.as<cplx<T>>(), kModeCross);
       gather_pk<T>(c, w);
@@ -1297,7 +1297,7 @@ void yamamoto_correlate(fc_corr* c, fc_grid* g1, bool own) {
         power_x<T, TI>(c, w, nullptr, kModeAuto);
       } else {
         LoadYlm ld{ell, m, p.n[1], ylm_coeff(ell, 0, 1.0), ylm_coeff(ell, 1, 1.0), start[0],
-                   start[1], start[2], (uint32_t)p.nrows()};
+                   start[1], start[2], (uint32_t)p.nrows(), (uint32_t)nm};
         forward_zy<T, TI>(c, g1, w, ld, nm);
         if (pending) {
           FC_HIP(hipStreamWaitEvent(s, c->ev_join, 0));

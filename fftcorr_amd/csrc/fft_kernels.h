@@ -863,7 +863,7 @@ __global__ void __launch_bounds__(1024)
   cplx<To>* lds = reinterpret_cast<cplx<To>*>(smem_raw);
   const LayRowPad lay{RS};
   const int c = threadIdx.x / TCOL, t = threadIdx.x % TCOL;
-  const int64_t row = (int64_t)blockIdx.x * tr + c;
+  const int64_t row = (int64_t)ld.block(blockIdx.x, gridDim.x) * tr + c;
   const bool rowok = row < nrows;
   C v[1][E];
   {
@@ -880,7 +880,8 @@ __global__ void __launch_bounds__(1024)
 #pragma unroll
     for (int s = 0; s < E; ++s) {
       const int e = t + in_m<M, V>(s) * TCOL;
-      const C z{T(lr((double)pv[s].x, 2 * e)), T(lr((double)pv[s].y, 2 * e + 1))};
+      const double2 x = lr.pair((double)pv[s].x, (double)pv[s].y, 2 * e);
+      const C z{T(x.x), T(x.y)};
       v[0][s] = rowok ? z : C{T(0), T(0)};
     }
   }
@@ -1078,8 +1079,14 @@ __global__ void __launch_bounds__(256)
 struct LoadCopy {
   struct Row {
     __device__ __forceinline__ double operator()(double v, int) const { return v; }
+    // Samples k and k + 1.
+    __device__ __forceinline__ double2 pair(double v, double w, int) const {
+      return make_double2(v, w);
+    }
   };
   __device__ __forceinline__ Row row(int64_t) const { return Row{}; }
+  // Order of nb blocks.
+  __device__ __forceinline__ uint32_t block(uint32_t b, uint32_t) const { return b; }
   // Input row of output row r.
   __device__ __forceinline__ int64_t src(int64_t r) const { return r; }
   void shift_x(int) {}  // rows restart at a later x slab: nothing to adjust
