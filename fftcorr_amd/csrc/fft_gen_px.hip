@@ -9,8 +9,15 @@
 namespace fc {
 namespace {
 
-template <typename T, typename TI, int MODE, int RM>
-__global__ void __launch_bounds__(512)
+// WAVES: waves per SIMD the registers are held for.  Four (128 registers) leave
+// room for two workgroups of up to eight waves on a CU; free, they take 137 in
+// interlaced mode and 162 in cross mode, and a CU runs one (interlaced, 500
+// points FP64: 483 us, held 337).  In cross mode holding them costs spills
+// that workgroups of up to four waves, of which three fit anyway, do not earn
+// back (100 points FP64 41 us, held 48; 400 points, seven and a half waves, 291
+// and 222).  Radices above 10 need more than 128.
+template <typename T, typename TI, int MODE, int RM, int WAVES>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WAVES)))
     k_gen_px(PxArgs<T> p, int tilesC, int tiles_per_batch, GenDev g) {
   using C = cplx<T>;
   using CI = cplx<TI>;
@@ -117,12 +124,19 @@ void launch_gen_px(const GenAxis& ax, const PxArgs<T>& p, hipStream_t s) {
   if (nblocks > INT32_MAX) fail(FC_ERR_INVALID, "grid too large for the fused x pass");
   const dim3 blk((unsigned)tc, (unsigned)ax.tcol);
   const size_t lds = (size_t)ax.N * tc * cl;
-  if (ax.rmax <= kGenRadSmall)
-    hipLaunchKernelGGL((k_gen_px<T, TI, MODE, kGenRadSmall>), dim3((unsigned)nblocks), blk, lds,
-                       s, p, tilesC, (int)per, gen_dev(ax));
+  auto go = [&](auto rm, auto waves) {
+    hipLaunchKernelGGL((k_gen_px<T, TI, MODE, decltype(rm)::value, decltype(waves)::value>),
+                       dim3((unsigned)nblocks), blk, lds, s, p, tilesC, (int)per, gen_dev(ax));
+  };
+  using Free = std::integral_constant<int, 2>;
+  using Held = std::integral_constant<int, 4>;
+  using Small = std::integral_constant<int, kGenRadSmall>;
+  if (ax.rmax > kGenRadSmall)
+    go(std::integral_constant<int, 16>{}, Free{});
+  else if (MODE == kModeCross && tc * ax.tcol <= 256)
+    go(Small{}, Free{});
   else
-    hipLaunchKernelGGL((k_gen_px<T, TI, MODE, 16>), dim3((unsigned)nblocks), blk, lds, s, p,
-                       tilesC, (int)per, gen_dev(ax));
+    go(Small{}, Held{});
   FC_LAUNCH_CHECK();
 }
 
