@@ -311,6 +311,10 @@ struct Stencil<3> {  // CIC about cell centres: key cell a <= x - 1/2 < a + 1
 // through the periodic wrap).
 __host__ __device__ inline int row_bounds(int n2) { return 2 * ((n2 + TZ - 1) / TZ) + 2; }
 
+// The 64 entries of a wave lie close together: its two halves first search
+// for the rows they begin and end with, 32 probes a step, and each lane then
+// searches between the two (13 dependent loads instead of 24 at 20 million
+// particles in 512^3; bound by that latency: 203 -> 117 us).
 template <int SCHEME>
 __global__ void k_row_bounds(const uint32_t* __restrict__ keys,
                              const unsigned long long* __restrict__ nvalid_p, int64_t nrows,
@@ -318,8 +322,33 @@ __global__ void k_row_bounds(const uint32_t* __restrict__ keys,
   using S = Stencil<SCHEME>;
   const int nb = row_bounds(n2), ntz = nb / 2 - 1;
   const int nvalid = (int)*nvalid_p;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nrows * nb;
-       i += (int64_t)gridDim.x * blockDim.x) {
+  const int lane = threadIdx.x % kWave;
+  const int64_t entries = nrows * nb;
+  for (int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x - lane; i0 < entries;
+       i0 += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t i1 = i0 + kWave - 1 < entries ? i0 + kWave - 1 : entries - 1;
+    // First particle at or after the start of the first row (lanes 0 .. 31)
+    // and of the row after the last one (32 .. 63).
+    const int64_t edge = (lane < 32 ? i0 / nb : i1 / nb + 1) * n2;  // at most ncells < 2^31
+    const int sub = lane % 32;
+    int lo = 0, hi = nvalid;  // keys[lo - 1] < edge <= keys[hi]
+    while (__ballot(lo < hi) != 0ull) {
+      // 32 probes part [lo, hi) into 33 pieces.
+      const int step = (hi - lo) / 33 + 1;
+      const int64_t at = lo + (int64_t)(sub + 1) * step - 1;
+      const bool below = at < hi && (int64_t)keys[at] < edge;
+      const uint32_t under = (uint32_t)(__ballot(below) >> (lane & 32));
+      const int n = __popc(under);  // probes 0 .. n - 1 are below the edge
+      const int64_t nlo = lo + (int64_t)n * step, nhi = nlo + step - 1;
+      if (lo < hi) {
+        lo = (int)nlo;
+        hi = (int)(nhi < hi ? nhi : hi);
+        if (lo > hi) lo = hi;
+      }
+    }
+    const int first = __shfl(lo, 0, kWave), last = __shfl(lo, 32, kWave);
+    const int64_t i = i0 + lane;
+    if (i >= entries) continue;
     const int64_t row = i / nb;
     const int j = (int)(i - row * nb), b = j >> 1;
     int z;
@@ -328,7 +357,8 @@ __global__ void k_row_bounds(const uint32_t* __restrict__ keys,
     else
       z = (j & 1) ? 1 : n2 - 1;
     const uint32_t key = (uint32_t)(row * n2 + z);
-    int lo = 0, hi = nvalid;  // keys[lo - 1] < key <= keys[hi]
+    lo = first;
+    hi = last;  // keys[lo - 1] < key <= keys[hi]
     while (lo < hi) {
       const int mid = lo + (hi - lo) / 2;
       if (keys[mid] < key)
