@@ -431,9 +431,9 @@ void fill(V* p, int64_t n, V v, hipStream_t s) {
   FC_LAUNCH_CHECK();
 }
 
-// The outputs of one correlation as one run of doubles, cleared by one launch
-// and read back by one copy: r histogram, k histogram, zero lag, then the
-// int32 counts (r, k).
+// The outputs of one correlation as one run of doubles, read back by one copy:
+// r histogram, k histogram, zero lag, then the int32 counts (r, k).  Cleared
+// when allocated; a correlation writes every row once.
 struct OutLayout {
   int64_t nr, nk;
   explicit OutLayout(const fc_corr* c)
@@ -632,16 +632,13 @@ void setup_geometry(fc_corr* c) {
   upload(c->wz, w[2]);
   const OutLayout lay(c);
   c->outputs.allocate(sizeof(double) * lay.doubles());
+  FC_HIP(hipMemset(c->outputs.as<void>(), 0, sizeof(double) * lay.doubles()));
   double* out = c->outputs.as<double>();
   c->r_hist.wrap(out, sizeof(double) * lay.nr);
   c->k_hist.wrap(out + lay.k_hist(), sizeof(double) * lay.nk);
   c->zerolag.wrap(out + lay.zerolag(), sizeof(double));
   c->r_counts.wrap(out + lay.r_counts(), sizeof(int) * lay.nr);
   c->k_counts.wrap(c->r_counts.as<int>() + lay.nr, sizeof(int) * lay.nk);
-}
-
-void reset_hists(fc_corr* c, hipStream_t s) {
-  fill<double>(c->outputs.as<double>(), OutLayout(c).doubles(), 0.0, s);
 }
 
 // Orders the correlator's stream after all work queued on the grid's stream.
@@ -1409,7 +1406,6 @@ void correlate(fc_corr* c, fc_grid* g1, fc_grid* gb, int mode) {
   ensure_work(c);
   flush_stage_times(c);
   FC_HIP(hipEventRecord(c->ev0, s));
-  reset_hists(c, s);
   if (c->kind == FC_YAMAMOTO) {
     // Correlator::autocorrelate = cross(grid, grid)
     if (mode == kModeAuto && c->algo == FC_ALGO_PLAIN) set_grid2_device(c, g1);
@@ -1736,7 +1732,6 @@ void batch_sequence(fc_batch* bt, int n) {
   double* out = bt->outputs.as<double>();
   int* r_counts = reinterpret_cast<int*>(out + ol.r_counts());
   int* k_counts = r_counts + ol.nr;
-  fill<double>(out, ol.doubles() * n, 0.0, s);
   cplx<T>* w = bt->work.as<cplx<T>>();
   const int64_t rows = (int64_t)n * p.n[0] * p.n[1];
   // Forward z and y in the arithmetic of TI (FP64 for the mixed form),
@@ -1870,6 +1865,7 @@ int fc_batch_create(fc_ctx* ctx, const int shape[3], double cell_size, int windo
     b->q2.allocate(csi * b->nq2 * nbatch);
     b->xisub.allocate(tsi * b->nxs * nbatch);
     b->outputs.allocate(sizeof(double) * fc::OutLayout(c).doubles() * nbatch);
+    FC_HIP(hipMemsetAsync(b->outputs.as<void>(), 0, b->outputs.bytes(), ctx->stream));
     b->part.allocate(sizeof(double) * 3 *
                      (size_t)std::max({c->kbin.nchunks, c->rbin.nchunks, c->khalf.nchunks}) *
                      nbatch);

@@ -197,9 +197,9 @@ __global__ void __launch_bounds__(kSegThreads)
   }
 }
 
-// One wave per (multipole, bin): hist[row0 + q][bin] += the chunk partials
+// One wave per (multipole, bin): hist[row0 + q][bin] = the chunk partials
 // of the bin (lane l sums chunks l, l + 64, ... in order, then a fixed xor
-// tree); counts rows [crow0, crow1) += counts of the bin.  nsets sets of
+// tree); counts rows [crow0, crow1) = counts of the bin.  nsets sets of
 // partials, one behind the other, are summed in turn.
 template <int NV>
 __global__ void __launch_bounds__(kWave)
@@ -221,10 +221,10 @@ __global__ void __launch_bounds__(kWave)
       for (int c = c0; c < c1; c += kWave) s += part[((size_t)t * nchunks + c) * NV + q];
       sum += wave_sum(s);
     }
-    if (lane == 0) hist[(size_t)(row0 + q) * nbins + bin] += sum;
+    if (lane == 0) hist[(size_t)(row0 + q) * nbins + bin] = sum;
   }
   if (i < nbins && lane == 0)
-    for (int r = crow0; r < crow1; ++r) counts[(size_t)r * nbins + i] += bin_counts[i];
+    for (int r = crow0; r < crow1; ++r) counts[(size_t)r * nbins + i] = bin_counts[i];
 }
 
 // One block per (multipole, bin): hist[row0 + q][bin] += the block partials
@@ -274,7 +274,7 @@ struct HistScratch {
 
 // nb batch members: member m's outputs (histogram rows, counts, zero lag) lie
 // m * out_bstride doubles behind the first member's.
-// bin_counts (optional): the counts added per bin, instead of bc's own.
+// bin_counts (optional): the counts per bin, instead of bc's own.
 template <int NV, class G>
 void hist_seg_partials(G g, const BinnedCells& bc, double* part, hipStream_t s,
                        int64_t zpos = -1, double* zval = nullptr, int nb = 1,
