@@ -11,11 +11,11 @@
 //     Y_l0(k) W^-1(k) + histogram, every l in one pass);
 //   pruned inverse y pass, pruned z C2R straight into the r subgrid;
 //   r-space multipoles (extract_submatrix + Y_l0(r) + histogram).
-// Correlator (Yamamoto, observer at the survey origin), per (l, m):
+// Correlator (Yamamoto, observer at the survey origin), per group of m of one l:
 //   z pass with Y_lm(x) * delta fused into the load -> y -> the same fused x
-//   pass with F conj(G2) against the stored FFT of grid 2 -> pruned inverse
-//   y, z -> accumulate the k and r subgrids with Y_lm(k), Y_lm(r);
-//   histograms once per l.
+//   pass with F conj(G2) against the stored FFT of grid 2 -> k histogram
+//   partials with Y_lm(k), pruned inverse y, z -> accumulate the r subgrid
+//   with Y_lm(r); partials summed and r histogram once per l.
 // Work arrays are FP64 (FC_FP64) or FP32 (FC_FP32); Y_lm, windows, bin
 // indices and every sum stay in FP64.
 #include <algorithm>
