@@ -395,6 +395,19 @@ int fc_fft_radices(int L, int var, int radices[8], int* count) {
   });
 }
 
+int fc_fft_row_lds(int n2, int precision, size_t* bytes) {
+  return fc::guard([&] {
+    if (!bytes) fc::fail(FC_ERR_INVALID, "null argument");
+    if (precision != FC_FP64 && precision != FC_FP32)
+      fc::fail(FC_ERR_INVALID, "unknown precision");
+    *bytes = 0;
+    if (n2 % 2 == 0 && fc::rc_len_ok(n2 / 2)) return;
+    const fc::GenAxis ax = fc::gen_axis_stages(n2);
+    if (ax.N == 0) return;
+    *bytes = fc::gen_row_lds(ax, precision == FC_FP64 ? sizeof(double2) : sizeof(float2));
+  });
+}
+
 int fc_plan_cache_forget(void) {
   return fc::guard([&] {
     std::lock_guard<std::mutex> lk(fc::g_plan_mu);

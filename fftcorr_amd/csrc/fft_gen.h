@@ -47,9 +47,14 @@ struct GenAxis {
 // has another factor.  Fewest stages, then the largest smallest radix (the
 // threads per column), then the smallest largest one (registers).
 std::vector<int> gen_radices(int L);
-// Whether this engine takes a length, and its tables on the current device.
+// Whether this engine takes a length, its stages (no tables; N = 0 if it does
+// not take it) and its tables on the current device.
 bool gen_len_ok(int L);
+GenAxis gen_axis_stages(int L);
 std::shared_ptr<GenAxis> make_gen_axis(int L);
+// LDS bytes of a workgroup of the row passes of a length, rows stored in
+// complex values of cs bytes.
+size_t gen_row_lds(const GenAxis& ax, size_t cs);
 
 // Columns of [A][L][G][B] (ColView of fft_plan.h): outputs as k_fft_cols_rc.
 struct GenCols {

@@ -178,31 +178,38 @@ bool gen_len_ok(int L) {
   return L >= 1 && L <= kGenMaxLen && (L <= kGenMaxBlue || !gen_radices(L).empty());
 }
 
-std::shared_ptr<GenAxis> make_gen_axis(int L) {
-  if (!gen_len_ok(L)) return nullptr;
-  auto ax = std::make_shared<GenAxis>();
-  ax->L = L;
-  ax->radices = gen_radices(L);
-  ax->N = L;
-  if (ax->radices.empty()) {
+GenAxis gen_axis_stages(int L) {
+  GenAxis ax;
+  if (!gen_len_ok(L)) return ax;
+  ax.L = L;
+  ax.radices = gen_radices(L);
+  int N = L;
+  if (ax.radices.empty()) {
     // The convolution length: among the lengths in [2 L - 1, 1.25 (2 L - 1)],
     // fewest stages, then shortest.
-    ax->blue = true;
+    ax.blue = true;
     for (int n = 2 * L - 1; n <= kGenMaxLen && n <= (2 * L - 1) * 5 / 4 + 1; ++n) {
       std::vector<int> r = gen_radices(n);
       if (r.empty()) continue;
-      if (ax->radices.empty() || r.size() < ax->radices.size()) {
-        ax->radices = r;
-        ax->N = n;
+      if (ax.radices.empty() || r.size() < ax.radices.size()) {
+        ax.radices = r;
+        N = n;
       }
     }
-    if (ax->radices.empty()) return nullptr;
+    if (ax.radices.empty()) return ax;
   }
-  ax->ns = (int)ax->radices.size();
-  for (int r : ax->radices) {
-    ax->tcol = std::max(ax->tcol, ax->N / r);
-    ax->rmax = std::max(ax->rmax, r);
+  ax.N = N;
+  ax.ns = (int)ax.radices.size();
+  for (int r : ax.radices) {
+    ax.tcol = std::max(ax.tcol, ax.N / r);
+    ax.rmax = std::max(ax.rmax, r);
   }
+  return ax;
+}
+
+std::shared_ptr<GenAxis> make_gen_axis(int L) {
+  auto ax = std::make_shared<GenAxis>(gen_axis_stages(L));
+  if (ax->N == 0) return nullptr;
   std::vector<GenStage> st;
   add_stages(st, ax->radices, ax->N, 0);
   std::vector<int> rev(ax->radices.rbegin(), ax->radices.rend());

@@ -340,10 +340,10 @@ __device__ __forceinline__ void gen_run_blue(CL* lds, const GenStage* __restrict
       bar_sink);
 }
 
-// Row tile: row c of rs slots, element e at e + e / 8 (as LayRowPad).
+// Row tile: row c of rs slots, element e at e + e / 2^sh (sh = 3: as LayRowPad).
 struct LayGenRow {
-  int rs;
-  __device__ __forceinline__ int operator()(int c, int e) const { return c * rs + e + (e >> 3); }
+  int rs, sh;
+  __device__ __forceinline__ int operator()(int c, int e) const { return c * rs + e + (e >> sh); }
 };
 // Column tile of tc columns: element e of column c at e tc + c.
 struct LayGenCol {

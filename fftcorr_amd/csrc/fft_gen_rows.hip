@@ -18,15 +18,14 @@ __device__ __forceinline__ bool row_pair(int64_t item, int64_t grp, int64_t nrow
 // imaginary part of one complex row of n2, so odd and even lengths take the
 // same path and no half-length post-processing is needed.  Rows come in groups
 // (batch members) of grp, and a pair never spans two groups: a member's
-// results do not depend on its place.  LDS tr rows of rs.
+// results do not depend on its place.  LDS tr rows of lay.rs.
 template <typename Tin, typename Tout, class Loader, bool BLUE, int RM>
 __global__ void __launch_bounds__(gen_max_threads<RM>())
     k_gen_r2c(const Tin* in, int64_t ldi, cplx<Tout>* out, int64_t ldo, int64_t nrows, int64_t grp,
-              int rs, Loader ld, GenDev g) {
+              LayGenRow lay, Loader ld, GenDev g) {
   using CL = cplx<typename std::conditional<BLUE, double, Tout>::type>;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   CL* lds = reinterpret_cast<CL*>(smem_raw);
-  const LayGenRow lay{rs};
   const int c = threadIdx.y, j = threadIdx.x;
   const int L = g.L;
   int64_t r0;
@@ -71,11 +70,10 @@ __global__ void __launch_bounds__(gen_max_threads<RM>())
 template <typename T, typename Tout, bool BLUE, int RM>
 __global__ void __launch_bounds__(gen_max_threads<RM>())
     k_gen_c2r(const cplx<T>* in, int64_t ldi, Tout* out, int64_t ldo, int64_t nrows, int64_t grp,
-              int rs, int nsel, int offm, GenDev g) {
+              LayGenRow lay, int nsel, int offm, GenDev g) {
   using CL = cplx<typename std::conditional<BLUE, double, T>::type>;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   CL* lds = reinterpret_cast<CL*>(smem_raw);
-  const LayGenRow lay{rs};
   const int c = threadIdx.y, j = threadIdx.x;
   const int L = g.L;
   int64_t r0;
@@ -112,17 +110,26 @@ __global__ void __launch_bounds__(gen_max_threads<RM>())
     gen_run<RM, 0>(lds, g.stg, g.ns, g.W, c, j, lay, load, NoMid{}, put, false);
 }
 
+constexpr size_t kRowLds = 65536;  // of a workgroup (gen_row_tile's limit)
 struct RowShape {
-  int tr, rs;
+  LayGenRow lay;
+  int tr;
   size_t lds;
   unsigned nb;
 };
 RowShape row_shape(const GenAxis& ax, size_t cl, int64_t nrows, int64_t grp) {
   RowShape r;
   const int64_t items = (nrows + grp - 1) / grp * ((grp + 1) / 2);
-  r.rs = ax.N + ax.N / 8 + 1;
-  r.tr = gen_row_tile(ax, (size_t)r.rs * cl);
-  r.lds = (size_t)r.tr * r.rs * cl;
+  // A gap after every eighth element, so that neither the stages' strides nor
+  // neighbouring rows meet in one bank; where one row with its gaps exceeds the
+  // budget (FP64 values, more than 3640 of them), as many as it leaves room
+  // for: a gap after every 16th to 128th element, none at 4096 points.
+  r.lay = LayGenRow{ax.N + ax.N / 8 + 1, 3};
+  while ((size_t)r.lay.rs * cl > kRowLds && r.lay.sh < 16)
+    r.lay.rs = ax.N + ((ax.N - 1) >> ++r.lay.sh);
+  r.tr = gen_row_tile(ax, (size_t)r.lay.rs * cl);
+  r.lds = (size_t)r.tr * r.lay.rs * cl;
+  if (r.lds > kRowLds) fail(FC_ERR_RUNTIME, "internal: row tile exceeds the LDS budget");
   const int64_t nb = (items + r.tr - 1) / r.tr;
   if (nb > INT32_MAX) fail(FC_ERR_INVALID, "transform too large for one launch");
   r.nb = (unsigned)nb;
@@ -130,6 +137,10 @@ RowShape row_shape(const GenAxis& ax, size_t cl, int64_t nrows, int64_t grp) {
 }
 
 }  // namespace
+
+size_t gen_row_lds(const GenAxis& ax, size_t cs) {
+  return row_shape(ax, ax.blue ? sizeof(double2) : cs, 1, 1).lds;
+}
 
 template <typename Tin, typename Tout, class Loader>
 void launch_gen_r2c(const GenAxis& ax, const Tin* in, int64_t ldi, cplx<Tout>* out, int64_t ldo,
@@ -139,7 +150,7 @@ void launch_gen_r2c(const GenAxis& ax, const Tin* in, int64_t ldi, cplx<Tout>* o
   auto go = [&](auto blue, auto rm) {
     hipLaunchKernelGGL(
         (k_gen_r2c<Tin, Tout, Loader, decltype(blue)::value, decltype(rm)::value>), dim3(r.nb),
-        dim3((unsigned)ax.tcol, (unsigned)r.tr), r.lds, s, in, ldi, out, ldo, nrows, grp, r.rs,
+        dim3((unsigned)ax.tcol, (unsigned)r.tr), r.lds, s, in, ldi, out, ldo, nrows, grp, r.lay,
         ld, gen_dev(ax));
   };
   gen_dispatch(ax, go);
@@ -154,7 +165,7 @@ void launch_gen_c2r(const GenAxis& ax, const cplx<T>* in, int64_t ldi, Tout* out
   auto go = [&](auto blue, auto rm) {
     hipLaunchKernelGGL((k_gen_c2r<T, Tout, decltype(blue)::value, decltype(rm)::value>), dim3(r.nb),
                        dim3((unsigned)ax.tcol, (unsigned)r.tr), r.lds, s, in, ldi, out, ldo,
-                       nrows, grp, r.rs, nsel, offm, gen_dev(ax));
+                       nrows, grp, r.lay, nsel, offm, gen_dev(ax));
   };
   gen_dispatch(ax, go);
   FC_LAUNCH_CHECK();

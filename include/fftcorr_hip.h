@@ -312,6 +312,9 @@ int fc_plan_variants(int device, const int shape[3], int precision, int vars[3])
  * returns their count (at most 8) in *count, 0 when the register-chained
  * kernels have no such variant for L (other lengths use fixed plans). */
 int fc_fft_radices(int L, int var, int radices[8], int* count);
+/* LDS bytes a workgroup of the row passes of n2 samples takes where they run
+ * the mixed-radix stages (0 for other lengths).  No GPU needed. */
+int fc_fft_row_lds(int n2, int precision, size_t* bytes);
 
 #ifdef __cplusplus
 }
