@@ -632,8 +632,10 @@ void setup_geometry(fc_corr* c) {
   upload(c->wz, w[2]);
   const OutLayout lay(c);
   c->outputs.allocate(sizeof(double) * lay.doubles());
-  FC_HIP(hipMemset(c->outputs.as<void>(), 0, sizeof(double) * lay.doubles()));
   double* out = c->outputs.as<double>();
+  // On the stream that writes them later: the null stream, whose clearing the
+  // host need not wait for, is not ordered with it.
+  fill<double>(out, lay.doubles(), 0.0, c->ctx->stream);
   c->r_hist.wrap(out, sizeof(double) * lay.nr);
   c->k_hist.wrap(out + lay.k_hist(), sizeof(double) * lay.nk);
   c->zerolag.wrap(out + lay.zerolag(), sizeof(double));
