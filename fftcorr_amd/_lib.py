@@ -73,6 +73,7 @@ SIGNATURES = {
     "fc_ctx_destroy": (ctypes.c_int, [_vp]),
     "fc_ctx_footprint": (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_size_t)]),
     "fc_ctx_release_scratch": (ctypes.c_int, [_vp]),
+    "fc_ctx_host_footprint": (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_size_t)]),
     "fc_ctx_synchronize": (ctypes.c_int, [_vp]),
     "fc_grid_create": (ctypes.c_int, [_vp, _ip, _dp, ctypes.c_double, ctypes.c_int,
                                       ctypes.POINTER(_vp)]),

@@ -161,6 +161,7 @@ class PinnedBuffer {
     bytes_ = 0;
   }
   char* data() const { return static_cast<char*>(ptr_); }
+  size_t bytes() const { return bytes_; }
 
  private:
   void* ptr_ = nullptr;

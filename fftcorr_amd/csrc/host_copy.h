@@ -70,11 +70,20 @@ class HostCopier {
     if (fork_) (void)hipEventDestroy(fork_);
   }
 
+  // Page-locked bytes it holds.
+  size_t pinned_bytes() const {
+    size_t b = 0;
+    for (const Slot& s : slots_) b += s.mem ? kChunk : 0;
+    return b;
+  }
+
   HostCopier(const HostCopier&) = delete;
   HostCopier& operator=(const HostCopier&) = delete;
 
   // Copies dst[0, bytes) = src[0, bytes) after the work queued on stream s and
-  // before what s is given next; src may change or go when this returns.  The caller's current device is the copier's.
+  // before what s is given next.  src may change or go when this returns, or
+  // (shorter copies out of page-locked memory) when s has been waited for.
+  // The caller's current device is the copier's.
   hipError_t copy(void* dst, const void* src, size_t bytes, hipStream_t s) {
     if (bytes < kMinBytes || !usable_)
       return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s);

@@ -911,9 +911,16 @@ int fc_mass_assign(fc_grid* grid, const double* pos, int64_t n, int ncol,
     ctx->scratch[10].reserve(sizeof(double) * n * (ncol + (weights ? 1 : 0)));
     double* dpos = ctx->scratch[10].as<double>();
     double* dw = weights ? dpos + n * ncol : nullptr;
-    if (!ctx->copier) ctx->copier.reset(new fc::HostCopier(ctx->device));
-    FC_HIP(ctx->copier->copy(dpos, pos, sizeof(double) * n * ncol, s));
-    if (weights) FC_HIP(ctx->copier->copy(dw, weights, sizeof(double) * n, s));
+    // Staged copies from the length on that HostCopier takes them, which only
+    // then is made (its page-locked slots, streams and events take 140 us).
+    const bool staged = sizeof(double) * n * ncol >= fc::HostCopier::kMinBytes;
+    if (staged && !ctx->copier) ctx->copier.reset(new fc::HostCopier(ctx->device));
+    auto copy = [&](double* d, const double* h, size_t bytes) {
+      FC_HIP(staged ? ctx->copier->copy(d, h, bytes, s)
+                    : hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, s));
+    };
+    copy(dpos, pos, sizeof(double) * n * ncol);
+    if (weights) copy(dw, weights, sizeof(double) * n);
     fc::mass_assign_device(grid, dpos, n, ncol, dw, w_scalar, scheme, periodic_wrap, shift, stats);
   });
 }

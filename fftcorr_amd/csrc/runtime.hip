@@ -113,6 +113,18 @@ int fc_ctx_release_scratch(fc_ctx* ctx) {
     fc::DeviceGuard g(ctx->device);
     FC_HIP(hipStreamSynchronize(ctx->stream));
     for (auto& b : ctx->scratch) b.release();
+    ctx->copier.reset();
+    std::lock_guard<std::mutex> lk(ctx->results_mu);
+    ctx->results.release();
+  });
+}
+
+int fc_ctx_host_footprint(fc_ctx* ctx, size_t* bytes) {
+  return fc::guard([&] {
+    fc::check_ctx(ctx);
+    if (!bytes) fc::fail(FC_ERR_INVALID, "null argument");
+    std::lock_guard<std::mutex> lk(ctx->results_mu);
+    *bytes = ctx->results.bytes() + (ctx->copier ? ctx->copier->pinned_bytes() : 0);
   });
 }
 

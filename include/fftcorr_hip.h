@@ -79,6 +79,10 @@ int fc_ctx_synchronize(fc_ctx* ctx);
  * again).  No reference counterpart. */
 int fc_ctx_footprint(fc_ctx* ctx, size_t* bytes);
 int fc_ctx_release_scratch(fc_ctx* ctx);
+/* Page-locked host bytes the context holds: staging of host catalogues of 4 MB
+ * and more (16 MB, from the first of them on) and results on their way to the
+ * caller.  fc_ctx_release_scratch releases them too. */
+int fc_ctx_host_footprint(fc_ctx* ctx, size_t* bytes);
 
 /* ---- ConfigSpaceGrid: cc/grid/config_space_grid.h:10-56,
  *      fftcorr/grid/config_space_grid.pyx:11-207 -------------------------- */
