@@ -72,14 +72,12 @@ struct fc_corr {
   fc::HistScratch hs;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   bool timed = false;
-  // Periodic correlations run the k histogram on a second stream (default
-  // priority) beside the pruned inverse; created on first use.
-  hipStream_t side = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  // Yamamoto correlations run the pruned inverse of a transform on a third
-  // stream, beside the forward passes of the next one.
-  hipStream_t inv = nullptr;
-  hipEvent_t ev_inv = nullptr;
+  // Periodic correlations run the k histogram on a second stream beside the
+  // pruned inverse, Yamamoto correlations the pruned inverse of a transform on
+  // a third one, beside the forward passes of the next (the context's
+  // beside_stream 0 and 1); the events that fork from the context's stream and
+  // join it again, made on first use.
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_inv = nullptr;
   fc::DeviceBuffer part_k;  // the k histogram's partials (the r histogram's are hs.part_seg)
   // Per-stage profiling: event pairs recorded during the last call(s).
   bool profile = false;
@@ -1035,23 +1033,17 @@ void periodic_r_hist(fc_corr* c) {
                    0, NV, c->ctx->stream, c->rbin.tracked_pos, c->zerolag.as<double>());
 }
 
-// The side stream and its fork / join events (created on first use).
+// The side stream, and the fork / join events on first use.
 hipStream_t side_stream(fc_corr* c) {
-  if (!c->side) {
-    FC_HIP(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
-    FC_HIP(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
-    FC_HIP(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
-  }
-  return c->side;
+  if (!c->ev_fork) FC_HIP(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
+  if (!c->ev_join) FC_HIP(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
+  return beside_stream(c->ctx, 0);
 }
 
 // The stream of the Yamamoto correlations' pruned inverse (likewise).
 hipStream_t inverse_stream(fc_corr* c) {
-  if (!c->inv) {
-    FC_HIP(hipStreamCreateWithFlags(&c->inv, hipStreamNonBlocking));
-    FC_HIP(hipEventCreateWithFlags(&c->ev_inv, hipEventDisableTiming));
-  }
-  return c->inv;
+  if (!c->ev_inv) FC_HIP(hipEventCreateWithFlags(&c->ev_inv, hipEventDisableTiming));
+  return beside_stream(c->ctx, 1);
 }
 
 // After the forward passes: power spectrum and pruned inverse x, then the k
@@ -1478,13 +1470,10 @@ int fc_corr_destroy(fc_corr* corr) {
     if (!corr) return;
     fc::DeviceGuard dg(corr->ctx->device);
     (void)hipStreamSynchronize(corr->ctx->stream);
-    if (corr->side) {
-      (void)hipStreamSynchronize(corr->side);
-      (void)hipStreamDestroy(corr->side);
-    }
-    if (corr->inv) {
-      (void)hipStreamSynchronize(corr->inv);
-      (void)hipStreamDestroy(corr->inv);
+    {  // a call that failed may have left work on the other streams
+      std::lock_guard<std::mutex> lk(corr->ctx->beside_mu);
+      for (hipStream_t b : corr->ctx->beside)
+        if (b) (void)hipStreamSynchronize(b);
     }
     if (corr->ev_inv) (void)hipEventDestroy(corr->ev_inv);
     if (corr->ev_fork) (void)hipEventDestroy(corr->ev_fork);

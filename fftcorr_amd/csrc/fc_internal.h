@@ -175,6 +175,9 @@ class PinnedBuffer {
 struct fc_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
+  // Two more streams for work beside the first one's (fc::beside_stream).
+  hipStream_t beside[2] = {nullptr, nullptr};
+  std::mutex beside_mu;
   // Scratch reused across calls on this context (sort temp storage, staging).
   fc::DeviceBuffer scratch[12];  // per-context work buffers, grown on demand
   std::unique_ptr<fc::HostCopier> copier;  // staged copies of host arrays, on first use
@@ -200,6 +203,17 @@ struct DeviceGuard {
     if (prev >= 0 && cur != prev) (void)hipSetDevice(prev);
   }
 };
+
+// Stream i of the two beside the context's own, default priority, made on first
+// use and kept: one with a hardware queue of its own takes 50 to 400 us to make
+// and as long to end, too much for a correlator that is called once.  The
+// context's correlators share them; each orders its work there by its own events
+// after and before the context's stream.
+inline hipStream_t beside_stream(fc_ctx* ctx, int i) {
+  std::lock_guard<std::mutex> lk(ctx->beside_mu);
+  if (!ctx->beside[i]) FC_HIP(hipStreamCreateWithFlags(&ctx->beside[i], hipStreamNonBlocking));
+  return ctx->beside[i];
+}
 
 // Copies device memory to the host in one transfer on the context's stream,
 // waits for it and hands the bytes to use(const char*).  A copy to pageable

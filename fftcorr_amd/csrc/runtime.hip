@@ -92,6 +92,11 @@ int fc_ctx_destroy(fc_ctx* ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     ctx->copier.reset();
     for (auto& b : ctx->scratch) b.release();
+    for (hipStream_t b : ctx->beside)
+      if (b) {
+        (void)hipStreamSynchronize(b);
+        (void)hipStreamDestroy(b);
+      }
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
   });
