@@ -1256,7 +1256,6 @@ void yamamoto_correlate(fc_corr* c, fc_grid* g1, bool own) {
   hipStream_t s = c->ctx->stream;
   const FftPlan& p = *c->plan;
   const int most = yamamoto_most(c);
-  c->work.reserve(most * p.complex_bytes());
   cplx<T>* w = c->work.as<cplx<T>>();
   const uint64_t ncells = (uint64_t)c->shape[0] * c->shape[1] * c->shape[2];
   ensure_periodic_buffers<T, TI>(c, most);
@@ -1355,7 +1354,12 @@ void yamamoto_correlate(fc_corr* c, fc_grid* g1, bool own) {
   }
 }
 
-void ensure_work(fc_corr* c) { c->work.reserve(c->plan->complex_bytes()); }
+// The work spectra, at once in the size the sequence takes: growing them later
+// would free what was just allocated, which waits for the device.
+void ensure_work(fc_corr* c) {
+  const bool groups = c->kind == FC_YAMAMOTO && c->algo != FC_ALGO_PLAIN;
+  c->work.reserve((groups ? yamamoto_most(c) : 1) * c->plan->complex_bytes());
+}
 
 void set_grid2_device(fc_corr* c, fc_grid* g2) {
   ensure_work(c);

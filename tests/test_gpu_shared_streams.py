@@ -1,6 +1,7 @@
 """Correlators of one context share the streams beside its own: interleaved calls,
 calls from several threads and a correlator that ends between two calls of another
 give the bits of a correlator alone."""
+import ctypes
 import threading
 
 import numpy as np
@@ -70,3 +71,24 @@ def test_threads():
     for t in th:
         t.join()
     assert not bad, bad
+
+
+def test_work_spectra_are_allocated_once():
+    """A survey correlator's work buffer has its full size (nine spectra for
+    l <= 4) from set_grid2 on: the first correlation adds only the rest."""
+    n = 64
+    c, a = make("survey", n, _lib.context())
+    spectrum = n * n * 40 * 16  # complex rows of 33 values padded to 40
+
+    def held():
+        now, full = ctypes.c_size_t(), ctypes.c_size_t()
+        _lib.check(_lib.lib().fc_corr_footprint(c._handle, 0, ctypes.byref(now),
+                                                ctypes.byref(full)))
+        return now.value
+
+    before = held()
+    c.set_grid2(a)
+    assert held() - before == (9 + 1) * spectrum  # and grid 2's own
+    middle = held()
+    c.cross_correlate(a)
+    assert held() - middle < 8 * spectrum
