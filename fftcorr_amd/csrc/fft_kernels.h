@@ -1,5 +1,6 @@
-// LDS-staged Stockham FFT kernels for the 3D R2C / C2R transforms of the
-// padded work grid [n0][n1][n2/2+1] (the layout of cc/grid/fft_grid.cc:10-50).
+// Stockham FFT kernels for the 3D R2C / C2R transforms of the padded work grid
+// [n0][n1][n2/2+1] (the layout of cc/grid/fft_grid.cc:10-50): compile-time plans
+// whose values stay in registers between LDS exchanges, and direct sums.
 //
 //  * z pass (rows, contiguous): a real row of n2 samples is packed as n2/2
 //    complex values, transformed with a half-length complex FFT and
@@ -9,14 +10,14 @@
 //    the Y_lm(x) weighting of the density into this load.
 //  * y and x passes (columns, strided): a workgroup owns TC adjacent
 //    columns (contiguous along z), so each global access is a run of TC
-//    complex values; the TC transforms run in LDS with E complex values per
-//    thread in registers between stages.
+//    complex values; the TC transforms exchange through LDS with E complex
+//    values per thread in registers between stages.
 //
 // Lengths 2^a (8..4096) and 3*2^a (192..3072) use compile-time radix plans;
 // every other length runs the mixed-radix passes (fft_gen.h) or, where those
-// are slower, a direct O(L^2) DFT per column/row.  Forward transforms use sign -1 and no
-// normalisation, the inverse sign +1 and no 1/N, matching FFTW's r2c/c2r as
-// called by the reference (cc/grid/fft_grid.cc:81-84).
+// are slower, a direct O(L^2) DFT per column/row.  Forward transforms use sign
+// -1 and no normalisation, the inverse sign +1 and no 1/N, matching FFTW's
+// r2c/c2r as called by the reference (cc/grid/fft_grid.cc:81-84).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -371,7 +372,7 @@ constexpr int fft_plan_of() {
 // E), after the last stage (radix Rl) slot s holds element
 // t + out_m(s) L/E.  The first stage therefore reads global memory directly
 // and the last stage's outputs go straight to global memory (or to the next
-// fused step): two LDS passes fewer than the LDS-staged form above.
+// fused step): a pass of three stages exchanges through LDS twice.
 template <class R>
 struct RadixInfo;
 template <int R>
@@ -595,11 +596,6 @@ void stage_twiddles_(Radices<R, Rest...>, Put put) {
 }
 
 
-// Register-chained strided column pass over [A][L][G][B] (see k_fft_cols),
-// TC columns per workgroup, one launch of A * G * ceil(B / TC) workgroups.
-// Output o < nout holds element (o - off) mod L (offm = off mod L; nout may
-// exceed L).  In place when in == out: every workgroup reads its whole tile
-// before writing it.  Arithmetic in T; loads Tin; LDS and stores in To.
 // Waves per SIMD a register-chained column kernel is held to when its
 // arithmetic is wider than its LDS tiles (the occupancy of the narrow form).
 // Variant 1 holds twice the values per thread and is sized for half the waves.
@@ -609,6 +605,13 @@ constexpr int rc_wide_waves() {
   return sizeof(T) > sizeof(To) ? (V == 1 ? 4 : FftCfgV<L, V>::E > 8 ? 5 : 8) : 1;
 }
 
+// Register-chained strided column pass over a column view [A][L][G][B] (G groups
+// of B contiguous columns; element (a, e, g, b) at a inA + e inL + g inG + b of
+// the input, outA, outL, outG of the output), TC columns per workgroup, one
+// launch of A * G * ceil(B / TC) workgroups.  Output o < nout holds element
+// (o - off) mod L (offm = off mod L; nout may exceed L).  In place when in ==
+// out: every workgroup reads its whole tile before writing it.  Arithmetic in
+// T; loads Tin; LDS and stores in To.
 template <typename T, int L, int DIR, int TC, typename Tin = T, typename To = T, int V = 0>
 __global__ void __launch_bounds__(TC*(L / FftCfgV<L, V>::E))
 __attribute__((amdgpu_waves_per_eu(rc_wide_waves<T, To, V, L>())))
@@ -618,7 +621,8 @@ __attribute__((amdgpu_waves_per_eu(rc_wide_waves<T, To, V, L>())))
   using C = cplx<T>;
   constexpr int E = FftCfgV<L, V>::E;
   constexpr int TCOL = L / E;
-  // Tiles above 64 KB (the longest lengths) are static: dynamic LDS stops there.
+  // Tiles above 64 KB (the longest lengths) are static arrays: every dynamic
+  // request of this library stays within 64 KB.
   constexpr size_t kTile = (size_t)L * TC * sizeof(cplx<To>);
   constexpr bool kStatic = kTile > 65536;
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -845,8 +849,8 @@ struct PairOf<double> {
 };
 
 // Register-chained R2C rows: a real row of 2M samples packed as M complex
-// values, a length-M FFT, then the Hermitian post-process (see
-// k_fft_rows_r2c).  Block = tr rows x M/E threads, LDS tr row_pad_len(M).
+// values, a length-M FFT, then the Hermitian post-process.  Block = tr rows x
+// M/E threads, LDS tr row_pad_len(M).
 // Arithmetic in T; LDS and outputs in To.
 // in2 (optional): rows from nrows1 on come from in2 (row - nrows1), so one
 // launch transforms two grids into consecutive output rows.
@@ -929,8 +933,8 @@ __global__ void __launch_bounds__(1024)
   }
 }
 
-// Register-chained C2R rows (see k_fft_rows_c2r): the pre-process runs in LDS,
-// the length-M FFT starts from registers and the real samples go straight
+// Register-chained C2R rows: the inverse of the Hermitian post-process runs in
+// LDS, the length-M FFT starts from registers and the real samples go straight
 // from registers to global memory.  nsel == 0 writes whole rows; nsel > 0
 // writes sample (o - off) mod 2M at o < nsel (offm = off mod 2M).  In place
 // when the real rows overlay the complex rows: every workgroup reads its rows

@@ -68,7 +68,7 @@ int default_col_tile(int L, size_t cs);
 int default_row_tile(int M, size_t cs);
 
 // ---- launchers -------------------------------------------------------------
-// Column view [A][L][G][B] for k_fft_cols / k_dft_cols (see fft_kernels.h).
+// Column view [A][L][G][B] for k_fft_cols_rc / k_dft_cols (see fft_kernels.h).
 template <typename T, typename Tin = T>
 struct ColView {
   const cplx<Tin>* in;

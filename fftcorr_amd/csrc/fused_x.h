@@ -214,7 +214,7 @@ __device__ __forceinline__ void x2_store_q(const cplx<TI> (&u)[1][FftCfgV<L, V>:
 }
 
 // ---- the fused kernel -------------------------------------------------------
-// Lengths the fused kernel takes: plans whose first radix is E.
+// Lengths the fused kernel takes: those with a compile-time plan.
 __host__ __device__ constexpr bool px_len_ok(int L) { return rc_len_ok(L); }
 // LDS of tc columns: the forward tiles hold the storage type T, the inverse
 // tile TI.
@@ -254,8 +254,8 @@ template <typename T, typename TI, int L>
 constexpr int px_waves() {
   return sizeof(T) == 4 && px_plan<T, TI, L>() == 0 ? 4 : 2;
 }
-// Whether the stage twiddles are copied to LDS: not at 1024 points, whose two
-// tables (38 KB in the mixed form) would leave one workgroup per CU.
+// Whether the stage twiddles are copied to LDS: not from 1024 points on, whose
+// two tables (38 KB in the mixed form) would leave one workgroup per CU.
 template <int L>
 constexpr bool px_tw_lds() {
   return L <= 768;

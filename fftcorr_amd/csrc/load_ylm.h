@@ -6,15 +6,6 @@
 
 namespace fc {
 
-// Along a row x and y are fixed, so Y_lm c is a polynomial of degree l in z
-// over r^l: the row's coefficients are formed once per thread (one switch over
-// (l, m)) and a sample costs four multiply-adds and a division instead of the
-// whole formula of ylm_eval with its switch (256^3 FP64 weighted z pass 53.2 ->
-// 49.7 us, the plain copy taking 48.6).  FP64; differs from ylm_eval by
-// rounding (a few ulp).
-//
-// Several transforms of one l may share a launch: output rows g rows_per + r
-// are the grid's row r weighted with m + g.
 // 1 / d for normal d > 0 well inside the exponent range: the hardware's
 // estimate and two Newton steps (to about 1 ulp), without the scaling and the
 // special cases of the division.  With one reciprocal per two samples the
@@ -26,6 +17,15 @@ __device__ __forceinline__ double inv_normal(double d) {
   return fma(r, fma(-d, r, 1.0), r);
 }
 
+// Along a row x and y are fixed, so Y_lm c is a polynomial of degree l in z
+// over r^l: the row's coefficients are formed once per thread (one switch over
+// (l, m)) and a sample costs four multiply-adds and half a reciprocal instead of
+// the whole formula of ylm_eval with its switch (256^3 FP64 weighted z pass 53.2
+// -> 49.7 us, still with a division per sample, the plain copy taking 48.6).
+// FP64; differs from ylm_eval by rounding (a few ulp).
+//
+// Several transforms of one l may share a launch: output rows g rows_per + r
+// are the grid's row r weighted with m + g.
 struct LoadYlm {
   int ell, m, n1;
   double c0, c;          // normalisation of m = 0 and of the others
